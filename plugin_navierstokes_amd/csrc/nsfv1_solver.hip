@@ -493,135 +493,339 @@ dense_matvec(const double* __restrict__ A, const double* __restrict__ x, double*
 //   M'[p][k] = 1/a, M'[p][j] = -M[p][j]/a,
 //   M'[i][k] = M[i][k]/a, M'[i][j] = M[i][j] - M'[i][k] M[p][j]   (i != p),
 // a = M[p][k].  After n steps x_k = sum_j M[p_k][j] y_{p_j}, so
-// inv[k][p_j] = M[p_k][j].  Ping-pong tableaux; every workgroup repeats the
-// pivot search with the same fixed-order reduction (ties go to the smaller
-// row).  A column that vanishes on every unpivoted row (a null mode of the
-// coarse operator, e.g. the constant pressure of a domain with Dirichlet
-// velocity everywhere) pins its unknown to zero in the coarse correction
-// (a = 0 is replaced by 1/a := 0), instead of dividing by zero; a column
-// with no finite entry left is reported.
+// inv[k][p_j] = M[p_k][j].  Ties of the pivot search go to the smaller row.
+// A column that vanishes on every unpivoted row (a null mode of the coarse
+// operator, e.g. the constant pressure of a domain with Dirichlet velocity
+// everywhere) pins its unknown to zero in the coarse correction (a = 0 is
+// replaced by 1/a := 0), instead of dividing by zero; a column with no
+// finite entry left is reported.
+//
+// GJ_BLOCK steps form a panel.  Its columns, exchanged step by step, hold
+// G = A A_pp^-1 in the end (A the panel's columns, A_pp its pivot rows; A_pp^-1
+// itself in the pivot rows), so on the other columns the panel is one product
+// M' = C - G M_p with M_p the pivot rows before the panel and C = M, or 0 in the
+// pivot rows.  gj_step applies panel k to ping-pong tableaux, one wave per 16
+// rows on the FP64 matrix cores; its first workgroup meanwhile brings the
+// columns of panel k + 1 up to date with the same products and exchanges them,
+// rows in registers, and leaves their G for the next launch.
+//
+// The bound is the dependent chain of the pivots (search, one barrier, one
+// division, one row update), so it stays in one workgroup without a global
+// access, with few waves (each instruction of the search costs every wave),
+// and everything else runs beside it.  The search compares the upper 32 bits of
+// the sizes: the pivot is the largest to a factor 1 + 2^-20.
+// Measured: 16 pivots take 28 us of a launch's 36 us; n = 867: 2.1 ms (four
+// pivots per launch, each workgroup repeating the search: 7.2 ms), n = 448:
+// 0.8 ms (1.9 ms).  512 threads beat 256 (37.0 us a launch: the loads of the
+// next panel's columns) and 1024 (51 us: the search).
 // ---------------------------------------------------------------------
 template <typename JT>
 __global__ void __launch_bounds__(256)
 gj_load(const int64_t* __restrict__ rowptr, const int32_t* __restrict__ colidx, const JT* __restrict__ J, int n,
-        double* __restrict__ M, double* __restrict__ cabs, int* __restrict__ done, int* __restrict__ err)
+        double* __restrict__ M, int* __restrict__ done, int* __restrict__ err)
 {
     const int r = blockIdx.x;
     double* row = M + (int64_t)r * n;
     for (int j = threadIdx.x; j < n; j += blockDim.x) row[j] = 0.0;
     __syncthreads();
     for (int64_t k = rowptr[r] + threadIdx.x; k < rowptr[r + 1]; k += blockDim.x) row[colidx[k]] = (double)J[k];
-    __syncthreads();
     if (threadIdx.x == 0) {
-        cabs[r] = fabs(row[0]);
         done[r] = 0;
         if (r == 0) *err = 0;
     }
 }
 
-// GJ_BLOCK exchange steps per launch (same pivots, same arithmetic as one
-// step per launch, with every update an explicit fma).  Each workgroup
-// loads columns k0 .. k0+nb-1 of every row (the panel) and replays the
-// steps on it: the pivot search of step s reads the panel after steps
-// 0 .. s-1, the pivot row of step s is row p_s of the input evolved through
-// those steps, and the multiplier of row r at step s (its column-k value
-// after the step, f = M[r][k] / a) is kept for the row updates.  The panel
-// and the full rows take the same operations in the same order, so the
-// pivots are those the full rows give.  Then each workgroup applies the nb
-// steps to its rows.  Pivoted flags ping-pong between launches (din ->
-// dout), so no workgroup reads a flag that another one writes.
-constexpr int GJ_BLOCK = 4;
+constexpr int GJ_BLOCK = 16;  // pivots of a panel
+constexpr int GJ_TPB = 512;
+typedef double f64x4 __attribute__((ext_vector_type(4)));
 
-__global__ void __launch_bounds__(256)
-gj_block(const double* __restrict__ Min, double* __restrict__ Mout, const int* __restrict__ din,
-         int* __restrict__ dout, int* __restrict__ piv, int* __restrict__ err, int n, int k0, int nb)
+// what a panel leaves for its update
+struct GJPanel {
+    double* G;  // [n][GJ_BLOCK], 0 past the panel's last column
+    int* flag;  // [n]: 1 for the rows pivoted in the panel
+    int* piv;   // [GJ_BLOCK]: pivot rows, -1 past the last step
+};
+
+// pivot rows of the panel at columns j0 ..: B operands of the four products
+// (lane l: row 4 s + (l >> 4), column l & 15)
+__device__ __forceinline__ void gj_pivot_rows(const double* __restrict__ M, const GJPanel& G, int n, int j0, int lane,
+                                              double (&P)[GJ_BLOCK / 4])
 {
-    __shared__ double pan[MG_DENSE_MAX][GJ_BLOCK];   // panel columns of every row
-    __shared__ double prow[GJ_BLOCK][MG_DENSE_MAX];  // pivot row of step s, before step s
-    __shared__ double fm[GJ_BLOCK][MG_DENSE_MAX];    // multiplier of every row at step s
-    __shared__ int sdone[MG_DENSE_MAX];
-    __shared__ double sv[4], sia[GJ_BLOCK];
-    __shared__ int si[4], sp[GJ_BLOCK];
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-    for (int r = t; r < n; r += 256) {
-        sdone[r] = din[r];
+    const int j = j0 + (lane & 15) < n ? j0 + (lane & 15) : n - 1;
 #pragma unroll
-        for (int q = 0; q < GJ_BLOCK; ++q) pan[r][q] = q < nb ? Min[(int64_t)r * n + k0 + q] : 0.0;
+    for (int s = 0; s < GJ_BLOCK / 4; ++s) {
+        const int r = G.piv[4 * s + (lane >> 4)];
+        const double m = M[r > 0 ? r * n + j : j];
+        P[s] = r >= 0 ? m : 0.0;
     }
-    __syncthreads();
+}
+
+// 16 x 16 tile at (r0, j0) of C - G M_p: lane l holds column l & 15, rows
+// (l >> 4) + 4 i (the FP64 16x16x4 accumulator layout).  Loads are
+// unconditional (indices clamped; what lies outside the tableau is not used),
+// so that those of several tiles are in flight together.
+struct GJTile {
+    double c[4], g[GJ_BLOCK / 4];
+    int flag[4];
+};
+
+__device__ __forceinline__ void gj_load_tile(const double* __restrict__ M, const GJPanel& G, int n, int r0, int j0,
+                                             int lane, GJTile& T)
+{
+    const int cl = lane & 15, kq = lane >> 4;
+    const int j = j0 + cl < n ? j0 + cl : n - 1, ra = r0 + cl < n ? r0 + cl : n - 1;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int r = r0 + kq + 4 * i < n ? r0 + kq + 4 * i : n - 1;
+        T.c[i] = M[r * n + j];
+        T.flag[i] = G.flag[r];
+    }
+#pragma unroll
+    for (int s = 0; s < GJ_BLOCK / 4; ++s) T.g[s] = G.G[ra * GJ_BLOCK + 4 * s + kq];
+}
+
+__device__ __forceinline__ f64x4 gj_tile(const GJTile& T, const double (&P)[GJ_BLOCK / 4])
+{
+    f64x4 acc;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[i] = T.flag[i] ? 0.0 : T.c[i];
+#pragma unroll
+    for (int s = 0; s < GJ_BLOCK / 4; ++s) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(-T.g[s], P[s], acc, 0, 0, 0);
+    return acc;
+}
+
+template <int ROR>
+__device__ __forceinline__ uint32_t row_max_step(uint32_t v)
+{
+    const uint32_t o = (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x120 + ROR, 0xf, 0xf, false);
+    return v > o ? v : o;
+}
+
+__device__ __forceinline__ uint32_t wave_max(uint32_t v)
+{
+    v = row_max_step<8>(v);
+    v = row_max_step<4>(v);
+    v = row_max_step<2>(v);
+    v = row_max_step<1>(v);
+    const uint32_t a = (uint32_t)__builtin_amdgcn_readlane((int)v, 0), b = (uint32_t)__builtin_amdgcn_readlane((int)v, 16);
+    const uint32_t c = (uint32_t)__builtin_amdgcn_readlane((int)v, 32), d = (uint32_t)__builtin_amdgcn_readlane((int)v, 48);
+    const uint32_t ab = a > b ? a : b, cd = c > d ? c : d;
+    return ab > cd ? ab : cd;
+}
+
+struct GJSlot {
+    double row[GJ_BLOCK];
+    uint32_t key;
+    int r;
+};
+
+// The nb pivots of a panel, row t + GJ_TPB h in thread t, the panel's values in
+// registers.  The registers rotate, pan[h][0] being the column of the current
+// step: a step writes column x + 1 to register x and the step's own column to
+// the last one, so every index is a compile-time constant.
+template <int R>
+__device__ __forceinline__ void gj_pivots(double (&pan)[R][GJ_BLOCK], int (&dn)[R], int (&in)[R],
+                                          GJSlot (&slot)[2][GJ_TPB / 64], int (&sp)[GJ_BLOCK], int& bad, int n, int nb,
+                                          int t, int lane, int wave)
+{
+    constexpr int B = GJ_BLOCK, W = GJ_TPB / 64;
+    // sort keys: 0 for pivoted rows, NaN and rows past the end
+    const auto sort_key = [](double v, int pivoted) {
+        const double a = fabs(v);
+        return (pivoted || a != a) ? 0u : (uint32_t)(__builtin_bit_cast(uint64_t, a) >> 32) + 1u;
+    };
+    uint32_t key[R], mx = 0;
+#pragma unroll
+    for (int h = 0; h < R; ++h) {
+        key[h] = sort_key(pan[h][0], dn[h]);
+        mx = key[h] > mx ? key[h] : mx;
+    }
+    mx = wave_max(mx);
+#pragma unroll 1
     for (int q = 0; q < nb; ++q) {
-        const int k = k0 + q;
-        // pivot search over the unpivoted rows (ties to the smaller row)
-        double bv = -2.0;
-        int bi = 0;
-        for (int r = t; r < n; r += 256) {
-            const double v = sdone[r] ? -1.0 : fabs(pan[r][q]);
-            if (v > bv) bv = v, bi = r;
-        }
+        // the wave's smallest row of the largest key publishes its panel row
+        GJSlot& sl = slot[q & 1][wave];
+        bool open = true;
 #pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-            const double ov = __shfl_xor(bv, o, 64);
-            const int oi = __shfl_xor(bi, o, 64);
-            if (ov > bv || (ov == bv && oi < bi)) bv = ov, bi = oi;
-        }
-        if (lane == 0) sv[w] = bv, si[w] = bi;
-        __syncthreads();
-        bv = sv[0], bi = si[0];
+        for (int h = 0; h < R; ++h) {
+            const uint64_t hit = __ballot(key[h] == mx);
+            if (open && hit != 0) {
+                open = false;
+                if (lane == (int)__builtin_ctzll(hit)) {
 #pragma unroll
-        for (int x = 1; x < 4; ++x)
-            if (sv[x] > bv || (sv[x] == bv && si[x] < bi)) bv = sv[x], bi = si[x];
-        const int p = bi;
-        const bool pin = bv == 0.0;
-        if (t == 0 && blockIdx.x == 0 && !(bv >= 0.0)) *err = 1;
-        // the pivot row before this step: row p evolved through steps 0 .. q-1
-        for (int j = t; j < n; j += 256) {
-            double v = Min[(int64_t)p * n + j];
-            for (int x = 0; x < q; ++x) {
-                const double f = fm[x][p];
-                v = j == k0 + x ? f : fma(-f, prow[x][j], v);
-            }
-            prow[q][j] = v;
-        }
-        double pv[GJ_BLOCK];
-#pragma unroll
-        for (int x = 0; x < GJ_BLOCK; ++x) pv[x] = pan[p][x];
-        __syncthreads();
-        const double ia = pin ? 0.0 : 1.0 / prow[q][k];
-        if (t == 0) sp[q] = p, sia[q] = ia;
-        for (int r = t; r < n; r += 256) {
-            if (r == p) {
-                fm[q][r] = ia;
-#pragma unroll
-                for (int x = 0; x < GJ_BLOCK; ++x)
-                    if (x > q) pan[r][x] = -pv[x] * ia;
-            } else {
-                const double f = pan[r][q] * ia;
-                fm[q][r] = f;
-#pragma unroll
-                for (int x = 0; x < GJ_BLOCK; ++x)
-                    if (x > q) pan[r][x] = fma(-f, pv[x], pan[r][x]);
-            }
-        }
-        if (t == 0) sdone[p] = 1;
-        __syncthreads();
-    }
-    if (blockIdx.x == 0 && t < nb) piv[k0 + t] = sp[t];
-    // the workgroup's rows through the nb steps
-    for (int i = blockIdx.x; i < n; i += gridDim.x) {
-        for (int j = t; j < n; j += 256) {
-            double v = Min[(int64_t)i * n + j];
-            for (int x = 0; x < nb; ++x) {
-                const int kx = k0 + x;
-                if (i == sp[x]) {
-                    v = j == kx ? sia[x] : -v * sia[x];
-                } else {
-                    const double f = fm[x][i];
-                    v = j == kx ? f : fma(-f, prow[x][j], v);
+                    for (int x = 0; x < B; ++x) sl.row[x] = pan[h][x];
+                    sl.key = mx;
+                    sl.r = t + GJ_TPB * h;
                 }
             }
-            Mout[(int64_t)i * n + j] = v;
         }
-        if (t == 0) dout[i] = sdone[i];
+        __syncthreads();
+        // best of the waves (ties: the smaller row)
+        const uint32_t ks = slot[q & 1][lane & (W - 1)].key;
+        const int rs = slot[q & 1][lane & (W - 1)].r;
+        int w = 0, p = __builtin_amdgcn_readlane(rs, 0);
+        uint32_t best = (uint32_t)__builtin_amdgcn_readlane((int)ks, 0);
+#pragma unroll
+        for (int o = 1; o < W; ++o) {
+            const uint32_t k2 = (uint32_t)__builtin_amdgcn_readlane((int)ks, o);
+            const int p2 = __builtin_amdgcn_readlane(rs, o);
+            if (k2 > best || (k2 == best && p2 < p)) {
+                best = k2;
+                p = p2;
+                w = o;
+            }
+        }
+        double pr[B];
+#pragma unroll
+        for (int x = 0; x < B; ++x) pr[x] = slot[q & 1][w].row[x];
+        const double ia = pr[0] == 0.0 ? 0.0 : 1.0 / pr[0];
+        if (t == 0) sp[q] = p;
+        bad |= best == 0;
+        // the next step's column first: its search runs beside the other columns
+        double f[R];
+        mx = 0;
+#pragma unroll
+        for (int h = 0; h < R; ++h) {
+            f[h] = pan[h][0] * ia;
+            pan[h][0] = fma(-f[h], pr[1], pan[h][1]);
+            if (t + GJ_TPB * h == p) dn[h] = in[h] = 1;
+            key[h] = sort_key(pan[h][0], dn[h]);
+            mx = key[h] > mx ? key[h] : mx;
+        }
+        mx = wave_max(mx);
+#pragma unroll
+        for (int h = 0; h < R; ++h) {
+#pragma unroll
+            for (int x = 1; x + 1 < B; ++x) pan[h][x] = fma(-f[h], pr[x + 1], pan[h][x + 1]);
+            pan[h][B - 1] = f[h];
+        }
+        if (((p >> 6) & (W - 1)) == wave)
+#pragma unroll
+            for (int h = 0; h < R; ++h)
+                if (t + GJ_TPB * h == p) {  // the pivot row
+#pragma unroll
+                    for (int x = 0; x + 1 < B; ++x) pan[h][x] = -pr[x + 1] * ia;
+                    pan[h][B - 1] = ia;
+                }
+    }
+    // a short last panel: rotate on until column x sits in register x
+#pragma unroll 1
+    for (int q = nb; q < B; ++q) {
+#pragma unroll
+        for (int h = 0; h < R; ++h) {
+            const double v = pan[h][0];
+#pragma unroll
+            for (int x = 0; x + 1 < B; ++x) pan[h][x] = pan[h][x + 1];
+            pan[h][B - 1] = v;
+        }
+        if (t == 0) sp[q] = -1;
+    }
+}
+
+// R rows of the panel per thread (n <= GJ_TPB R)
+template <int R>
+__global__ void __launch_bounds__(GJ_TPB)
+gj_step(const double* __restrict__ Min, double* __restrict__ Mout, GJPanel cur, GJPanel nxt, int* __restrict__ done,
+        int* __restrict__ piv, int* __restrict__ err, int n, int k0, int first)
+{
+    constexpr int B = GJ_BLOCK;
+    const int t = threadIdx.x, lane = t & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    if (blockIdx.x > 0) {
+        // update: one 16 x 16 tile per wave
+        const int tiles = (n + B - 1) / B;
+        const int tile = ((int)blockIdx.x - 1) * (GJ_TPB / 64) + wave;
+        const int j0 = (tile % tiles) * B, r0 = (tile / tiles) * B;
+        if (r0 >= n) return;
+        const int j = j0 + (lane & 15);
+        f64x4 v;
+        if (j0 == k0) {  // the panel's own columns: G
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int r = r0 + (lane >> 4) + 4 * i;
+                v[i] = r < n ? cur.G[(int64_t)r * B + (lane & 15)] : 0.0;
+            }
+        } else {
+            double P[B / 4];
+            GJTile T;
+            gj_load_tile(Min, cur, n, r0, j0, lane, T);
+            gj_pivot_rows(Min, cur, n, j0, lane, P);
+            v = gj_tile(T, P);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int r = r0 + (lane >> 4) + 4 * i;
+            if (r < n && j < n) Mout[(int64_t)r * n + j] = v[i];
+        }
+        return;
+    }
+
+    // the next panel: columns [k1, k1 + nb)
+    __shared__ double stage[GJ_TPB / 64][16][17];  // per wave: one tile, to hand its rows to lanes
+    __shared__ GJSlot slot[2][GJ_TPB / 64];
+    __shared__ int sp[B];
+    const int k1 = first ? 0 : k0 + B;
+    if (k1 >= n) return;
+    const int nb = n - k1 < B ? n - k1 : B;
+    double pan[R][B];
+    int dn[R], in[R];
+#pragma unroll
+    for (int h = 0; h < R; ++h) {
+        const int r = t + GJ_TPB * h;
+        dn[h] = r < n ? done[r] : 1;
+        in[h] = 0;
+#pragma unroll
+        for (int x = 0; x < B; ++x) pan[h][x] = 0.0;
+    }
+    double P[B / 4];
+    if (!first) gj_pivot_rows(Min, cur, n, k1, lane, P);
+#pragma unroll
+    for (int h = 0; h < R; ++h) {
+        f64x4 v[4];
+        GJTile T[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) gj_load_tile(Min, cur, n, GJ_TPB * h + wave * 64 + q * 16, k1, lane, T[q]);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            if (!first) {
+                v[q] = gj_tile(T[q], P);
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[q][i] = T[q].c[i];
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) stage[wave][(lane >> 4) + 4 * i][lane & 15] = v[q][i];
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            // every lane reads (row lane & 15); the tile's lanes keep it
+#pragma unroll
+            for (int x = 0; x < B; ++x) {
+                const double w = stage[wave][lane & 15][x];
+                pan[h][x] = (lane >> 4) == q ? w : pan[h][x];
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        }
+    }
+    int bad = 0;
+    gj_pivots<R>(pan, dn, in, slot, sp, bad, n, nb, t, lane, wave);
+    __syncthreads();
+    if (t < B) {
+        nxt.piv[t] = sp[t];
+        if (t < nb) piv[k1 + t] = sp[t];
+    }
+    if (t == 0 && bad) *err = 1;
+#pragma unroll
+    for (int h = 0; h < R; ++h) {
+        const int r = t + GJ_TPB * h;
+        if (r >= n) continue;
+        done[r] = dn[h];
+        nxt.flag[r] = in[h];
+#pragma unroll
+        for (int x = 0; x < B; ++x) nxt.G[(int64_t)r * B + x] = x < nb ? pan[h][x] : 0.0;
     }
 }
 
@@ -844,32 +1048,53 @@ hipError_t launch_inject(const int64_t* inj, const double* uf, double* uc, int64
     return hipGetLastError();
 }
 
+// two tableaux, two panels (G, flags, pivots), the pivoted flags, the pivot
+// rows of all steps and, as its last word, the error flag
 size_t dense_inverse_work_bytes(int n)
 {
-    return sizeof(double) * (2 * (size_t)n * n + 2 * (size_t)n) + sizeof(int) * (2 * (size_t)n + 4);
+    const size_t m = (size_t)n;
+    return sizeof(double) * (2 * m * m + 2 * m * GJ_BLOCK) + sizeof(int) * (2 * (m + GJ_BLOCK) + 2 * m + 2);
 }
 
 hipError_t launch_dense_inverse(int jprec, const int64_t* rowptr, const int32_t* colidx, const void* J, int n,
                                 void* work, double* inv, int* err, hipStream_t s)
 {
     if (n <= 0) return hipSuccess;
-    double* M[2] = {(double*)work, (double*)work + (size_t)n * n};
-    double* c[2] = {M[1] + (size_t)n * n, M[1] + (size_t)n * n + n};
-    int* done = (int*)(c[1] + n);
-    int* piv = done + n;
-    if (jprec == 64) gj_load<double><<<n, 256, 0, s>>>(rowptr, colidx, (const double*)J, n, M[0], c[0], done, err);
-    else gj_load<float><<<n, 256, 0, s>>>(rowptr, colidx, (const float*)J, n, M[0], c[0], done, err);
     if (n > MG_DENSE_MAX) return hipErrorInvalidValue;
-    // GJ_BLOCK steps per launch; the pivoted flags alternate between `done`
-    // and the (unused here) second pivot-magnitude array
-    int* dflag[2] = {done, reinterpret_cast<int*>(c[1])};
-    const int nl = (n + GJ_BLOCK - 1) / GJ_BLOCK;
-    const unsigned g = n < 256 ? (unsigned)n : 256u;
-    for (int l = 0; l < nl; ++l) {
-        const int k0 = l * GJ_BLOCK, nb = n - k0 < GJ_BLOCK ? n - k0 : GJ_BLOCK;
-        gj_block<<<g, 256, 0, s>>>(M[l & 1], M[(l + 1) & 1], dflag[l & 1], dflag[(l + 1) & 1], piv, err, n, k0, nb);
+    static_assert(MG_DENSE_MAX <= 3 * GJ_TPB, "gj_step is built for at most three rows per thread");
+    const size_t nn = (size_t)n * n;
+    double* M[2] = {(double*)work, (double*)work + nn};
+    GJPanel G[2];
+    G[0].G = M[1] + nn;
+    G[1].G = G[0].G + (size_t)n * GJ_BLOCK;
+    int* iw = (int*)(G[1].G + (size_t)n * GJ_BLOCK);
+    for (int q = 0; q < 2; ++q) {
+        G[q].flag = iw;
+        G[q].piv = iw + n;
+        iw += n + GJ_BLOCK;
     }
-    gj_unpermute<<<blocks_for((int64_t)n * n, 256), 256, 0, s>>>(M[nl & 1], piv, n, inv);
+    int* done = iw;
+    int* piv = done + n;
+    if (jprec == 64) gj_load<double><<<n, 256, 0, s>>>(rowptr, colidx, (const double*)J, n, M[0], done, err);
+    else gj_load<float><<<n, 256, 0, s>>>(rowptr, colidx, (const float*)J, n, M[0], done, err);
+    // launch l applies panel l - 1 (none for l = 0) and factors panel l
+    const int np = (n + GJ_BLOCK - 1) / GJ_BLOCK;
+    const unsigned wgs = ((unsigned)np * np + GJ_TPB / 64 - 1) / (GJ_TPB / 64);
+    for (int l = 0; l <= np; ++l) {
+        const double* in = M[l > 0 ? (l - 1) & 1 : 0];
+        double* out = M[l > 0 ? l & 1 : 1];
+        const unsigned g = l > 0 ? 1 + wgs : 1;
+        const int k0 = l > 0 ? (l - 1) * GJ_BLOCK : 0;
+        const auto step = [&](auto kern) {
+            kern<<<g, GJ_TPB, 0, s>>>(in, out, G[(l + 1) & 1], G[l & 1], done, piv, err, n, k0, l == 0);
+        };
+        switch ((n + GJ_TPB - 1) / GJ_TPB) {
+        case 1: step(gj_step<1>); break;
+        case 2: step(gj_step<2>); break;
+        default: step(gj_step<3>); break;
+        }
+    }
+    gj_unpermute<<<blocks_for((int64_t)n * n, 256), 256, 0, s>>>(M[np & 1], piv, n, inv);
     return hipGetLastError();
 }
 
