@@ -1298,17 +1298,7 @@ assemble_rows_split(KMeshPtrs M, KParams P, const double* __restrict__ u, const 
         }
         __syncthreads();
     }
-    if (wantJ) {
-        if constexpr (PADE == 0) {
-            for (int i = threadIdx.x; i < jlen; i += blockDim.x) J[jbase + i] = jbuf[i];
-        } else {
-            for (int j = 0; j < v1 - v0; ++j) {
-                const int off = (int)(M.rowptr[(int64_t)(v0 + j) * NC] - jbase);
-                const int len = (int)(M.rowptr[(int64_t)(v0 + j + 1) * NC] - jbase) - off;
-                for (int i = threadIdx.x; i < len; i += blockDim.x) J[jbase + off + i] = jbuf[off + j * PADE + i];
-            }
-        }
-    }
+    if (wantJ) store_rows<NC, PADE>(M.rowptr, v0, v1 - v0, jbase, jlen, jbuf, J + jbase);
     if (dout)
         for (int i = threadIdx.x; i < dlen; i += blockDim.x) dout[(int64_t)v0 * NC + i] = dbuf[i];
 }
@@ -1548,17 +1538,7 @@ assemble_rows_rowlane(KMeshPtrs M, KParams P, const double* __restrict__ u, cons
         }
         __syncthreads();
     }
-    if (wantJ) {
-        if constexpr (PADE == 0) {
-            for (int i = threadIdx.x; i < jlen; i += blockDim.x) J[jbase + i] = jbuf[i];
-        } else {
-            for (int j = 0; j < v1 - v0; ++j) {
-                const int off = (int)(M.rowptr[(int64_t)(v0 + j) * NC] - jbase);
-                const int len = (int)(M.rowptr[(int64_t)(v0 + j + 1) * NC] - jbase) - off;
-                for (int i = threadIdx.x; i < len; i += blockDim.x) J[jbase + off + i] = jbuf[off + j * PADE + i];
-            }
-        }
-    }
+    if (wantJ) store_rows<NC, PADE>(M.rowptr, v0, v1 - v0, jbase, jlen, jbuf, J + jbase);
     if (dout)
         for (int i = threadIdx.x; i < dlen; i += blockDim.x) dout[(int64_t)v0 * NC + i] = dbuf[i];
 }

@@ -164,4 +164,39 @@ __device__ inline void lds_add_block(T* p, const T (&x)[NC])
     }
 }
 
+// Finished rows of the nodes [v0, v0 + nn) from LDS (PADE pad values after each
+// node's rows) to the CSR values that start at J.  Waves take nodes in turn.
+// The lanes of a wave load the offsets of 64 nodes at once: one dependent load
+// per node, in a loop of the whole workgroup over the nodes, was a third to
+// a half of the 3D row kernels' time (56^3 distorted hexahedra, LPS, FP32: 672 -> 588 us an assembly; 1.3 M tetrahedra: 1555 -> 1490 us).
+template <int NC, int PADE, typename JT>
+__device__ inline void store_rows(const int64_t* __restrict__ rowptr, int v0, int nn, int64_t jbase, int jlen,
+                                  const JT* jbuf, JT* __restrict__ J)
+{
+    if constexpr (PADE == 0) {
+        for (int i = threadIdx.x; i < jlen; i += blockDim.x) J[i] = jbuf[i];
+    } else {
+        static_assert(NC == 4, "padded rows are rows of 3D meshes");
+        constexpr int V = 16 / (int)sizeof(JT);  // a row block is NC^2 values: a multiple of V
+        struct alignas(16) Vec { JT x[V]; };
+        const int lane = threadIdx.x & 63, nw = (int)blockDim.x >> 6;
+        const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+        const bool vec = ((uintptr_t)J & 15) == 0;
+        for (int b = 0; b < nn; b += 64) {
+            const int a = b + lane < nn ? b + lane : nn - 1;
+            const int o0 = (int)(rowptr[(int64_t)(v0 + a) * NC] - jbase);
+            const int o1 = (int)(rowptr[(int64_t)(v0 + a + 1) * NC] - jbase);
+            for (int j = wave; j < 64 && b + j < nn; j += nw) {
+                const int off = __builtin_amdgcn_readlane(o0, j), len = __builtin_amdgcn_readlane(o1, j) - off;
+                const JT* src = jbuf + off + (b + j) * PADE;
+                if (vec)
+                    for (int i = lane; i < len / V; i += 64)
+                        reinterpret_cast<Vec*>(J + off)[i] = reinterpret_cast<const Vec*>(src)[i];
+                else
+                    for (int i = lane; i < len; i += 64) J[off + i] = src[i];
+            }
+        }
+    }
+}
+
 }  // namespace nsfv1
