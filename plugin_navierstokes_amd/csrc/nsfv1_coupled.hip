@@ -12,12 +12,20 @@
 // Kernel coupled_scvf: a workgroup is one wavefront holding EPW = 64 / nip
 // elements, one lane per (element, SCVF).  The lanes of an element exchange
 // their SCVF data through LDS (ip velocities, shapes, gradients, mass
-// fluxes, upwind shapes) and invert the ip system together: Gauss-Jordan
-// with partial pivoting, one row per lane, the pivot search by the
-// element's first lane.  Each lane then writes its SCVF's contribution to
-// the row block of its `from` corner -- (dim+1) x nsh x (dim+1) Jacobian
-// values and dim+1 defect values; the `to` corner receives the negative --
-// or, for the data export, the stabilised velocity.
+// fluxes, right-hand sides) and invert the ip system together: Gauss-Jordan
+// in exchange form with partial pivoting, a lane's row in registers, the
+// pivot row and the sizes of the column's entries through LDS.  Each lane then
+// forms its SCVF's contribution to the row block of its `from` corner
+// (dim+1) x nsh x (dim+1) Jacobian values and dim+1 defect values; the `to`
+// corner receives the negative.  The first nsh lanes of an element add the
+// SCVFs of their corner and write the element matrix, one row block per
+// corner (the gather reads one row block per (node, element) instead of
+// three).  For the data export the lanes write the stabilised velocity.
+// Measured, FP32 Jacobian: FIELDS + positive upwind on 40^3 hexahedra 1533 -> 752
+// us an assembly (the elimination by the first lane, element by element in LDS,
+// and every lane forming the right-hand sides of all ips took half of it),
+// FLOW + LPS on 48^3 hexahedra 1321 -> 1102 us.  What is left is FP64 work at one
+// wave per SIMD: two casts against twelve side triangles per SCVF with FLOW.
 //
 // Kernel coupled_rows: the row-owner gather shared with the other paths:
 // one lane per (node, element) incidence adds the records of the SCVFs at
@@ -28,6 +36,7 @@
 #include <stdint.h>
 
 #include "nsfv1_internal.hpp"
+#include "nsfv1_geom.hpp"
 #include "nsfv1_ray.hpp"
 #include "nsfv1_topo.hpp"
 
@@ -41,11 +50,20 @@ struct CplShared {
     double phi[NIP][N], g[NIP][N][D];
     double mflux[NIP];
     int has[NIP];
-    double vv[NIP], vc[NIP], vd[NIP];
-    double Us[NIP][N], Ud[NIP][N];
-    double aug[NIP][2 * NIP];
-    int piv;
+    double cd0[NIP][N];           // matrix case: shapes of the right-hand side, common part of all components
+    double f[NIP][D];             // matrix case: right-hand sides
+    double irho[NIP];             // 1 / density (imported densities)
+    double inv[NIP][NIP];         // inverse of the ip system
+    double key[NIP], row[NIP];    // elimination: sizes of the column's entries, pivot row
+    int pv[NIP];                  // pivot lane of each column
 };
+
+// LDS exchange between the lanes of the workgroup's one wave
+__device__ __forceinline__ void wave_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+}
 
 // corner c (runtime) of a per-lane coordinate array, by selects over the
 // compile-time corners, so the array stays in registers
@@ -314,6 +332,7 @@ coupled_scvf(KMeshPtrs M, KParams P, const double* __restrict__ u, const double*
     using T = Topo<ET>;
     constexpr int D = T::dim, N = T::nsh, NC = D + 1, NIP = T::nip, EPW = CplCfg<ET>::EPW;
     __shared__ CplShared<ET> shm[EPW];
+    __shared__ union { double d[64][NC]; JT j[64][NC * NC]; } xch;  // per lane: defect, column block
     const int lane = threadIdx.x;
     const int es = lane / NIP, ip = lane - (lane / NIP) * NIP;
     const int64_t e = (int64_t)blockIdx.x * EPW + es;
@@ -478,67 +497,116 @@ coupled_scvf(KMeshPtrs M, KParams P, const double* __restrict__ u, const double*
             vc = nrm / Ls;
             if (flow) vd = nrm / (Ld + Ls);
         }
-        if (matrix) {
-            S.vv[ip] = vv;
-            S.vc[ip] = vc;
-            S.vd[ip] = vd;
+    }
+    const double rho = (RHOIP && act) ? M.rho_ip[e * NIP + ip] : P.rho;  // density at the lane's ip
+
+    // ---- matrix case: the ip system (stabilization.cpp:244-403, 604-772).
+    //      Lane ip holds row ip and forms its own right-hand sides (corner
+    //      contributions of every velocity component and the pressure, in
+    //      ascending corners)
+    if (matrix) {
+        double m[NIP];
+#pragma unroll
+        for (int j = 0; j < NIP; ++j) {
+            double a = 0.0;
+            if (j == ip) {
+                if (P.has_old) a += P.inv_dt;
+                a += vv;
+                a += vc;
+            }
+            a -= Ws[j] * vc;
+            if (flow) a += vd * (Ws[j] - Wd[j]);
+            m[j] = a;
+        }
+        if (act) {
+            double f[D], f0[D];
+#pragma unroll
+            for (int d = 0; d < D; ++d) {
+                f0[d] = P.has_source ? (M.f_scvf ? M.f_scvf[(e * NIP + ip) * D + d] : P.f[d]) : 0.0;
+                if (P.has_old) {
+                    double o = 0.0;
+#pragma unroll
+                    for (int k = 0; k < N; ++k) o += S.phi[ip][k] * uold[(int64_t)M.conn[e * N + k] * NC + d];
+                    f0[d] += o * P.inv_dt;
+                }
+                f[d] = flow ? 0.0 : f0[d];
+            }
 #pragma unroll
             for (int k = 0; k < N; ++k) {
-                S.Us[ip][k] = Us[k];
-                S.Ud[ip][k] = Ud[k];
+                double cd0 = vv * S.phi[ip][k];
+                cd0 += vc * Us[k];
+                if (flow) cd0 += vd * (Ud[k] - Us[k]);
+                S.cd0[ip][k] = cd0;
+#pragma unroll
+                for (int d = 0; d < D; ++d) {
+                    const double cp = -1.0 * S.g[ip][k][d] / rho;
+                    double cd = cd0;
+                    if (flow) {
+#pragma unroll
+                        for (int d2 = 0; d2 < D; ++d2)
+                            if (d2 != d) cd -= S.sv[ip][d2] * S.g[ip][k][d2];
+#pragma unroll
+                        for (int d2 = 0; d2 < D; ++d2)
+                            f[d] += ul[k][d2] * (d2 == d ? cd : S.sv[ip][d] * S.g[ip][k][d2]);
+                    } else {
+                        f[d] += ul[k][d] * cd;
+                    }
+                    f[d] += ul[k][D] * cp;
+                }
             }
 #pragma unroll
-            for (int j = 0; j < NIP; ++j) {
-                double m = 0.0;
-                if (j == ip) {
-                    if (P.has_old) m += P.inv_dt;
-                    m += vv;
-                    m += vc;
-                }
-                m -= Ws[j] * vc;
-                if (flow) m += vd * (Ws[j] - Wd[j]);
-                S.aug[ip][j] = m;
-                S.aug[ip][NIP + j] = j == ip ? 1.0 : 0.0;
-            }
+            for (int d = 0; d < D; ++d) S.f[ip][d] = flow ? f[d] + f0[d] : f[d];
+            if constexpr (RHOIP) S.irho[ip] = 1.0 / rho;
         }
-    }
-    __syncthreads();
-
-    // ---- Gauss-Jordan inversion of the ip system, one row per lane
-    if (matrix) {
+        // exchange-form elimination: step c exchanges column c with the
+        // unpivoted row of its largest entry.  A row rotates through its
+        // registers (m[0] is column c), so one loop body serves every step.
+        int mycol = -1;
+#pragma unroll 1
         for (int c = 0; c < NIP; ++c) {
-            if (act && ip == 0) {
-                int pv = c;
-                for (int r = c + 1; r < NIP; ++r)
-                    if (fabs(S.aug[r][c]) > fabs(S.aug[pv][c])) pv = r;
-                if (S.aug[pv][c] == 0.0) ok_geo = false;
-                if (pv != c)
-                    for (int j = 0; j < 2 * NIP; ++j) {
-                        const double t = S.aug[c][j];
-                        S.aug[c][j] = S.aug[pv][j];
-                        S.aug[pv][j] = t;
-                    }
+            if (act) S.key[ip] = mycol < 0 ? fabs(m[0]) : -1.0;
+            wave_sync();
+            int p = 0;
+            double best = S.key[0];
+#pragma unroll
+            for (int r = 1; r < NIP; ++r) {
+                const double v = S.key[r];
+                if (v > best) {
+                    best = v;
+                    p = r;
+                }
             }
-            __syncthreads();
-            if (act && ip == c && S.aug[c][c] != 0.0) {
-                const double iv = 1.0 / S.aug[c][c];
-                for (int j = 0; j < 2 * NIP; ++j) S.aug[c][j] *= iv;
+            if (act && ip == p) {
+#pragma unroll
+                for (int j = 0; j < NIP; ++j) S.row[j] = m[j];
+                S.pv[c] = p;
             }
-            __syncthreads();
-            if (act && ip != c) {
-                const double f = S.aug[ip][c];
-                if (f != 0.0)
-                    for (int j = 0; j < 2 * NIP; ++j) S.aug[ip][j] -= f * S.aug[c][j];
+            wave_sync();
+            const double a = S.row[0];
+            if (a == 0.0) ok_geo = false;
+            const double ia = a == 0.0 ? 0.0 : 1.0 / a;
+            const bool own = ip == p;
+            const double f = own ? ia : m[0] * ia;
+#pragma unroll
+            for (int j = 0; j + 1 < NIP; ++j) {
+                const double r = S.row[j + 1];
+                m[j] = own ? -r * ia : m[j + 1] - f * r;
             }
-            __syncthreads();
+            m[NIP - 1] = f;
+            if (own) mycol = c;
+            wave_sync();
         }
+        // inverse: entry (k, p_j) is entry j of the row that column k pivoted on
+        if (act && mycol >= 0)
+#pragma unroll
+            for (int j = 0; j < NIP; ++j) S.inv[mycol][S.pv[j]] = m[j];
+        wave_sync();
     }
     if (!act) return;
 
     // ---- stabilised velocity of the lane's ip.  Its shapes (the derivatives
     //      by each corner's unknowns) are formed corner by corner in the
     //      Jacobian loop below, from the same expressions.
-    const double rho = RHOIP ? M.rho_ip[e * NIP + ip] : P.rho;  // density at the lane's ip
     double svel[D], diag = 1.0;
     if (P.stab_type == STAB_WITHOUT) {  // stabilization.cpp:805-850
 #pragma unroll
@@ -581,78 +649,11 @@ coupled_scvf(KMeshPtrs M, KParams P, const double* __restrict__ u, const double*
             svel[d] = rhs / diag;
         }
     } else {  // matrix case: stabilization.cpp:244-403, 604-772
-        // corner contributions of every velocity component and the pressure
-        // to each ip's right-hand side f[d][j], then mapped through row ip of
-        // the inverse; each f[d][j] takes its corners in ascending order, and
-        // the ip data of (j, k) is read once for all components
-        const double* iv = &S.aug[ip][NIP];
-        double f[D][NIP];
-#pragma unroll
-        for (int d = 0; d < D; ++d)
-#pragma unroll
-            for (int j = 0; j < NIP; ++j) {
-                f[d][j] = 0.0;
-                if (!flow) {
-                    if (P.has_source) f[d][j] = M.f_scvf ? M.f_scvf[(e * NIP + j) * D + d] : P.f[d];
-                    if (P.has_old) {
-                        double o = 0.0;
-#pragma unroll
-                        for (int k = 0; k < N; ++k) o += S.phi[j][k] * uold[(int64_t)M.conn[e * N + k] * NC + d];
-                        f[d][j] += o * P.inv_dt;
-                    }
-                }
-            }
-#pragma unroll
-        for (int k = 0; k < N; ++k) {
-#pragma unroll
-            for (int j = 0; j < NIP; ++j) {
-                double gj[D], svj[D];
-#pragma unroll
-                for (int d = 0; d < D; ++d) {
-                    gj[d] = S.g[j][k][d];
-                    svj[d] = S.sv[j][d];
-                }
-                double cd0 = S.vv[j] * S.phi[j][k];
-                cd0 += S.vc[j] * S.Us[j][k];
-                if (flow) cd0 += S.vd[j] * (S.Ud[j][k] - S.Us[j][k]);
-#pragma unroll
-                for (int d = 0; d < D; ++d) {
-                    const double cp = -1.0 * gj[d] / (RHOIP ? M.rho_ip[e * NIP + j] : rho);
-                    double cd = cd0;
-                    if (flow) {
-#pragma unroll
-                        for (int d2 = 0; d2 < D; ++d2) {
-                            if (d2 == d) continue;
-                            cd -= svj[d2] * gj[d2];
-                        }
-                        // f: corner contributions of every component, then pressure
-#pragma unroll
-                        for (int d2 = 0; d2 < D; ++d2)
-                            f[d][j] = f[d][j] + ul[k][d2] * (d2 == d ? cd : svj[d] * gj[d2]);
-                        f[d][j] = f[d][j] + ul[k][D] * cp;
-                    } else {
-                        f[d][j] = f[d][j] + ul[k][d] * cd;
-                        f[d][j] = f[d][j] + ul[k][D] * cp;
-                    }
-                }
-            }
-        }
 #pragma unroll
         for (int d = 0; d < D; ++d) {
-            if (flow)
-#pragma unroll
-                for (int j = 0; j < NIP; ++j) {
-                    if (P.has_source) f[d][j] += M.f_scvf ? M.f_scvf[(e * NIP + j) * D + d] : P.f[d];
-                    if (P.has_old) {
-                        double o = 0.0;
-#pragma unroll
-                        for (int k = 0; k < N; ++k) o += S.phi[j][k] * uold[(int64_t)M.conn[e * N + k] * NC + d];
-                        f[d][j] += o * P.inv_dt;
-                    }
-                }
             double x = 0.0;
 #pragma unroll
-            for (int j = 0; j < NIP; ++j) x += iv[j] * f[d][j];
+            for (int j = 0; j < NIP; ++j) x += S.inv[ip][j] * S.f[j][d];
             svel[d] = x;
         }
     }
@@ -710,6 +711,7 @@ coupled_scvf(KMeshPtrs M, KParams P, const double* __restrict__ u, const double*
     const double sa = P.s_a;
 
     // ---- defect of the `from` row: navier_stokes_fv1.cpp:667-777
+    double* xd = xch.d[lane];
     {
         double gv[D][D];
 #pragma unroll
@@ -724,7 +726,6 @@ coupled_scvf(KMeshPtrs M, KParams P, const double* __restrict__ u, const double*
         double pr = 0.0;
 #pragma unroll
         for (int k = 0; k < N; ++k) pr += S.phi[ip][k] * ul[k][D];
-        double* rd = recD + (e * NIP + ip) * NC;
 #pragma unroll
         for (int d1 = 0; d1 < D; ++d1) {
             double df = 0.0;
@@ -736,10 +737,38 @@ coupled_scvf(KMeshPtrs M, KParams P, const double* __restrict__ u, const double*
             double r = df * (-1.0 * nu * rho);
             if (!stokes) r += upv[d1] * prod;
             r += pr * n[d1];
-            rd[d1] = sa * r;
+            xd[d1] = sa * r;
         }
-        rd[D] = sa * (dot_nc<D>(svel, n) * rho);
+        xd[D] = sa * (dot_nc<D>(svel, n) * rho);
     }
+    // rows of the element matrix: corner `ip` adds its SCVFs in ascending
+    // order, the `to` corner with the negative sign
+    const bool corner = ip < N;
+    int cs[T::cip];
+    bool cf[T::cip];
+#pragma unroll
+    for (int q = 0; q < T::cip; ++q) {
+        const int i = TabH<ET>::t.cip[corner ? ip : 0][q];
+        cs[q] = es * NIP + i;
+        cf[q] = T::edge[i][0] == ip;
+    }
+    wave_sync();
+    if (corner) {
+        double* rd = recD + (e * N + ip) * NC;
+#pragma unroll
+        for (int a = 0; a < NC; ++a) {
+            double x = 0.0;
+#pragma unroll
+            for (int q = 0; q < T::cip; ++q) {
+                const double v = xch.d[cs[q]][a];
+                x += cf[q] ? v : -v;
+            }
+            rd[a] = x;
+        }
+    }
+    wave_sync();
+
+    if (!recJ) return;  // defect only
 
     // ---- Jacobian block of the `from` row, one column block per corner:
     //      navier_stokes_fv1.cpp:317-593
@@ -781,11 +810,8 @@ coupled_scvf(KMeshPtrs M, KParams P, const double* __restrict__ u, const double*
                 Sp[d] = sumP / diag;
             }
         } else {
-            // every accumulator takes its terms in ascending j, as in the
-            // stabilised velocity above; the ip data of j is read once for
-            // all components
-            const double* iv = &S.aug[ip][NIP];
-            double xp[D], xv[D][D];
+            // every accumulator takes its terms in ascending j
+            double xp[D], xc = 0.0, xv[D][D];
 #pragma unroll
             for (int d = 0; d < D; ++d) {
                 xp[d] = 0.0;
@@ -794,40 +820,39 @@ coupled_scvf(KMeshPtrs M, KParams P, const double* __restrict__ u, const double*
             }
 #pragma unroll
             for (int j = 0; j < NIP; ++j) {
-                const double ivj = iv[j];
-                double gj[D], svj[D];
+                const double ivj = S.inv[ip][j];
+                double gj[D];
 #pragma unroll
                 for (int d = 0; d < D; ++d) {
                     gj[d] = S.g[j][sh][d];
-                    svj[d] = S.sv[j][d];
+                    xp[d] += ivj * (RHOIP ? gj[d] * S.irho[j] : gj[d]);
                 }
-                double cd0 = S.vv[j] * S.phi[j][sh];
-                cd0 += S.vc[j] * S.Us[j][sh];
-                if (flow) cd0 += S.vd[j] * (S.Ud[j][sh] - S.Us[j][sh]);
+                if (!flow) {
+                    xc += ivj * S.cd0[j][sh];
+                    continue;
+                }
+                double svj[D];
+#pragma unroll
+                for (int d = 0; d < D; ++d) svj[d] = S.sv[j][d];
+                const double cd0 = S.cd0[j][sh];
 #pragma unroll
                 for (int d = 0; d < D; ++d) {
-                    const double cp = -1.0 * gj[d] / (RHOIP ? M.rho_ip[e * NIP + j] : rho);
                     double cd = cd0;
-                    double cvo[D];
-                    if (flow) {
 #pragma unroll
-                        for (int d2 = 0; d2 < D; ++d2) {
-                            if (d2 == d) continue;
-                            cd -= svj[d2] * gj[d2];
-                            cvo[d2] = svj[d] * gj[d2];
-                        }
+                    for (int d2 = 0; d2 < D; ++d2) {
+                        if (d2 == d) continue;
+                        cd -= svj[d2] * gj[d2];
+                        xv[d][d2] += ivj * (svj[d] * gj[d2]);
                     }
-                    xp[d] += ivj * cp;
                     xv[d][d] += ivj * cd;
-                    if (flow)
-#pragma unroll
-                        for (int d2 = 0; d2 < D; ++d2)
-                            if (d2 != d) xv[d][d2] += ivj * cvo[d2];
                 }
             }
+            if (!flow)
+#pragma unroll
+                for (int d = 0; d < D; ++d) xv[d][d] = xc;
 #pragma unroll
             for (int d = 0; d < D; ++d) {
-                Sp[d] = xp[d];
+                Sp[d] = RHOIP ? -xp[d] : -xp[d] / rho;
 #pragma unroll
                 for (int d2 = 0; d2 < D; ++d2)
                     if (flow || d2 == d) Sv[d][d2] = xv[d][d2];
@@ -924,13 +949,25 @@ coupled_scvf(KMeshPtrs M, KParams P, const double* __restrict__ u, const double*
             for (int d1 = 0; d1 < D; ++d1) cpp += Sp[d1] * n[d1] * rho;
             Jb[D][D] += cpp;
         }
-        if (recJ) {
-            JT* rj = recJ + ((e * NIP + ip) * N + sh) * (NC * NC);
 #pragma unroll
-            for (int a = 0; a < NC; ++a)
+        for (int a = 0; a < NC; ++a)
 #pragma unroll
-                for (int b = 0; b < NC; ++b) rj[a * NC + b] = JT(sa * Jb[a][b]);
+            for (int b = 0; b < NC; ++b) xch.j[lane][a * NC + b] = JT(sa * Jb[a][b]);
+        wave_sync();
+        if (corner) {
+            JT* rj = recJ + ((e * N + ip) * N + sh) * (NC * NC);
+#pragma unroll
+            for (int a = 0; a < NC * NC; ++a) {
+                JT x = JT(0);
+#pragma unroll
+                for (int q = 0; q < T::cip; ++q) {
+                    const JT v = xch.j[cs[q]][a];
+                    x += cf[q] ? v : -v;
+                }
+                rj[a] = x;
+            }
         }
+        wave_sync();
     }
 }
 
@@ -943,7 +980,7 @@ coupled_rows(KMeshPtrs M, KParams P, const double* __restrict__ u, const JT* __r
              const double* __restrict__ recD, JT* __restrict__ J, double* __restrict__ dout)
 {
     using T = Topo<ET>;
-    constexpr int D = T::dim, N = T::nsh, NC = D + 1, NIP = T::nip;
+    constexpr int D = T::dim, N = T::nsh, NC = D + 1;
     extern __shared__ __align__(16) unsigned char smem[];
     // consecutive workgroups go to the same XCD (block i runs on XCD i % 8)
     const int w = [] {
@@ -1006,26 +1043,18 @@ coupled_rows(KMeshPtrs M, KParams P, const double* __restrict__ u, const JT* __r
         const int kv = info & 0xff;
         slot = info >> 8;
         if (P.parts & 1) {
+            const int64_t r = e * N + kv;
+            if (wantJ) {
+                const JT* rj = recJ + r * N * (NC * NC);
 #pragma unroll
-            for (int ip = 0; ip < NIP; ++ip) {
-                const bool isf = T::edge[ip][0] == kv, ist = T::edge[ip][1] == kv;
-                if (!isf && !ist) continue;
-                const int64_t r = e * NIP + ip;
-                if (wantJ) {
-                    const JT* rj = recJ + r * N * (NC * NC);
+                for (int k = 0; k < N; ++k)
 #pragma unroll
-                    for (int k = 0; k < N; ++k)
+                    for (int a = 0; a < NC; ++a)
 #pragma unroll
-                        for (int a = 0; a < NC; ++a)
-#pragma unroll
-                            for (int b = 0; b < NC; ++b) {
-                                const JT x = rj[k * (NC * NC) + a * NC + b];
-                                jacc[a][k][b] += isf ? x : -x;
-                            }
-                }
-#pragma unroll
-                for (int a = 0; a < NC; ++a) dacc[a] += isf ? recD[r * NC + a] : -recD[r * NC + a];
+                        for (int b = 0; b < NC; ++b) jacc[a][k][b] = rj[k * (NC * NC) + a * NC + b];
             }
+#pragma unroll
+            for (int a = 0; a < NC; ++a) dacc[a] = recD[r * NC + a];
         }
         // mass part and source: navier_stokes_fv1.cpp:781-869
         if (P.parts & 6) {
@@ -1076,17 +1105,7 @@ coupled_rows(KMeshPtrs M, KParams P, const double* __restrict__ u, const JT* __r
         }
         __syncthreads();
     }
-    if (wantJ) {
-        if constexpr (PADE == 0) {
-            for (int i = threadIdx.x; i < jlen; i += blockDim.x) J[jbase + i] = jbuf[i];
-        } else {
-            for (int j = 0; j < v1 - v0; ++j) {
-                const int off = (int)(M.rowptr[(int64_t)(v0 + j) * NC] - jbase);
-                const int len = (int)(M.rowptr[(int64_t)(v0 + j + 1) * NC] - jbase) - off;
-                for (int i = threadIdx.x; i < len; i += blockDim.x) J[jbase + off + i] = jbuf[off + j * PADE + i];
-            }
-        }
-    }
+    if (wantJ) store_rows<NC, PADE>(M.rowptr, v0, v1 - v0, jbase, jlen, jbuf, J + jbase);
     if (dout)
         for (int i = threadIdx.x; i < dlen; i += blockDim.x) dout[(int64_t)v0 * NC + i] = dbuf[i];
 }
@@ -1111,8 +1130,8 @@ static hipError_t launch_coupled_et(const KMeshPtrs& m, const KParams& p, const 
     JT* recJ = nullptr;
     double* recD = nullptr;
     if (!vel_out) {
-        recJ = static_cast<JT*>(recs);
-        const int64_t jb = ne * NIP * N * NC * NC * (int64_t)sizeof(JT);
+        if (J) recJ = static_cast<JT*>(recs);
+        const int64_t jb = ne * N * N * NC * NC * (int64_t)sizeof(JT);
         recD = reinterpret_cast<double*>(static_cast<char*>(recs) + ((jb + 255) / 256) * 256);
     }
     if (blocks > 0) {
