@@ -867,6 +867,7 @@ static int set_mesh_groups(nsfv1_handle* h, const double* xyz, int64_t nv, const
     h->upw_dec.release();
     h->upw_recorded = false;
     h->nu_elem.release();
+    h->nt_m = 0;
     h->nu_ip.release();
     h->rho_ip.release();
     h->rho_scv.release();
