@@ -861,13 +861,13 @@ static int set_mesh_groups(nsfv1_handle* h, const double* xyz, int64_t nv, const
     h->geo_valid = false;
     // solver state sized for the previous mesh
     h->gm_restart = 0;
+    h->nt_m = 0;
     h->ndir = 0;
     h->mg.clear();
     h->mg_ready = false;
     h->upw_dec.release();
     h->upw_recorded = false;
     h->nu_elem.release();
-    h->nt_m = 0;
     h->nu_ip.release();
     h->rho_ip.release();
     h->rho_scv.release();
@@ -2264,7 +2264,7 @@ int nsfv1_linear_solve(nsfv1_handle* h, const void* jvals, int jprec, const doub
     if (h->gm_restart != m) {
         if (h->gm_V.alloc(sizeof(double) * n * (m + 1)) != hipSuccess || h->gm_w.alloc(sizeof(double) * n * 2) != hipSuccess ||
             h->gm_Binv.alloc(sizeof(double) * nv * nc * nc) != hipSuccess ||
-            h->gm_part.alloc(sizeof(double) * RED_PARTIALS) != hipSuccess ||
+            h->gm_part.alloc(sizeof(double) * red_partials(n)) != hipSuccess ||
             h->gm_small.alloc(sizeof(double) * 256) != hipSuccess)
             return fail(NSFV1_ERR_DEVICE, "GMRES workspace");
         h->gm_restart = m;
@@ -2279,9 +2279,9 @@ int nsfv1_linear_solve(nsfv1_handle* h, const void* jvals, int jprec, const doub
     const int32_t* ci = h->colidx.as<int32_t>();
     const int32_t* ad = h->adj.as<int32_t>();
     auto chk = [&](hipError_t e) { return e == hipSuccess; };
-    auto dot = [&](const double* Vb, int k, const double* vec, double* out) -> bool {
-        if (!chk(launch_multi_dot(Vb, n, k, vec, n, part, dsm, s))) return false;
-        return hipMemcpyAsync(out, dsm, sizeof(double) * k, hipMemcpyDeviceToHost, s) == hipSuccess &&
+    auto norm2 = [&](const double* vec, double* out) -> bool {
+        if (!chk(launch_norm2(vec, n, part, dsm, s))) return false;
+        return hipMemcpyAsync(out, dsm, sizeof(double), hipMemcpyDeviceToHost, s) == hipSuccess &&
                hipStreamSynchronize(s) == hipSuccess;
     };
     if (h->use_mg && (!h->mg_ready || h->mg_jprec != jprec))
@@ -2294,7 +2294,7 @@ int nsfv1_linear_solve(nsfv1_handle* h, const void* jvals, int jprec, const doub
     };
     if (hipMemsetAsync(x, 0, sizeof(double) * n, s) != hipSuccess) return fail(NSFV1_ERR_DEVICE, "memset");
     double bn2;
-    if (!dot(b, 1, b, &bn2)) return fail(NSFV1_ERR_DEVICE, "dot");
+    if (!norm2(b, &bn2)) return fail(NSFV1_ERR_DEVICE, "dot");
     const double bnorm = std::sqrt(bn2);
     int it = 0;
     double res = bnorm;
@@ -2309,7 +2309,7 @@ int nsfv1_linear_solve(nsfv1_handle* h, const void* jvals, int jprec, const doub
         if (!chk(launch_spmv(jprec, rp, ci, ad, h->dim + 1, jvals, x, w, n, h->nnz, s)) || !chk(launch_axpby(1.0, b, -1.0, w, n, s)))
             return fail(NSFV1_ERR_DEVICE, "residual");
         double rn2;
-        if (!dot(w, 1, w, &rn2)) return fail(NSFV1_ERR_DEVICE, "dot");
+        if (!norm2(w, &rn2)) return fail(NSFV1_ERR_DEVICE, "dot");
         const double beta = std::sqrt(rn2);
         res = beta;
         if (beta <= rtol * bnorm) break;
@@ -2325,15 +2325,11 @@ int nsfv1_linear_solve(nsfv1_handle* h, const void* jvals, int jprec, const doub
             constexpr int HS = GMRES_MAX_RESTART + 1;
             static_assert(128 + 2 * HS + 1 <= 256, "GMRES device scratch holds 256 doubles");
             double* hd = dsm + 128;  // [h1 (HS) | h2 (HS) | ||w||^2]
-            for (int pass = 0; pass < 2; ++pass)
-                if (!chk(launch_multi_dot(V, n, j + 1, w, n, part, hd + pass * HS, s)) ||
-                    !chk(launch_multi_axpy(V, n, j + 1, hd + pass * HS, w, n, s)))
-                    return fail(NSFV1_ERR_DEVICE, "orthogonalise");
             double hh[2 * HS + 1];
-            if (!chk(launch_multi_dot(w, n, 1, w, n, part, hd + 2 * HS, s)) ||
+            if (!chk(launch_orthogonalise(V, n, j + 1, w, n, part, hd, HS, s)) ||
                 hipMemcpyAsync(hh, hd, sizeof(hh), hipMemcpyDeviceToHost, s) != hipSuccess ||
                 hipStreamSynchronize(s) != hipSuccess)
-                return fail(NSFV1_ERR_DEVICE, "dot");
+                return fail(NSFV1_ERR_DEVICE, "orthogonalise");
             for (int i = 0; i <= j; ++i) H[i * m + j] = hh[i] + hh[HS + i];
             const double hn = std::sqrt(hh[2 * HS]);
             H[(j + 1) * m + j] = hn;
@@ -2404,7 +2400,7 @@ static int newton_prepare(nsfv1_handle* h, const double* u, const double* u_old,
     if (h->nt_m < m) {
         if (h->nt_V.alloc(sizeof(double) * n * (m + 1)) != hipSuccess || h->nt_w.alloc(sizeof(double) * n * 2) != hipSuccess ||
             h->nt_Binv.alloc(sizeof(double) * nv * nc * nc) != hipSuccess ||
-            h->nt_part.alloc(sizeof(double) * RED_PARTIALS) != hipSuccess ||
+            h->nt_part.alloc(sizeof(double) * red_partials(n)) != hipSuccess ||
             h->nt_dev.alloc(sizeof(double) * NT_DEV_DOUBLES) != hipSuccess)
             return fail(NSFV1_ERR_DEVICE, "Newton step workspace");
         h->nt_m = m;
@@ -2446,14 +2442,11 @@ static int newton_body(nsfv1_handle* h, double* u, const double* u_old, double d
         ok = ok && chk(launch_dirichlet(jprec, rp, ci, h->dir_rows.as<int64_t>(), h->ndir, jvals, d, u, g, s));
     ok = ok && chk(launch_block_jacobi_setup(jprec, nc, rp, ci, jvals, nv, Binv, h->errflag.as<int>(), s));
     // GMRES(m) from x = 0: r = d, beta = ||d||, V0 = d / beta
-    ok = ok && chk(launch_multi_dot(d, n, 1, d, n, part, n2, s)) && chk(launch_gm_beta(n2, beta, res2, s)) &&
+    ok = ok && chk(launch_norm2(d, n, part, n2, s)) && chk(launch_gm_beta(n2, beta, res2, s)) &&
          chk(launch_gm_scale(d, beta, V, n, s));
     for (int j = 0; ok && j < m; ++j) {
         ok = chk(precond(V + (int64_t)j * n, z)) && chk(launch_spmv(jprec, rp, ci, ad, nc, jvals, z, w, n, h->nnz, s));
-        for (int pass = 0; ok && pass < 2; ++pass)
-            ok = chk(launch_multi_dot(V, n, j + 1, w, n, part, hd + pass * NT_HS, s)) &&
-                 chk(launch_multi_axpy(V, n, j + 1, hd + pass * NT_HS, w, n, s));
-        ok = ok && chk(launch_multi_dot(w, n, 1, w, n, part, hd + 2 * NT_HS, s)) &&
+        ok = ok && chk(launch_orthogonalise(V, n, j + 1, w, n, part, hd, NT_HS, s)) &&
              chk(launch_gm_hcol(hd, NT_HS, H, m, j, s)) &&
              chk(launch_gm_scale(w, H + (int64_t)(j + 1) * m + j, V + (int64_t)(j + 1) * n, n, s));
     }

@@ -8,7 +8,7 @@
 namespace nsfv1 {
 
 constexpr int GMRES_MAX_RESTART = 60;
-constexpr int RED_PARTIALS = 1024 * 64;
+int64_t red_partials(int64_t n);  // doubles of the partial sums of vectors of n entries
 constexpr int MG_MAX_LEVELS = 12;
 constexpr int MG_DENSE_MAX = 1200;  // largest coarsest-level system inverted densely
 
@@ -21,9 +21,12 @@ hipError_t launch_spmv(int jprec, const int64_t* rowptr, const int32_t* colidx, 
 hipError_t launch_block_jacobi_setup(int jprec, int nc, const int64_t* rowptr, const int32_t* colidx, const void* A,
                                      int64_t nv, double* Binv, int* err, hipStream_t s);
 hipError_t launch_block_jacobi_apply(int nc, const double* Binv, const double* x, double* y, int64_t nv, hipStream_t s);
-hipError_t launch_multi_dot(const double* V, int64_t ld, int k, const double* w, int64_t n, double* partial,
-                            double* out, hipStream_t s);
-hipError_t launch_multi_axpy(const double* V, int64_t ld, int k, const double* h, double* w, int64_t n, hipStream_t s);
+// *out = ||w||^2; partial: red_partials(n) doubles
+hipError_t launch_norm2(const double* w, int64_t n, double* partial, double* out, hipStream_t s);
+// w orthogonalised against V_0 .. V_{k-1} (leading dimension ld), twice: the
+// projections of both passes to h[0..k) and h[hs..hs + k), ||w||^2 to h[2 hs]
+hipError_t launch_orthogonalise(const double* V, int64_t ld, int k, double* w, int64_t n, double* partial, double* h,
+                                int hs, hipStream_t s);
 hipError_t launch_multi_add(const double* V, int64_t ld, int k, const double* c, double* x, int64_t n, hipStream_t s);
 hipError_t launch_axpby(double a, const double* x, double b, double* y, int64_t n, hipStream_t s);
 // device-side pieces of the fixed-iteration GMRES of the capturable Newton
