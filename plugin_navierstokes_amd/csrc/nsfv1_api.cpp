@@ -160,7 +160,8 @@ struct nsfv1_handle {
     Plan plan32, plan64;
     // Newton-loop linear algebra
     DevBuf cpl_recs;  // coupled path: per-SCVF row blocks
-    DevBuf dir_rows, gm_V, gm_Binv, gm_part, gm_small, gm_w;
+    DevBuf dir_rows, dir_mask;  // Dirichlet rows, and 1 per Dirichlet DoF
+    DevBuf gm_V, gm_Binv, gm_part, gm_small, gm_w;
     int64_t ndir = 0;
     int gm_restart = 0;
     // geometric multigrid preconditioner
@@ -1849,8 +1850,12 @@ int nsfv1_set_dirichlet(nsfv1_handle* h, const int64_t* dofs, int64_t n)
     std::vector<int64_t> d(dofs, dofs + (n > 0 ? n : 0));
     for (int64_t x : d)
         if (x < 0 || x >= h->ndof) return fail(NSFV1_ERR_ARGUMENT, "Dirichlet DoF out of range");
+    std::vector<uint8_t> mask((size_t)h->ndof, 0);
+    for (int64_t x : d) mask[(size_t)x] = 1;
     if (h->dir_rows.alloc(sizeof(int64_t) * std::max<int64_t>(n, 1)) != hipSuccess ||
-        (n > 0 && hipMemcpy(h->dir_rows.p, d.data(), sizeof(int64_t) * n, hipMemcpyHostToDevice) != hipSuccess))
+        h->dir_mask.alloc(mask.size()) != hipSuccess ||
+        (n > 0 && hipMemcpy(h->dir_rows.p, d.data(), sizeof(int64_t) * n, hipMemcpyHostToDevice) != hipSuccess) ||
+        (n > 0 && hipMemcpy(h->dir_mask.p, mask.data(), mask.size(), hipMemcpyHostToDevice) != hipSuccess))
         return fail(NSFV1_ERR_DEVICE, "Dirichlet upload");
     h->ndir = n;
     return NSFV1_OK;
@@ -2110,21 +2115,21 @@ static hipError_t mg_cycle(nsfv1_handle* h, size_t l, const void* J0, const doub
     MGLevel& C = *h->mg[l];
     nsfv1_handle* cc = C.h;
     // Dirichlet rows neither send residual to nor take corrections from the
-    // coarse level (their equations are decoupled identities)
-    e = launch_residual(jp, rp, ci, ad, nc, J, x, b, r, n, c->nnz, s);
-    if (e == hipSuccess) e = launch_zero_rows(c->dir_rows.as<int64_t>(), c->ndir, r, s);
-    if (e == hipSuccess) e = launch_node_transfer(C.R_rp.as<int64_t>(), C.R_ci.as<int32_t>(), C.R_w.as<double>(), r, C.b.as<double>(), cc->nv, nc, 0, s);
-    if (e == hipSuccess) e = launch_zero_rows(cc->dir_rows.as<int64_t>(), cc->ndir, C.b.as<double>(), s);
+    // coarse level (their equations are decoupled identities): the transfers
+    // and the residual carry their masks, so a level is a handful of launches.
+    // The corrected iterate goes where the sweeps' alternation ends in x
+    const uint8_t* mask = c->ndir ? c->dir_mask.as<uint8_t>() : nullptr;
+    const uint8_t* cmask = cc->ndir ? cc->dir_mask.as<uint8_t>() : nullptr;
+    e = launch_residual(jp, rp, ci, ad, nc, J, x, b, r, n, c->nnz, mask, s);
+    if (e == hipSuccess) e = launch_node_transfer(C.R_rp.as<int64_t>(), C.R_ci.as<int32_t>(), C.R_w.as<double>(), r, nullptr, cmask, C.b.as<double>(), cc->nv, nc, s);
     if (e == hipSuccess) e = mg_cycle(h, l + 1, J0, Binv0, C.b.as<double>(), C.x.as<double>(), s);
-    if (e == hipSuccess) e = launch_node_transfer(C.P_rp.as<int64_t>(), C.P_ci.as<int32_t>(), C.P_w.as<double>(), C.x.as<double>(), r, nv, nc, 0, s);
-    if (e == hipSuccess) e = launch_zero_rows(c->dir_rows.as<int64_t>(), c->ndir, r, s);
-    if (e == hipSuccess) e = launch_axpby(1.0, r, 1.0, x, n, s);
-    cur = x, alt = t;
+    cur = (h->mg_post & 1) ? t : x;
+    alt = (h->mg_post & 1) ? x : t;
+    if (e == hipSuccess) e = launch_node_transfer(C.P_rp.as<int64_t>(), C.P_ci.as<int32_t>(), C.P_w.as<double>(), C.x.as<double>(), x, mask, cur, nv, nc, s);
     for (int k = 0; k < h->mg_post && e == hipSuccess; ++k) {
         e = launch_smooth(jp, rp, ci, ad, nc, J, cur, b, Bi, w, r, alt, n, c->nnz, s);
         std::swap(cur, alt);
     }
-    if (e == hipSuccess && cur != x) e = hipMemcpyAsync(x, cur, sizeof(double) * n, hipMemcpyDeviceToDevice, s);
     return e;
 }
 

@@ -373,8 +373,8 @@ __global__ void multi_add(const double* __restrict__ V, int64_t ld, int k, const
 // row when NC = 4), and keeps NC FP64 partial sums.  The G partials are then
 // combined by a reduce-scatter across the group (two exchange steps that
 // halve the set of rows a lane carries, then a butterfly), in a fixed order.
-// y = A x (RES = 0), y = b - A x (RES = 1), or one damped point-block
-// Jacobi sweep y = x + omega Binv (b - A x) (RES = 2; y must not alias x).
+// y = A x (RES = 0), y = b - A x with zeros in the rows of a mask (RES = 1),
+// or one damped point-block Jacobi sweep y = x + omega Binv (b - A x) (RES = 2; y must not alias x).
 template <typename JT, int NC>
 __device__ __forceinline__ void block_row(const JT* __restrict__ p, double (&q)[NC])
 {
@@ -398,7 +398,7 @@ template <typename JT, int NC, int G, int RES>
 __global__ void __launch_bounds__(256)
 nodeblock_mv(const int64_t* __restrict__ rowptr, const int32_t* __restrict__ adj, const JT* __restrict__ A,
              const double* __restrict__ x, const double* __restrict__ b, double* __restrict__ y, int64_t nv,
-             const double* __restrict__ Binv, double omega)
+             const double* __restrict__ Binv, double omega, const uint8_t* __restrict__ mask)
 {
     static_assert(NC == 3 || NC == 4, "node blocks of 3 or 4 unknowns");
     static_assert(G >= 4 && G <= 64 && (G & (G - 1)) == 0, "group size");
@@ -462,14 +462,15 @@ nodeblock_mv(const int64_t* __restrict__ rowptr, const int32_t* __restrict__ adj
         }
     } else if (v < nv && (sub & (G / 4 - 1)) == 0 && a < NC) {
         const int64_t row = v * NC + a;
-        y[row] = RES ? b[row] - z : z;
+        y[row] = RES ? (mask && mask[row] ? 0.0 : b[row] - z) : z;
     }
 }
 
 template <typename JT>
 __global__ void __launch_bounds__(256)
 residual_csr(const int64_t* __restrict__ rowptr, const int32_t* __restrict__ colidx, const JT* __restrict__ A,
-             const double* __restrict__ x, const double* __restrict__ b, double* __restrict__ r, int64_t n)
+             const double* __restrict__ x, const double* __restrict__ b, double* __restrict__ r, int64_t n,
+             const uint8_t* __restrict__ mask)
 {
     const int64_t row = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 4;
     const int sub = threadIdx.x & 15;
@@ -480,7 +481,7 @@ residual_csr(const int64_t* __restrict__ rowptr, const int32_t* __restrict__ col
     }
 #pragma unroll
     for (int o = 8; o > 0; o >>= 1) s += __shfl_xor(s, o, 16);
-    if (row < n && sub == 0) r[row] = b[row] - s;
+    if (row < n && sub == 0) r[row] = mask && mask[row] ? 0.0 : b[row] - s;
 }
 
 // x = (first ? 0 : x) + omega * Binv r, per node block
@@ -502,10 +503,11 @@ __global__ void bj_update(const double* __restrict__ Binv, const double* __restr
     }
 }
 
-// y[row, c] (= or +=) sum_k w_k x[col_k, c] for every component c < nc
+// y[row, c] = base[row, c] + sum_k w_k x[col_k, c] for every component c < nc
+// (base may be null: 0); where the mask is set the sum is dropped
 __global__ void node_transfer(const int64_t* __restrict__ rowptr, const int32_t* __restrict__ colidx,
-                              const double* __restrict__ w, const double* __restrict__ x, double* __restrict__ y,
-                              int64_t nrows, int nc, int accumulate)
+                              const double* __restrict__ w, const double* __restrict__ x, const double* base,
+                              const uint8_t* __restrict__ mask, double* y, int64_t nrows, int nc)
 {
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= nrows * nc) return;
@@ -516,13 +518,8 @@ __global__ void node_transfer(const int64_t* __restrict__ rowptr, const int32_t*
     // unrolled so that several index -> value load chains are in flight
 #pragma unroll 4
     for (int64_t k = a; k < b; ++k) s += w[k] * x[(int64_t)colidx[k] * nc + c];
-    y[t] = accumulate ? y[t] + s : s;
-}
-
-__global__ void zero_rows(const int64_t* __restrict__ rows, int64_t nrows, double* __restrict__ y)
-{
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < nrows) y[rows[t]] = 0.0;
+    if (mask && mask[t]) s = 0.0;
+    y[t] = base ? base[t] + s : s;
 }
 
 // coarse state: uc[w, c] = uf[inj[w], c]
@@ -922,15 +919,16 @@ hipError_t launch_dirichlet(int jprec, const int64_t* rowptr, const int32_t* col
 // covers the mean number of neighbour blocks per node
 template <typename JT, int NC, int RES>
 static void launch_nodeblock(const int64_t* rowptr, const int32_t* adj, const JT* A, const double* x, const double* b,
-                             double* y, int64_t nv, int64_t nnz, const double* Binv, double omega, hipStream_t s)
+                             double* y, int64_t nv, int64_t nnz, const double* Binv, double omega,
+                             const uint8_t* mask, hipStream_t s)
 {
     const int64_t slots = nv > 0 ? nnz / ((int64_t)NC * NC * nv) : 0;
     if (slots > 16)
-        nodeblock_mv<JT, NC, 32, RES><<<blocks_for(nv * 32, 256), 256, 0, s>>>(rowptr, adj, A, x, b, y, nv, Binv, omega);
+        nodeblock_mv<JT, NC, 32, RES><<<blocks_for(nv * 32, 256), 256, 0, s>>>(rowptr, adj, A, x, b, y, nv, Binv, omega, mask);
     else if (slots > 8)
-        nodeblock_mv<JT, NC, 16, RES><<<blocks_for(nv * 16, 256), 256, 0, s>>>(rowptr, adj, A, x, b, y, nv, Binv, omega);
+        nodeblock_mv<JT, NC, 16, RES><<<blocks_for(nv * 16, 256), 256, 0, s>>>(rowptr, adj, A, x, b, y, nv, Binv, omega, mask);
     else
-        nodeblock_mv<JT, NC, 8, RES><<<blocks_for(nv * 8, 256), 256, 0, s>>>(rowptr, adj, A, x, b, y, nv, Binv, omega);
+        nodeblock_mv<JT, NC, 8, RES><<<blocks_for(nv * 8, 256), 256, 0, s>>>(rowptr, adj, A, x, b, y, nv, Binv, omega, mask);
 }
 
 // with 4 unknowns per node the node-block kernels take 16-byte vector loads
@@ -943,15 +941,15 @@ static bool nodeblock_ok(const int32_t* adj, int nc, const void* A, const double
 template <int RES>
 static void launch_mv(int jprec, const int64_t* rowptr, const int32_t* adj, int nc, const void* A, const double* x,
                       const double* b, double* y, int64_t n, int64_t nnz, hipStream_t s,
-                      const double* Binv = nullptr, double omega = 0.0)
+                      const double* Binv = nullptr, double omega = 0.0, const uint8_t* mask = nullptr)
 {
     const int64_t nv = n / nc;
     if (nc == 4) {
-        if (jprec == 64) launch_nodeblock<double, 4, RES>(rowptr, adj, (const double*)A, x, b, y, nv, nnz, Binv, omega, s);
-        else launch_nodeblock<float, 4, RES>(rowptr, adj, (const float*)A, x, b, y, nv, nnz, Binv, omega, s);
+        if (jprec == 64) launch_nodeblock<double, 4, RES>(rowptr, adj, (const double*)A, x, b, y, nv, nnz, Binv, omega, mask, s);
+        else launch_nodeblock<float, 4, RES>(rowptr, adj, (const float*)A, x, b, y, nv, nnz, Binv, omega, mask, s);
     } else {
-        if (jprec == 64) launch_nodeblock<double, 3, RES>(rowptr, adj, (const double*)A, x, b, y, nv, nnz, Binv, omega, s);
-        else launch_nodeblock<float, 3, RES>(rowptr, adj, (const float*)A, x, b, y, nv, nnz, Binv, omega, s);
+        if (jprec == 64) launch_nodeblock<double, 3, RES>(rowptr, adj, (const double*)A, x, b, y, nv, nnz, Binv, omega, mask, s);
+        else launch_nodeblock<float, 3, RES>(rowptr, adj, (const float*)A, x, b, y, nv, nnz, Binv, omega, mask, s);
     }
 }
 
@@ -1079,14 +1077,14 @@ hipError_t launch_gm_lsq(double* H, const double* beta, int m, double* y, hipStr
 
 hipError_t launch_residual(int jprec, const int64_t* rowptr, const int32_t* colidx, const int32_t* adj, int nc,
                            const void* A, const double* x, const double* b, double* r, int64_t n, int64_t nnz,
-                           hipStream_t s)
+                           const uint8_t* mask, hipStream_t s)
 {
     if (nodeblock_ok(adj, nc, A, x)) {
-        launch_mv<1>(jprec, rowptr, adj, nc, A, x, b, r, n, nnz, s);
+        launch_mv<1>(jprec, rowptr, adj, nc, A, x, b, r, n, nnz, s, nullptr, 0.0, mask);
     } else {
         const int bl = blocks_for(n * 16, 256);
-        if (jprec == 64) residual_csr<double><<<bl, 256, 0, s>>>(rowptr, colidx, (const double*)A, x, b, r, n);
-        else residual_csr<float><<<bl, 256, 0, s>>>(rowptr, colidx, (const float*)A, x, b, r, n);
+        if (jprec == 64) residual_csr<double><<<bl, 256, 0, s>>>(rowptr, colidx, (const double*)A, x, b, r, n, mask);
+        else residual_csr<float><<<bl, 256, 0, s>>>(rowptr, colidx, (const float*)A, x, b, r, n, mask);
     }
     return hipGetLastError();
 }
@@ -1099,7 +1097,7 @@ hipError_t launch_smooth(int jprec, const int64_t* rowptr, const int32_t* colidx
         launch_mv<2>(jprec, rowptr, adj, nc, A, x, b, y, n, nnz, s, Binv, omega);
         return hipGetLastError();
     }
-    hipError_t e = launch_residual(jprec, rowptr, colidx, adj, nc, A, x, b, r, n, nnz, s);
+    hipError_t e = launch_residual(jprec, rowptr, colidx, adj, nc, A, x, b, r, n, nnz, nullptr, s);
     if (e == hipSuccess) e = hipMemcpyAsync(y, x, sizeof(double) * n, hipMemcpyDeviceToDevice, s);
     if (e == hipSuccess) e = launch_bj_update(nc, Binv, r, y, omega, 0, n / nc, s);
     return e;
@@ -1115,16 +1113,9 @@ hipError_t launch_bj_update(int nc, const double* Binv, const double* r, double*
 }
 
 hipError_t launch_node_transfer(const int64_t* rowptr, const int32_t* colidx, const double* w, const double* x,
-                                double* y, int64_t nrows, int nc, int accumulate, hipStream_t s)
+                                const double* base, const uint8_t* mask, double* y, int64_t nrows, int nc, hipStream_t s)
 {
-    node_transfer<<<blocks_for(nrows * nc, 256), 256, 0, s>>>(rowptr, colidx, w, x, y, nrows, nc, accumulate);
-    return hipGetLastError();
-}
-
-hipError_t launch_zero_rows(const int64_t* rows, int64_t nrows, double* y, hipStream_t s)
-{
-    if (nrows <= 0) return hipSuccess;
-    zero_rows<<<blocks_for(nrows, 256), 256, 0, s>>>(rows, nrows, y);
+    node_transfer<<<blocks_for(nrows * nc, 256), 256, 0, s>>>(rowptr, colidx, w, x, base, mask, y, nrows, nc);
     return hipGetLastError();
 }
 

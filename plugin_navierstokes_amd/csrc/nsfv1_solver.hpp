@@ -39,9 +39,10 @@ hipError_t launch_gm_beta(const double* n2, double* beta, double* res2, hipStrea
 hipError_t launch_gm_hcol(const double* hd, int hs, double* H, int m, int j, hipStream_t s);
 hipError_t launch_gm_scale(const double* x, const double* h, double* y, int64_t n, hipStream_t s);
 hipError_t launch_gm_lsq(double* H, const double* beta, int m, double* y, hipStream_t s);
+// r = b - A x, 0 in the rows of the mask (null: none)
 hipError_t launch_residual(int jprec, const int64_t* rowptr, const int32_t* colidx, const int32_t* adj, int nc,
                            const void* A, const double* x, const double* b, double* r, int64_t n, int64_t nnz,
-                           hipStream_t s);
+                           const uint8_t* mask, hipStream_t s);
 // one damped point-block Jacobi sweep y = x + omega Binv (b - A x) (y must not
 // alias x; r: scratch of n doubles, used only without node blocks)
 hipError_t launch_smooth(int jprec, const int64_t* rowptr, const int32_t* colidx, const int32_t* adj, int nc,
@@ -49,9 +50,9 @@ hipError_t launch_smooth(int jprec, const int64_t* rowptr, const int32_t* colidx
                          double* y, int64_t n, int64_t nnz, hipStream_t s);
 hipError_t launch_bj_update(int nc, const double* Binv, const double* r, double* x, double omega, int first,
                             int64_t nv, hipStream_t s);
+// y = base + W x (base null: W x; y may be base), W x dropped where the mask (null: none) is set
 hipError_t launch_node_transfer(const int64_t* rowptr, const int32_t* colidx, const double* w, const double* x,
-                                double* y, int64_t nrows, int nc, int accumulate, hipStream_t s);
-hipError_t launch_zero_rows(const int64_t* rows, int64_t nrows, double* y, hipStream_t s);
+                                const double* base, const uint8_t* mask, double* y, int64_t nrows, int nc, hipStream_t s);
 hipError_t launch_inject(const int64_t* inj, const double* uf, double* uc, int64_t nvc, int nc, hipStream_t s);
 hipError_t launch_dense_matvec(const double* A, const double* x, double* y, int n, hipStream_t s);
 // inverse of the n x n CSR matrix (n <= MG_DENSE_MAX) into the dense row-major
