@@ -1,6 +1,6 @@
 // nsfv1_mlp.hip -- learned Newton initial guess: a per-node MLP
 // 24 -> 128 -> 128 -> 4 (ReLU), BF16 weights and activations with FP32
-// accumulation on the MFMA units (v_mfma_f32_16x16x16_bf16), plus the
+// accumulation on the MFMA units (v_mfma_f32_16x16x32_bf16), plus the
 // backward pass on the MFMA units with FP32 operands
 // (v_mfma_f32_16x16x4_f32), deterministic gradient reduction and Adam used to train it
 // on trajectories of the plain solver, and the feature / guess kernels that
@@ -14,10 +14,10 @@
 // matrices are read.
 //
 // MFMA mapping (one wavefront = 16 nodes).  The layers are evaluated in
-// transposed form, H^T = W X^T, so that the accumulator layout of one layer
-// (lane l holds rows 4*(l/16)+j, column l%16) is exactly the B-operand
-// layout of the next (k = 4*(l/16)+j, column l%16): activations never leave
-// registers.  A operands (weights) come from LDS.
+// transposed form, H^T = W X^T, so that the accumulators of two tiles of one
+// layer (lane l holds rows 4*(l/16)+j, column l%16 of each) are the B operand
+// of the next (8 products per lane, column l%16), the weights being loaded in
+// the same order: activations never leave registers.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -42,93 +42,94 @@ __device__ inline float relu_bf(float z) { return bf2f(f2bf(z > 0.f ? z : 0.f));
 
 // ---------------------------------------------------------------------
 // forward: y[n][0..3] = W3 relu(W2 relu(W1 x + b1) + b2) + b3
+//
+// A wave holds the weights of layers 2 and 3 as MFMA A operands in registers
+// (144 VGPRs, two waves per SIMD), loaded once from the BF16 copy, and walks
+// 16-node blocks; layer 1 (a tile is 1 KB in lane order, read without bank
+// conflicts) and the biases, which start the accumulators, sit in LDS.
+// Bound by the conversions between layers and the matrix products, 44 MFMA of
+// 16x16x32 a block: 65536 nodes with the cached pre-activations (68 MB
+// written) 43.5 -> 31 us, 233000 nodes without them 66 -> 34 us against 64 nodes
+// a workgroup with weights and activations in LDS.
 // ---------------------------------------------------------------------
-__global__ void __launch_bounds__(256)
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
+// four weights at p and four at q (8-byte aligned) as one A operand
+__device__ __forceinline__ bf16x8 load_a(const uint16_t* __restrict__ p, const uint16_t* __restrict__ q)
+{
+    const uint2 lo = *reinterpret_cast<const uint2*>(p), hi = *reinterpret_cast<const uint2*>(q);
+    return __builtin_bit_cast(bf16x8, make_uint4(lo.x, lo.y, hi.x, hi.y));
+}
+
+__global__ void __launch_bounds__(256, 2)
 mlp_forward(const float* __restrict__ P, const uint16_t* __restrict__ WB, const float* __restrict__ X, int64_t n,
             float* __restrict__ Y, float* __restrict__ Z1, float* __restrict__ Z2)
 {
+    __shared__ __align__(16) float bias[2 * MLP_H + MLP_KOUT];
     __shared__ __align__(16) uint16_t w1[MLP_H * MLP_KIN];
-    __shared__ __align__(16) uint16_t w2[MLP_H * MLP_H];
-    __shared__ __align__(16) uint16_t w3[MLP_KOUT * MLP_H];
-    __shared__ float bias[2 * MLP_H + MLP_KOUT];
-    for (int i = threadIdx.x; i < MLP_H * MLP_KIN; i += blockDim.x) w1[i] = WB[MLP_OFF_W1 + i];
-    for (int i = threadIdx.x; i < MLP_H * MLP_H; i += blockDim.x) w2[i] = WB[MLP_OFF_W2 + i];
-    for (int i = threadIdx.x; i < MLP_KOUT * MLP_H; i += blockDim.x) w3[i] = WB[MLP_OFF_W3 + i];
+    for (int i = threadIdx.x; i < MLP_H * MLP_KIN / 2; i += blockDim.x)
+        reinterpret_cast<uint32_t*>(w1)[i] = reinterpret_cast<const uint32_t*>(WB + MLP_OFF_W1)[i];
     for (int i = threadIdx.x; i < MLP_H; i += blockDim.x) {
         bias[i] = P[MLP_OFF_B1 + i];
         bias[MLP_H + i] = P[MLP_OFF_B2 + i];
     }
     if (threadIdx.x < MLP_KOUT) bias[2 * MLP_H + threadIdx.x] = P[MLP_OFF_B3 + threadIdx.x];
+    const int lane = threadIdx.x & 63, col = lane & 15, g = lane >> 4;
+    // A operands: row col of the tile; the 8 products of lane group g sum over
+    // inputs 8 g .. (layer 1) and, so that an accumulator pair is the next
+    // layer's B operand as it stands, over hidden units 32 m + 4 g .. and
+    // 32 m + 16 + 4 g .. (layers 2 and 3)
+    bf16x8 a2[MLP_H / 16][MLP_H / 32], a3[MLP_H / 32];
+#pragma unroll
+    for (int t = 0; t < MLP_H / 16; ++t) {
+#pragma unroll
+        for (int m = 0; m < MLP_H / 32; ++m) {
+            const uint16_t* w2 = WB + MLP_OFF_W2 + (t * 16 + col) * MLP_H + 32 * m + 4 * g;
+            a2[t][m] = load_a(w2, w2 + 16);
+        }
+    }
+#pragma unroll
+    for (int m = 0; m < MLP_H / 32; ++m) {
+        const uint16_t* w3 = WB + MLP_OFF_W3 + col * MLP_H + 32 * m + 4 * g;
+        a3[m] = load_a(w3, w3 + 16);
+    }
     __syncthreads();
 
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int col = lane & 15, kq = (lane >> 4) * 4;
-    // the weights are staged once per workgroup (the compiler keeps each
-    // lane's A operands in registers across the loop); the workgroup then
-    // walks 64-node blocks (grid-stride), so the staging is amortised
-    const int64_t nblk = (n + 63) / 64;
-    for (int64_t blk = blockIdx.x; blk < nblk; blk += gridDim.x) {
-    const int64_t node = (blk * 4 + wave) * 16 + col;
-    const bool valid = node < n;
-
-    // layer 1: B = X^T tiles (k = input feature, column = node), two k-blocks
-    bf16x4 xb[MLP_KIN / 16];
+    const int64_t nblk = (n + 15) / 16, nw = (int64_t)gridDim.x * 4;
+    for (int64_t blk = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); blk < nblk; blk += nw) {
+        asm volatile("" ::: "memory");  // layer 1 and the biases stay in LDS: hoisted, they spill
+        const int64_t node = blk * 16 + col;
+        const bool valid = node < n;
+        // columns past the end repeat the last node (their results are dropped)
+        const float* xp = X + (valid ? node : n - 1) * MLP_KIN + 8 * g;
+        const float4 x0 = *reinterpret_cast<const float4*>(xp), x1 = *reinterpret_cast<const float4*>(xp + 4);
+        bf16x8 xb;
+        xb[0] = (__bf16)x0.x; xb[1] = (__bf16)x0.y; xb[2] = (__bf16)x0.z; xb[3] = (__bf16)x0.w;
+        xb[4] = (__bf16)x1.x; xb[5] = (__bf16)x1.y; xb[6] = (__bf16)x1.z; xb[7] = (__bf16)x1.w;
+        bf16x8 h1[MLP_H / 32], h2[MLP_H / 32];
 #pragma unroll
-    for (int ks = 0; ks < MLP_KIN / 16; ++ks) {
-        float xv[4] = {0.f, 0.f, 0.f, 0.f};
-        if (valid) {
-            const float4 t = *reinterpret_cast<const float4*>(X + node * MLP_KIN + ks * 16 + kq);
-            xv[0] = t.x; xv[1] = t.y; xv[2] = t.z; xv[3] = t.w;
+        for (int t = 0; t < MLP_H / 16; ++t) {
+            f32x4 acc = *reinterpret_cast<const f32x4*>(&bias[t * 16 + 4 * g]);
+            const bf16x8 a1 = *reinterpret_cast<const bf16x8*>(&w1[(t * 16 + col) * MLP_KIN + 8 * g]);
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, xb, acc, 0, 0, 0);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) h1[t >> 1][(t & 1) * 4 + j] = (__bf16)(acc[j] > 0.f ? acc[j] : 0.f);
+            if (Z1 && valid) *reinterpret_cast<f32x4*>(Z1 + node * MLP_H + t * 16 + 4 * g) = acc;
         }
 #pragma unroll
-        for (int j = 0; j < 4; ++j) xb[ks][j] = (short)f2bf(xv[j]);
-    }
-    bf16x4 h1[MLP_H / 16];
+        for (int t = 0; t < MLP_H / 16; ++t) {
+            f32x4 acc = *reinterpret_cast<const f32x4*>(&bias[MLP_H + t * 16 + 4 * g]);
 #pragma unroll
-    for (int ot = 0; ot < MLP_H / 16; ++ot) {
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+            for (int m = 0; m < MLP_H / 32; ++m) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2[t][m], h1[m], acc, 0, 0, 0);
 #pragma unroll
-        for (int ks = 0; ks < MLP_KIN / 16; ++ks) {
-            const bf16x4 a = *reinterpret_cast<const bf16x4*>(&w1[(ot * 16 + col) * MLP_KIN + ks * 16 + kq]);
-            acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, xb[ks], acc, 0, 0, 0);
+            for (int j = 0; j < 4; ++j) h2[t >> 1][(t & 1) * 4 + j] = (__bf16)(acc[j] > 0.f ? acc[j] : 0.f);
+            if (Z2 && valid) *reinterpret_cast<f32x4*>(Z2 + node * MLP_H + t * 16 + 4 * g) = acc;
         }
-        float z[4];
+        // layer 3 (rows 0..3 of the padded 16-row output)
+        f32x4 acc = *reinterpret_cast<const f32x4*>(&bias[2 * MLP_H + 4 * g]);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            z[j] = acc[j] + bias[ot * 16 + kq + j];
-            h1[ot][j] = (short)f2bf(z[j] > 0.f ? z[j] : 0.f);
-        }
-        if (Z1 && valid) *reinterpret_cast<float4*>(Z1 + node * MLP_H + ot * 16 + kq) = make_float4(z[0], z[1], z[2], z[3]);
-    }
-    // layer 2
-    bf16x4 h2[MLP_H / 16];
-#pragma unroll
-    for (int ot = 0; ot < MLP_H / 16; ++ot) {
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int ks = 0; ks < MLP_H / 16; ++ks) {
-            const bf16x4 a = *reinterpret_cast<const bf16x4*>(&w2[(ot * 16 + col) * MLP_H + ks * 16 + kq]);
-            acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, h1[ks], acc, 0, 0, 0);
-        }
-        float z[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            z[j] = acc[j] + bias[MLP_H + ot * 16 + kq + j];
-            h2[ot][j] = (short)f2bf(z[j] > 0.f ? z[j] : 0.f);
-        }
-        if (Z2 && valid) *reinterpret_cast<float4*>(Z2 + node * MLP_H + ot * 16 + kq) = make_float4(z[0], z[1], z[2], z[3]);
-    }
-    // layer 3 (rows 0..3 of the padded 16-row output)
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int ks = 0; ks < MLP_H / 16; ++ks) {
-        const bf16x4 a = *reinterpret_cast<const bf16x4*>(&w3[col * MLP_H + ks * 16 + kq]);
-        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, h2[ks], acc, 0, 0, 0);
-    }
-    if (valid && kq == 0)
-        *reinterpret_cast<float4*>(Y + node * MLP_OUT) =
-            make_float4(acc[0] + bias[2 * MLP_H + 0], acc[1] + bias[2 * MLP_H + 1], acc[2] + bias[2 * MLP_H + 2],
-                        acc[3] + bias[2 * MLP_H + 3]);
+        for (int m = 0; m < MLP_H / 32; ++m) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a3[m], h2[m], acc, 0, 0, 0);
+        if (valid && g == 0) *reinterpret_cast<f32x4*>(Y + node * MLP_OUT) = acc;
     }
 }
 
@@ -194,118 +195,162 @@ mlp_backward_act(const uint16_t* __restrict__ WB, const float* __restrict__ Z1, 
 }
 
 // ---------------------------------------------------------------------
-// weight gradients on the MFMA units: for a chunk of nodes per workgroup,
+// weight gradients on the MFMA units (FP32 operands, 16x16x4):
 //   dW1 = dZ1^T X,  dW2 = dZ2^T H1,  dW3 = dY^T H2
-// as 16x16 output tiles accumulated over the nodes (k = node, 4 per MFMA):
-// W1 8x2 tiles, W2 8x8, W3 1x8 (rows 4..15 zero): 88 tiles, 22 per
-// wavefront.  Nodes are staged in LDS 16 at a time; the biases' sums are
-// taken by 144 threads on the VALU.  Partials go to part[block][MLP_NPARAM]
-// and are reduced in block order afterwards (deterministic).
+// as 88 16x16 tiles (W1 8x2, W2 8x8, W3 1x8 with rows 4..15 zero) summed over
+// the nodes (k = node, 4 per MFMA).  A wave holds all 88 accumulators (352
+// registers, one wave per SIMD) and takes its operands straight from memory:
+// lane (col, g) reads entry col of a tile of node g, 64 contiguous bytes per
+// node, which is the operand layout of both sides, so every value is read
+// once and nothing is staged in LDS.  The next four nodes are loaded beside
+// the products of the current ones.  The bias sums ride on the operands.
+// The waves' tiles are added through LDS, partials go to
+// part[block][MLP_NPARAM] and are reduced in block order (deterministic).
+// Bound by the FP32 products (88 tiles, 2.95 GFLOP for 65536 nodes): 203 -> 59 us
+// at 65536 nodes against tiles staged in LDS.
 // ---------------------------------------------------------------------
-constexpr int WG_SUB = 16;                      // nodes staged in LDS at a time
-constexpr int WG_TILES = 16 + 64 + 8;           // output tiles of W1, W2, W3
-constexpr int WG_TPW = WG_TILES / 4;            // tiles per wavefront
-constexpr int WG_LD = MLP_H + 4;                // padded LDS row (floats)
+constexpr int WG_T1 = 16, WG_T2 = 64, WG_TILES = WG_T1 + WG_T2 + 8;  // tiles of W1, W2, all
+constexpr int WG_GROUP = 8;                                          // tiles combined at a time
 
-__global__ void __launch_bounds__(256)
+struct WgradNode {
+    float dz1[8], dz2[8], z1[8], z2[8], x[2], dy;
+};
+
+__device__ __forceinline__ void wgrad_load(WgradNode& N, const float* __restrict__ X, const float* __restrict__ Z1,
+                                           const float* __restrict__ Z2, const float* __restrict__ DY,
+                                           const float* __restrict__ DZ1, const float* __restrict__ DZ2, int64_t node,
+                                           int64_t end, int64_t n, int col)
+{
+    // nodes past the end read the last one and contribute zero gradients
+    const bool ok = node < end;
+    const int64_t r = ok ? node : n - 1;
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+        const float a = DZ1[r * MLP_H + 16 * t + col], b = DZ2[r * MLP_H + 16 * t + col];
+        N.dz1[t] = ok ? a : 0.f;
+        N.dz2[t] = ok ? b : 0.f;
+        N.z1[t] = Z1[r * MLP_H + 16 * t + col];
+        N.z2[t] = Z2[r * MLP_H + 16 * t + col];
+    }
+    N.x[0] = X[r * MLP_KIN + col];
+    N.x[1] = X[r * MLP_KIN + 16 + col];
+    const float d = DY[r * MLP_OUT + (col & 3)];
+    N.dy = ok && col < MLP_OUT ? d : 0.f;
+}
+
+// parameter of element (tile, r, lane)
+__device__ __forceinline__ int wgrad_param(int tile, int r, int lane)
+{
+    const int row = 4 * (lane >> 4) + r, col = lane & 15;
+    if (tile < WG_T1) return MLP_OFF_W1 + ((tile >> 1) * 16 + row) * MLP_KIN + (tile & 1) * 16 + col;
+    if (tile < WG_T1 + WG_T2)
+        return MLP_OFF_W2 + (((tile - WG_T1) >> 3) * 16 + row) * MLP_H + ((tile - WG_T1) & 7) * 16 + col;
+    return MLP_OFF_W3 + row * MLP_H + (tile - WG_T1 - WG_T2) * 16 + col;
+}
+
+__global__ void __launch_bounds__(256, 1)
 mlp_wgrad_partial(const float* __restrict__ X, const float* __restrict__ Z1, const float* __restrict__ Z2,
                   const float* __restrict__ DY, const float* __restrict__ DZ1, const float* __restrict__ DZ2,
                   int64_t n, int64_t chunk, float* __restrict__ part)
 {
-    __shared__ float sx[WG_SUB][MLP_KIN + 4];
-    __shared__ float sh1[WG_SUB][WG_LD];
-    __shared__ float sh2[WG_SUB][WG_LD];
-    __shared__ float sdz1[WG_SUB][WG_LD];
-    __shared__ float sdz2[WG_SUB][WG_LD];
-    __shared__ float sdy[WG_SUB][MLP_KOUT + 4];
+    __shared__ float sh[4][WG_GROUP][4][64];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int col = lane & 15, g = lane >> 4;
-    f32x4 acc[WG_TPW];
+    f32x4 acc[WG_TILES];
 #pragma unroll
-    for (int q = 0; q < WG_TPW; ++q) acc[q] = f32x4{0.f, 0.f, 0.f, 0.f};
-    float bsum = 0.f;   // b1 (threads 0..127) and b2 (threads 128..255) gradient sums
-    float b3sum = 0.f;  // b3 (threads 0..15)
+    for (int q = 0; q < WG_TILES; ++q) acc[q] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float b1[8], b2[8], b3 = 0.f;
+#pragma unroll
+    for (int t = 0; t < 8; ++t) b1[t] = b2[t] = 0.f;
     const int64_t a = (int64_t)blockIdx.x * chunk;
     const int64_t b = a + chunk < n ? a + chunk : n;
-    for (int64_t s0 = a; s0 < b; s0 += WG_SUB) {
-        const int cnt = (int)((b - s0) < WG_SUB ? (b - s0) : WG_SUB);
-        __syncthreads();
-        for (int i = threadIdx.x; i < WG_SUB * MLP_H; i += blockDim.x) {
-            const int t = i / MLP_H, f = i % MLP_H;
-            const bool ok = t < cnt;
-            const int64_t nd = s0 + t;
-            sh1[t][f] = ok ? relu_bf(Z1[nd * MLP_H + f]) : 0.f;
-            sh2[t][f] = ok ? relu_bf(Z2[nd * MLP_H + f]) : 0.f;
-            sdz1[t][f] = ok ? DZ1[nd * MLP_H + f] : 0.f;
-            sdz2[t][f] = ok ? DZ2[nd * MLP_H + f] : 0.f;
-        }
-        for (int i = threadIdx.x; i < WG_SUB * MLP_KIN; i += blockDim.x) {
-            const int t = i / MLP_KIN, f = i % MLP_KIN;
-            sx[t][f] = t < cnt ? bf2f(f2bf(X[(s0 + t) * MLP_KIN + f])) : 0.f;
-        }
-        for (int i = threadIdx.x; i < WG_SUB * MLP_KOUT; i += blockDim.x) {
-            const int t = i / MLP_KOUT, f = i % MLP_KOUT;
-            sdy[t][f] = (t < cnt && f < MLP_OUT) ? DY[(s0 + t) * MLP_OUT + f] : 0.f;
-        }
-        __syncthreads();
-        if (threadIdx.x < MLP_H) {
-            for (int t = 0; t < WG_SUB; ++t) bsum += sdz1[t][threadIdx.x];
-        } else if (threadIdx.x < 2 * MLP_H) {
-            for (int t = 0; t < WG_SUB; ++t) bsum += sdz2[t][threadIdx.x - MLP_H];
-        }
-        if (threadIdx.x < MLP_KOUT) {
-            for (int t = 0; t < WG_SUB; ++t) b3sum += sdy[t][threadIdx.x];
-        }
+    WgradNode N;
+    if (a < b) wgrad_load(N, X, Z1, Z2, DY, DZ1, DZ2, a + 4 * wave + g, b, n, col);
+#pragma unroll 1
+    for (int64_t s0 = a; s0 < b; s0 += 16) {
+        WgradNode C = N;
+        if (s0 + 16 < b) wgrad_load(N, X, Z1, Z2, DY, DZ1, DZ2, s0 + 16 + 4 * wave + g, b, n, col);
+        const float x0 = bf2f(f2bf(C.x[0])), x1 = bf2f(f2bf(C.x[1]));
 #pragma unroll
-        for (int q = 0; q < WG_TPW; ++q) {
-            const int tile = wave * WG_TPW + q;
+        for (int t = 0; t < 8; ++t) {
+            b1[t] += C.dz1[t];
+            b2[t] += C.dz2[t];
+            C.z1[t] = relu_bf(C.z1[t]);
+            C.z2[t] = relu_bf(C.z2[t]);
+        }
+        b3 += C.dy;
 #pragma unroll
-            for (int ks = 0; ks < WG_SUB / 4; ++ks) {
-                const int nd = ks * 4 + g;
-                float av, bv;
-                if (tile < 16) {  // W1: rows o (128), columns = inputs (32)
-                    av = sdz1[nd][(tile >> 1) * 16 + col];
-                    bv = sx[nd][(tile & 1) * 16 + col];
-                } else if (tile < 80) {  // W2
-                    av = sdz2[nd][((tile - 16) >> 3) * 16 + col];
-                    bv = sh1[nd][((tile - 16) & 7) * 16 + col];
-                } else {  // W3 (rows = outputs, padded to 16)
-                    av = sdy[nd][col];
-                    bv = sh2[nd][(tile - 80) * 16 + col];
-                }
-                acc[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, bv, acc[q], 0, 0, 0);
-            }
+        for (int t = 0; t < 8; ++t) {
+            acc[2 * t] = __builtin_amdgcn_mfma_f32_16x16x4f32(C.dz1[t], x0, acc[2 * t], 0, 0, 0);
+            acc[2 * t + 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(C.dz1[t], x1, acc[2 * t + 1], 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                acc[WG_T1 + 8 * t + i] = __builtin_amdgcn_mfma_f32_16x16x4f32(C.dz2[t], C.z1[i], acc[WG_T1 + 8 * t + i], 0, 0, 0);
+            acc[WG_T1 + WG_T2 + t] = __builtin_amdgcn_mfma_f32_16x16x4f32(C.dy, C.z2[t], acc[WG_T1 + WG_T2 + t], 0, 0, 0);
         }
     }
     float* out = part + (int64_t)blockIdx.x * MLP_NPARAM;
+    // tiles of the four waves, WG_GROUP at a time
 #pragma unroll
-    for (int q = 0; q < WG_TPW; ++q) {
-        const int tile = wave * WG_TPW + q;
+    for (int q0 = 0; q0 < WG_TILES; q0 += WG_GROUP) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            int64_t p;
-            if (tile < 16)
-                p = MLP_OFF_W1 + (int64_t)((tile >> 1) * 16 + 4 * g + r) * MLP_KIN + (tile & 1) * 16 + col;
-            else if (tile < 80)
-                p = MLP_OFF_W2 + (int64_t)(((tile - 16) >> 3) * 16 + 4 * g + r) * MLP_H + ((tile - 16) & 7) * 16 + col;
-            else
-                p = MLP_OFF_W3 + (int64_t)(4 * g + r) * MLP_H + (tile - 80) * 16 + col;
-            out[p] = acc[q][r];
+        for (int q = 0; q < WG_GROUP; ++q)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) sh[wave][q][r][lane] = acc[q0 + q][r];
+        __syncthreads();
+        for (int i = threadIdx.x; i < WG_GROUP * 256; i += 256) {
+            const int q = i >> 8, r = (i >> 6) & 3, l = i & 63;
+            out[wgrad_param(q0 + q, r, l)] = ((sh[0][q][r][l] + sh[1][q][r][l]) + sh[2][q][r][l]) + sh[3][q][r][l];
         }
+        __syncthreads();
     }
-    if (threadIdx.x < MLP_H) out[MLP_OFF_B1 + threadIdx.x] = bsum;
-    else if (threadIdx.x < 2 * MLP_H) out[MLP_OFF_B2 + threadIdx.x - MLP_H] = bsum;
-    if (threadIdx.x < MLP_KOUT) out[MLP_OFF_B3 + threadIdx.x] = b3sum;
+    // biases: over the four nodes of a wave, then over the waves
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+        b1[t] += __shfl_xor(b1[t], 16, 64);
+        b1[t] += __shfl_xor(b1[t], 32, 64);
+        b2[t] += __shfl_xor(b2[t], 16, 64);
+        b2[t] += __shfl_xor(b2[t], 32, 64);
+    }
+    b3 += __shfl_xor(b3, 16, 64);
+    b3 += __shfl_xor(b3, 32, 64);
+    float* sb = &sh[0][0][0][0] + wave * (2 * MLP_H + MLP_KOUT);
+    if (g == 0) {
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            sb[16 * t + col] = b1[t];
+            sb[MLP_H + 16 * t + col] = b2[t];
+        }
+        sb[2 * MLP_H + col] = b3;
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < 2 * MLP_H + MLP_KOUT; i += 256) {
+        const float* q = &sh[0][0][0][0] + i;
+        constexpr int S = 2 * MLP_H + MLP_KOUT;
+        const float v = ((q[0] + q[S]) + q[2 * S]) + q[3 * S];
+        out[i < MLP_H ? MLP_OFF_B1 + i : (i < 2 * MLP_H ? MLP_OFF_B2 + i - MLP_H : MLP_OFF_B3 + i - 2 * MLP_H)] = v;
+    }
 }
 
-__global__ void mlp_reduce(const float* __restrict__ part, int nblk, float* __restrict__ grad)
+// grad = sum of the block partials: 64 parameters a workgroup, a quarter of
+// the blocks per wave, the quarters added in order (61 -> 5.6 us for 256
+// blocks: one thread walked all blocks of its parameter)
+__global__ void __launch_bounds__(256)
+mlp_reduce(const float* __restrict__ part, int nblk, float* __restrict__ grad)
 {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= MLP_NPARAM) return;
+    __shared__ float sh[4][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int p = blockIdx.x * 64 + lane;
+    const int per = (nblk + 3) / 4, b0 = wave * per, b1 = b0 + per < nblk ? b0 + per : nblk;
     float s = 0.f;
-    for (int b = 0; b < nblk; ++b) s += part[(int64_t)b * MLP_NPARAM + p];
-    grad[p] = s;
+    if (p < MLP_NPARAM) {
+#pragma unroll 16
+        for (int b = b0; b < b1; ++b) s += part[(int64_t)b * MLP_NPARAM + p];
+    }
+    sh[wave][lane] = s;
+    __syncthreads();
+    if (wave == 0 && p < MLP_NPARAM) grad[p] = ((sh[0][lane] + sh[1][lane]) + sh[2][lane]) + sh[3][lane];
 }
 
 // MSE loss gradient on the 4 outputs: dy = 2 (y - t) / (4 n); loss partials
@@ -423,56 +468,52 @@ predict_scale_final(const double* __restrict__ part, int nparts, int64_t nv, dou
 
 // x[v] = clamp(( u, d1 / sigma, d2 / sigma, d3 / sigma,
 //                1-ring mean of u - u, (1-ring mean of d1 - d1) / sigma ) * scale),
-// 24 values padded to 32.  The 1-ring is the node's column blocks in the
-// CSR pattern (rows of component 0), the node itself excluded.
-__global__ void predict_features(const int64_t* __restrict__ rowptr, const int32_t* __restrict__ colidx,
-                                 const double* __restrict__ u, const double* __restrict__ u1,
-                                 const double* __restrict__ u2, const double* __restrict__ u3, int64_t nv,
-                                 const float* __restrict__ scale, const double* __restrict__ sigma,
-                                 float* __restrict__ X)
+// 24 values padded to 32.  The 1-ring is the node's neighbours in the pattern,
+// the node itself excluded.
+// Four lanes per node, one per component: a neighbour's state is 32
+// contiguous bytes, and neighbours come from the node-block list (one index
+// each) in ascending order, four in flight.  Latency and L2 bound:
+// 233000 nodes of a quad mesh 78 -> 38 us against one lane per node that walked
+// the columns of its first CSR row.
+__global__ void __launch_bounds__(256)
+predict_features(const int64_t* __restrict__ rowptr, const int32_t* __restrict__ adj, const double* __restrict__ u,
+                 const double* __restrict__ u1, const double* __restrict__ u2, const double* __restrict__ u3,
+                 int64_t nv, const float* __restrict__ scale, const double* __restrict__ sigma, float* __restrict__ X)
 {
-    const int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t v = t >> 2;
+    const int c = (int)(t & 3);
     if (v >= nv) return;
     const double is = 1.0 / *sigma;
-    double un[4], d1[4], d2[4], d3[4], m0[4] = {0, 0, 0, 0}, m1[4] = {0, 0, 0, 0};
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        const int64_t i = v * 4 + c;
-        un[c] = u[i];
-        const double a = u1[i], b = u2[i], e1 = a - b;
-        d1[c] = un[c] - a;
-        d2[c] = d1[c] - e1;
-        d3[c] = d2[c] - (e1 - (b - u3[i]));
-    }
-    const int64_t r0 = rowptr[v * 4], r1 = rowptr[v * 4 + 1];
+    const int64_t i = v * 4 + c;
+    const double un = u[i], a = u1[i], b = u2[i], e1 = a - b;
+    const double d1 = un - a, d2 = d1 - e1, d3 = d2 - (e1 - (b - u3[i]));
+    const int64_t r0 = rowptr[v * 4];
+    const int nb = (int)((rowptr[v * 4 + 1] - r0) >> 2);
+    const int32_t* ad = adj + (r0 >> 4);
+    double m0 = 0.0, m1 = 0.0;
     int cnt = 0;
-    for (int64_t k = r0; k < r1; k += 4) {
-        const int64_t w = colidx[k] / 4;
-        if (w == v) continue;
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            const double x = u[w * 4 + c];
-            m0[c] += x;
-            m1[c] += x - u1[w * 4 + c];
+#pragma unroll 4
+    for (int k = 0; k < nb; ++k) {
+        const int64_t w = ad[k];
+        const double x = u[w * 4 + c], y = u1[w * 4 + c];
+        if (w != v) {
+            m0 += x;
+            m1 += x - y;
+            ++cnt;
         }
-        ++cnt;
     }
     const double ic = cnt > 0 ? 1.0 / cnt : 0.0;
-    float out[MLP_KIN];
+    float out[MLP_KIN / 4];
+    out[0] = clampf((float)un * scale[c]);
+    out[1] = clampf((float)(d1 * is) * scale[4 + c]);
+    out[2] = clampf((float)(d2 * is) * scale[8 + c]);
+    out[3] = clampf((float)(d3 * is) * scale[12 + c]);
+    out[4] = clampf((float)(cnt > 0 ? m0 * ic - un : 0.0) * scale[16 + c]);
+    out[5] = clampf((float)(cnt > 0 ? (m1 * ic - d1) * is : 0.0) * scale[20 + c]);
+    out[6] = out[7] = 0.f;
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        out[c] = clampf((float)un[c] * scale[c]);
-        out[4 + c] = clampf((float)(d1[c] * is) * scale[4 + c]);
-        out[8 + c] = clampf((float)(d2[c] * is) * scale[8 + c]);
-        out[12 + c] = clampf((float)(d3[c] * is) * scale[12 + c]);
-        out[16 + c] = clampf((float)(cnt > 0 ? m0[c] * ic - un[c] : 0.0) * scale[16 + c]);
-        out[20 + c] = clampf((float)(cnt > 0 ? (m1[c] * ic - d1[c]) * is : 0.0) * scale[20 + c]);
-    }
-#pragma unroll
-    for (int c = MLP_IN; c < MLP_KIN; ++c) out[c] = 0.f;
-#pragma unroll
-    for (int q = 0; q < MLP_KIN; q += 4)
-        *reinterpret_cast<float4*>(X + v * MLP_KIN + q) = make_float4(out[q], out[q + 1], out[q + 2], out[q + 3]);
+    for (int q = 0; q < MLP_KIN / 4; ++q) X[v * MLP_KIN + 4 * q + c] = out[q];
 }
 
 // guess = u + d1 + d2 + y * out_scale * sigma (per component)
@@ -515,9 +556,9 @@ hipError_t launch_mlp_forward(const float* P, const uint16_t* WB, const float* X
                               float* Z2, hipStream_t s)
 {
     if (n <= 0) return hipSuccess;
-    // one workgroup per CU (256 CUs): each holds the weights in registers
-    // (one wave per SIMD) and walks its share of the 64-node blocks
-    const unsigned g = nblocks(n, 64) < 256u ? nblocks(n, 64) : 256u;
+    // two workgroups per CU (256 CUs): each wave holds the weights in
+    // registers (two waves per SIMD) and walks its share of the 16-node blocks
+    const unsigned g = nblocks(n, 64) < 512u ? nblocks(n, 64) : 512u;
     mlp_forward<<<g, 256, 0, s>>>(P, WB, X, n, Y, Z1, Z2);
     return hipGetLastError();
 }
@@ -534,7 +575,7 @@ hipError_t launch_mlp_backward(const uint16_t* WB, const float* X, const float* 
     mlp_backward_act<<<nblocks(n, 64), 256, 0, s>>>(WB, Z1, Z2, DY, n, dz1, dz2);
     const int64_t chunk = (n + MLP_WG_BLOCKS - 1) / MLP_WG_BLOCKS;
     mlp_wgrad_partial<<<MLP_WG_BLOCKS, 256, 0, s>>>(X, Z1, Z2, DY, dz1, dz2, n, chunk, part);
-    mlp_reduce<<<nblocks(MLP_NPARAM, 256), 256, 0, s>>>(part, MLP_WG_BLOCKS, grad);
+    mlp_reduce<<<nblocks(MLP_NPARAM, 64), 256, 0, s>>>(part, MLP_WG_BLOCKS, grad);
     return hipGetLastError();
 }
 
@@ -569,12 +610,12 @@ hipError_t launch_predict_scale(const double* u, const double* u1, const double*
     return hipGetLastError();
 }
 
-hipError_t launch_predict_features(const int64_t* rowptr, const int32_t* colidx, const double* u, const double* u1,
+hipError_t launch_predict_features(const int64_t* rowptr, const int32_t* adj, const double* u, const double* u1,
                                    const double* u2, const double* u3, int64_t nv, const float* scale,
                                    const double* sigma, float* X, hipStream_t s)
 {
     if (nv <= 0) return hipSuccess;
-    predict_features<<<nblocks(nv, 256), 256, 0, s>>>(rowptr, colidx, u, u1, u2, u3, nv, scale, sigma, X);
+    predict_features<<<nblocks(nv * 4, 256), 256, 0, s>>>(rowptr, adj, u, u1, u2, u3, nv, scale, sigma, X);
     return hipGetLastError();
 }
 

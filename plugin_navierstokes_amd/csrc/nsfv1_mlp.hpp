@@ -33,7 +33,8 @@ hipError_t launch_mlp_adam(float* P, float* M, float* V, const float* G, int ste
 hipError_t launch_mlp_pack(const float* P, uint16_t* WB, hipStream_t s);
 hipError_t launch_predict_scale(const double* u, const double* u1, const double* u2, const double* u3, int64_t nv,
                                 double* part, double* sigma, hipStream_t s);
-hipError_t launch_predict_features(const int64_t* rowptr, const int32_t* colidx, const double* u, const double* u1,
+// adj: node-block neighbour lists (node v's start at rowptr[4 v] / 16)
+hipError_t launch_predict_features(const int64_t* rowptr, const int32_t* adj, const double* u, const double* u1,
                                    const double* u2, const double* u3, int64_t nv, const float* scale,
                                    const double* sigma, float* X, hipStream_t s);
 hipError_t launch_predict_guess(const double* u, const double* u1, const double* u2, const float* Y,
