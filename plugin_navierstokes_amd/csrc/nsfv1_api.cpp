@@ -2223,7 +2223,7 @@ int nsfv1_predict_features(nsfv1_handle* h, const double* u, const double* u_pre
     hipStream_t s = (hipStream_t)stream;
     if (launch_predict_scale(u, u_prev, u_prev2, u_prev3, h->nv, h->pred_part.as<double>(), sigma, s) != hipSuccess)
         return fail(NSFV1_ERR_DEVICE, "predict scale");
-    if (launch_predict_features(h->rowptr.as<int64_t>(), h->colidx.as<int32_t>(), u, u_prev, u_prev2, u_prev3, h->nv,
+    if (launch_predict_features(h->rowptr.as<int64_t>(), h->adj.as<int32_t>(), u, u_prev, u_prev2, u_prev3, h->nv,
                                 scale, sigma, x, s) != hipSuccess)
         return fail(NSFV1_ERR_DEVICE, "predict features");
     return NSFV1_OK;
