@@ -174,8 +174,13 @@ struct nsfv1_handle {
     DevBuf mg_r0, mg_t0, mg_dense, mg_gj;  // mg_gj: Gauss-Jordan tableaux of the coarsest level
     bool geo_valid = false;
     int geo_difflen = -1;
-    // split assembly path (per-SCVF records)
+    // split assembly path (per-SCVF or, for simplices, per-element records)
     DevBuf recs;
+    // block lists of the simplex path (triangle and tetrahedron meshes)
+    DevBuf sx_blk, sx_node, sx_items, sx_wg;
+    int sx_nwg = 0;
+    bool sx_valid = false;
+    int64_t nblk() const { return nnz / ((dim + 1) * (dim + 1)); }
     // 0: split where supported, 1: fused kernel only, 2: split with row lanes,
     // 3: plane march on structured grids of parallelepipeds, otherwise 0
     int path = 3;
@@ -880,6 +885,7 @@ static int set_mesh_groups(nsfv1_handle* h, const double* xyz, int64_t nv, const
     h->ninst = 0;
     h->recs.release();
     h->cpl_recs.release();
+    h->sx_valid = false;
     return NSFV1_OK;
 }
 
@@ -1062,6 +1068,40 @@ static int make_plan(nsfv1_handle* h, const IncView& g, int jbytes, Plan& P)
     return NSFV1_OK;
 }
 
+// workgroups (nodes with at most 256 incidences together, at most 255 nodes)
+// and block lists of the simplex path, the lists built on the device
+static int ensure_simplex_lists(nsfv1_handle* h)
+{
+    if (h->sx_valid || h->mixed()) return NSFV1_OK;
+    int64_t most = 0;
+    std::vector<int32_t> wn{0};
+    for (int64_t v = 0, v0 = 0; v < h->nv; ++v) {
+        most = std::max(most, h->h_node_inc[v + 1] - h->h_node_inc[v]);
+        if (h->h_node_inc[v + 1] - h->h_node_inc[v0] > 256 || v - v0 >= 255) {
+            wn.push_back((int32_t)v);
+            v0 = v;
+        }
+    }
+    wn.push_back((int32_t)h->nv);
+    if (!simplex_supported(h->et, most)) return NSFV1_OK;
+    if (h->sx_blk.alloc(sizeof(uint32_t) * h->nblk()) != hipSuccess ||
+        h->sx_node.alloc(sizeof(int32_t) * h->nblk()) != hipSuccess ||
+        h->sx_items.alloc(sizeof(uint16_t) * h->ninc * nsh_count(h->et)) != hipSuccess ||
+        h->sx_wg.alloc(sizeof(int32_t) * wn.size()) != hipSuccess ||
+        hipMemcpy(h->sx_wg.p, wn.data(), sizeof(int32_t) * wn.size(), hipMemcpyHostToDevice) != hipSuccess)
+        return fail(NSFV1_ERR_DEVICE, "block lists");
+    KMeshPtrs m{};
+    m.rowptr = h->rowptr.as<int64_t>();
+    m.node_inc = h->node_inc.as<int32_t>();
+    m.inc_pos = h->inc_pos.as<uint64_t>();
+    const SxLists l{h->sx_blk.as<uint32_t>(), h->sx_node.as<int32_t>(), h->sx_items.as<uint16_t>(), h->sx_wg.as<int32_t>()};
+    if (launch_simplex_lists(h->et, l, m, h->nv, nullptr) != hipSuccess || hipStreamSynchronize(nullptr) != hipSuccess)
+        return fail(NSFV1_ERR_DEVICE, "block lists");
+    h->sx_nwg = (int)wn.size() - 1;
+    h->sx_valid = true;
+    return NSFV1_OK;
+}
+
 // configurations whose SCVFs are coupled within an element: the FLOW
 // stabilisation (connected velocity components) and upwinds with ip shapes
 static bool coupled_config(const nsfv1_handle* h)
@@ -1157,6 +1197,7 @@ static int assemble_impl(nsfv1_handle* h, const double* u, const double* u_old, 
                                             "needs one nsfv1_assemble call with the same jprec first (it builds the plan)");
         int rc = make_plan(h, IncView{h->h_node_inc, h->h_inc_info, h->h_inc_elem, h->ninc, h->inc_pos},
                            jprec == NSFV1_F64 ? 8 : 4, P);
+        if (!rc && jprec == NSFV1_F32) rc = ensure_simplex_lists(h);
         if (rc) return rc;
     }
     for (auto& gp : h->groups) {
@@ -1338,6 +1379,10 @@ static int assemble_impl(nsfv1_handle* h, const double* u, const double* u_old, 
         // also without a Jacobian (defect only): the gather then reads only
         // the records' fluxes, and the defect is bitwise the one assembled
         // together with the Jacobian
+        // triangles and tetrahedra: element records and block lists (16-byte
+        // stores need an aligned J in 3D); the row-lane gather on request
+        const bool simplex = h->sx_valid && !(h->path == 2 && P.rowlane) &&
+                             (h->dim == 2 || ((uintptr_t)jvals & 15) == 0);
         const size_t need = sizeof(float) * (size_t)split_record_floats(h->et, h->ne);
         float* recs = static_cast<float*>(scratch);
         if (scratch) {
@@ -1346,11 +1391,18 @@ static int assemble_impl(nsfv1_handle* h, const double* u, const double* u_old, 
                                                     " bytes of SCVF records for this mesh; the no-allocation entry holds at most " +
                                                     std::to_string(NOALLOC_SCRATCH_BYTES));
         } else {
-            if (h->recs.n < need && h->recs.alloc(need) != hipSuccess) return fail(NSFV1_ERR_DEVICE, "record buffer");
+            const size_t take = simplex ? (size_t)simplex_record_bytes(h->et, h->ne) : need;
+            if (h->recs.n < take && h->recs.alloc(take) != hipSuccess) return fail(NSFV1_ERR_DEVICE, "record buffer");
             recs = h->recs.as<float>();
         }
-        e = launch_assemble_split(h->et, m, k, u, u_old, static_cast<float*>(jvals), defect, h->errflag.as<int>(), P.nwg,
-                                  P.lds, h->ne, recs, h->path == 2 && P.rowlane, (hipStream_t)stream);
+        if (simplex) {
+            const SxLists l{h->sx_blk.as<uint32_t>(), h->sx_node.as<int32_t>(), h->sx_items.as<uint16_t>(),
+                            h->sx_wg.as<int32_t>()};
+            e = launch_assemble_simplex(h->et, l, m, k, u, u_old, static_cast<float*>(jvals), defect, h->errflag.as<int>(),
+                                        h->ne, h->sx_nwg, recs, (hipStream_t)stream);
+        } else
+            e = launch_assemble_split(h->et, m, k, u, u_old, static_cast<float*>(jvals), defect, h->errflag.as<int>(), P.nwg,
+                                      P.lds, h->ne, recs, h->path == 2 && P.rowlane, (hipStream_t)stream);
         h->last_path = (h->path == 2 && P.rowlane) ? 2 : 0;
     } else {
         e = launch_assemble(h->et, jprec, m, k, u, u_old, jvals, defect, h->errflag.as<int>(), P.nwg, P.lds,

@@ -1,0 +1,97 @@
+"""Triangle and tetrahedron meshes with FP32 Jacobian (element records and block
+lists): parity with the oracle at the edges of the record groups (eight
+elements) and workgroups, isolated nodes, one element, and the routes that
+fall back (an unaligned Jacobian, the fused path)."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import oracle as O
+from plugin_navierstokes_amd import F32, PART_A, PART_M, PART_RHS, UPWIND_FRESH, UPWIND_RECORD, UPWIND_REPLAY
+from plugin_navierstokes_amd import NavierStokesFV1
+from plugin_navierstokes_amd import meshes as M
+from tests._parity import configure_disc, fp32_violation, fp64_violation, run_case, worst, FP32_ABS, FP32_REL
+
+pytestmark = pytest.mark.gpu
+
+
+def _cut(mesh, ne):
+    """The first ne elements of a mesh; the nodes they leave stay, isolated."""
+    return M.Mesh(mesh.et, mesh.xyz, mesh.conn[:ne], {}, ())
+
+
+# element counts around groups of eight and workgroups of 256 elements
+MESHES = [(M.TRI, lambda ne: _cut(M.cavity_2d(14, M.TRI, 0.1, 3), ne), ne) for ne in (1, 7, 8, 9, 255, 257, 392)]
+MESHES += [(M.TET, lambda ne: _cut(M.cavity_3d(4, M.TET, 0.1, 3), ne), ne) for ne in (1, 7, 8, 9, 257, 384)]
+
+
+@pytest.mark.parametrize("up", ["no", "full", "skewed", "lps"])
+@pytest.mark.parametrize("et,make,ne", MESHES, ids=lambda x: str(x) if isinstance(x, int) else "m")
+def test_parity(cuda, et, make, ne, up):
+    cfg = {"upwind": up, "rho": 1.3, "source": (0.3, -0.2, 0.1)[:M.DIM[et]]}
+    J, d, Jr, dr, Ja, da, disc = run_case(cuda, et, cfg, mesh=make(ne), time_dep=True, parts=PART_A | PART_M | PART_RHS,
+                                          s=(0.7, 1.3, -0.7), jprec=32)
+    assert disc.assembly_path_used() == 0
+    assert fp64_violation(d, dr, da) <= 1.0, worst(d, dr, da)
+    assert fp32_violation(J, Jr, Ja) <= 1.0, worst(J, Jr, Ja, FP32_REL, FP32_ABS)
+
+
+@pytest.mark.parametrize("up", ["full", "lps"])
+def test_axis_aligned_zeros_and_laplace(cuda, up):
+    """Uniform Kuhn tetrahedra: entries without a contribution are exact zeros."""
+    J, d, Jr, dr, Ja, da, _ = run_case(cuda, M.TET, {"upwind": up, "laplace": True}, mesh=M.cavity_3d(3, M.TET), jprec=32)
+    assert fp64_violation(d, dr, da) <= 1.0, worst(d, dr, da)
+    assert fp32_violation(J, Jr, Ja) <= 1.0, worst(J, Jr, Ja, FP32_REL, FP32_ABS)
+
+
+@pytest.mark.parametrize("et", [M.TRI, M.TET])
+def test_routes_agree(cuda, et):
+    """Defect only, an unaligned Jacobian, a second run and the fused path."""
+    import torch
+
+    mesh = M.cavity_2d(9, et, 0.1, 2) if et == M.TRI else M.channel_3d((12, 6, 6), n_boxes=2, seed=5)
+    disc = NavierStokesFV1("u,v,p" if mesh.dim == 2 else "u,v,w,p", "Inner")
+    configure_disc(disc, {"upwind": "lps", "nu": 0.02})
+    disc.set_mesh(mesh)
+    u = torch.from_numpy(M.random_state(mesh, 4)).to(cuda)
+    uo = torch.from_numpy(M.random_state(mesh, 5)).to(cuda)
+    kw = dict(u_old=uo, dt=0.01, s_m=1.5, parts=PART_A | PART_M, jprec=F32)
+    J, d = disc.assemble(u, **kw)
+    J2, d2 = disc.assemble(u, **kw)
+    assert torch.equal(J, J2) and torch.equal(d, d2)
+    _, d3 = disc.assemble(u, want_J=False, **kw)
+    assert torch.equal(d, d3)
+    J4, _ = disc.assemble(u, want_d=False, **kw)
+    assert torch.equal(J, J4)
+    buf = torch.full((disc.nnz() + 1,), float("nan"), dtype=torch.float32, device=cuda)
+    J5, d5 = disc.assemble(u, J=buf[1:], **kw)
+    disc.set_assembly_path(1)
+    J6, d6 = disc.assemble(u, **kw)
+    assert disc.assembly_path_used() == 1
+    p = O.Params(dim=mesh.dim, upwind="lps", nu=0.02)
+    rp, ci = disc.pattern()
+    ua, ub = u.cpu().numpy(), uo.cpu().numpy()
+    Ja, da = O.assemble_abs(p, et, mesh.xyz, mesh.conn, ua, ub, 0.01, s_m=1.5, parts=3, rowptr=rp, colidx=ci)
+    # the routes round the same terms in different orders
+    for Jx, dx in ((J5, d5), (J6, d6)):
+        assert fp32_violation(Jx.cpu().numpy(), J.cpu().numpy(), 2 * Ja) <= 1.0
+        assert fp64_violation(dx.cpu().numpy(), d.cpu().numpy(), 2 * da) <= 1.0
+
+
+@pytest.mark.parametrize("et", [M.TRI, M.TET])
+def test_replayed_decisions(cuda, et):
+    import torch
+
+    mesh = M.cavity_2d(7, et, 0.1, 2) if et == M.TRI else M.cavity_3d(3, et, 0.1, 2)
+    disc = NavierStokesFV1("u,v,p" if mesh.dim == 2 else "u,v,w,p", "Inner")
+    configure_disc(disc, {"upwind": "skewed", "nu": 0.02})
+    disc.set_mesh(mesh)
+    u = torch.from_numpy(M.random_state(mesh, 4)).to(cuda)
+    J0, d0 = disc.assemble(u, jprec=F32)
+    disc.set_upwind_decisions(UPWIND_RECORD)
+    disc.assemble(u, jprec=F32)
+    disc.set_upwind_decisions(UPWIND_REPLAY)
+    J1, d1 = disc.assemble(u, jprec=F32)
+    assert torch.equal(J0, J1) and torch.equal(d0, d1)
+    disc.set_upwind_decisions(UPWIND_FRESH)
