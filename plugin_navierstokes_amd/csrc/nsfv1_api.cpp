@@ -156,6 +156,7 @@ struct nsfv1_handle {
     double slide_k = 0.0, slide_lim = 0.0;
     std::vector<int64_t> h_rowptr, h_node_inc;
     int max_threads = 256;
+    bool threads_set = false;  // by nsfv1_set_launch
     size_t lds_cap = 64 * 1024;
     Plan plan32, plan64;
     // Newton-loop linear algebra
@@ -945,6 +946,7 @@ int nsfv1_set_launch(nsfv1_handle* h, int threads, int lds_bytes)
     if (threads) {
         if (threads < 64 || threads > 256 || threads % 64) return fail(NSFV1_ERR_ARGUMENT, "threads must be 64..256, a multiple of 64");
         h->max_threads = threads;
+        h->threads_set = true;
     }
     if (lds_bytes && h->path == 3) {
         // the plane march reads the budget in KiB as node planes per work unit
@@ -960,17 +962,19 @@ int nsfv1_set_launch(nsfv1_handle* h, int threads, int lds_bytes)
 
 // Workgroup plan: consecutive nodes while their incidences fit the thread
 // budget and their rows (plus defect) fit the LDS budget (<= 64 KiB).
-static int make_plan(nsfv1_handle* h, const IncView& g, int jbytes, Plan& P)
+static int make_plan(nsfv1_handle* h, const IncView& g, int jbytes, Plan& P, int threads = 0)
 {
     const int nc = h->dim + 1;
     std::vector<int32_t> wn, wr;
     wn.push_back(0);
     int64_t v = 0;
     size_t maxlds = 0;
+    const bool chosen = threads != 0 || h->threads_set;
+    if (!threads) threads = h->max_threads;
     // the row-lane split gather puts dim+1 lanes on each incidence of a
     // 64-lane workgroup
-    const bool rowlane = h->path == 2 && jbytes == 4 && h->max_threads == 64;
-    const int64_t inc_budget = rowlane ? 64 / nc : h->max_threads;
+    const bool rowlane = h->path == 2 && jbytes == 4 && threads == 64;
+    const int64_t inc_budget = rowlane ? 64 / nc : threads;
     // element groups of a mixed mesh: a run of nodes without incidences of
     // the group is one empty range (its workgroup returns at once), so the
     // other ranges hold only the group's nodes
@@ -1000,9 +1004,17 @@ static int make_plan(nsfv1_handle* h, const IncView& g, int jbytes, Plan& P)
         wn.push_back((int32_t)v);
         wr.push_back(rounds);
     }
+    // Rows of 8-byte values of a hexahedral mesh fill the LDS budget with 18
+    // nodes, 144 of 256 lanes: once that makes more workgroups than the 256
+    // CUs hold (one each, by registers), half the lanes, all of them active,
+    // are faster (FP64 hexahedra, LPS: 20^3 98 -> 60 us, 36^3 517 -> 322 us,
+    // 50^3 1342 -> 874 us; 16^3, one workgroup a CU, 51 against 56 us)
+    if (!chosen && !skip_empty && threads == 256 && wr.size() > 256 && (size_t)g.ninc < wr.size() * 192 &&
+        *std::max_element(wr.begin(), wr.end()) <= 128)
+        return make_plan(h, g, jbytes, P, 128);
     P.nwg = (int)wr.size();
     P.lds = maxlds;
-    P.block = h->max_threads;
+    P.block = threads;
     P.rowlane = rowlane;
     // lane order inside each workgroup: by incidence slot, then node, so a
     // wavefront takes part in as few accumulation rounds as possible
@@ -2587,6 +2599,7 @@ int nsfv1_autotune(nsfv1_handle* h, const double* u, const double* u_old, double
     if (h->march_ok)
         for (int l : {8192, 16384, 32768}) cand.push_back({3, 256, l});
     const int keep_path = h->path, keep_threads = h->max_threads;
+    const bool keep_set = h->threads_set;
     const size_t keep_lds = h->lds_cap;
     const int keep_zc = h->march_zc;
     hipEvent_t e0, e1;
@@ -2624,6 +2637,7 @@ int nsfv1_autotune(nsfv1_handle* h, const double* u, const double* u_old, double
     if (bc.path < 0) {
         h->path = keep_path;
         h->max_threads = keep_threads;
+        h->threads_set = keep_set;
         h->lds_cap = keep_lds;
         h->march_zc = keep_zc;
         invalidate_plans(h);
