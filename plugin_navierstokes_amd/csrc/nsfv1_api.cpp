@@ -59,8 +59,10 @@ struct DevBuf {
     hipError_t alloc(size_t bytes)
     {
         release();
-        n = bytes;
-        return hipMalloc(&p, bytes ? bytes : 16);
+        const hipError_t e = hipMalloc(&p, bytes ? bytes : 16);
+        if (e == hipSuccess) n = bytes;
+        else p = nullptr;
+        return e;
     }
     template <typename T> T* as() const { return static_cast<T*>(p); }
 };
@@ -177,6 +179,15 @@ struct nsfv1_handle {
     int geo_difflen = -1;
     // split assembly path (per-SCVF or, for simplices, per-element records)
     DevBuf recs;
+    // FP64 element records, one buffer per stream that assembles (at most 4, the
+    // others take the fused kernel): FP64 assemblies of one handle on several
+    // streams share nothing but the error flag
+    struct StreamBuf {
+        void* stream = nullptr;
+        DevBuf buf;
+    };
+    StreamBuf recs64[4];
+    int nrecs64 = 0;
     // block lists of the simplex path (triangle and tetrahedron meshes)
     DevBuf sx_blk, sx_node, sx_items, sx_wg;
     int sx_nwg = 0;
@@ -885,6 +896,8 @@ static int set_mesh_groups(nsfv1_handle* h, const double* xyz, int64_t nv, const
     }
     h->ninst = 0;
     h->recs.release();
+    for (auto& r : h->recs64) r.buf.release();
+    h->nrecs64 = 0;
     h->cpl_recs.release();
     h->sx_valid = false;
     return NSFV1_OK;
@@ -1082,7 +1095,7 @@ static int make_plan(nsfv1_handle* h, const IncView& g, int jbytes, Plan& P, int
 
 // workgroups (nodes with at most 256 incidences together, at most 255 nodes)
 // and block lists of the simplex path, the lists built on the device
-static int ensure_simplex_lists(nsfv1_handle* h)
+static int ensure_simplex_lists(nsfv1_handle* h, int jprec)
 {
     if (h->sx_valid || h->mixed()) return NSFV1_OK;
     int64_t most = 0;
@@ -1095,7 +1108,7 @@ static int ensure_simplex_lists(nsfv1_handle* h)
         }
     }
     wn.push_back((int32_t)h->nv);
-    if (!simplex_supported(h->et, most)) return NSFV1_OK;
+    if (!simplex_supported(h->et, jprec, most)) return NSFV1_OK;
     if (h->sx_blk.alloc(sizeof(uint32_t) * h->nblk()) != hipSuccess ||
         h->sx_node.alloc(sizeof(int32_t) * h->nblk()) != hipSuccess ||
         h->sx_items.alloc(sizeof(uint16_t) * h->ninc * nsh_count(h->et)) != hipSuccess ||
@@ -1112,6 +1125,23 @@ static int ensure_simplex_lists(nsfv1_handle* h)
     h->sx_nwg = (int)wn.size() - 1;
     h->sx_valid = true;
     return NSFV1_OK;
+}
+
+// FP64 element records of the stream (null: none to be had)
+static void* stream_records(nsfv1_handle* h, void* stream, size_t need)
+{
+    int i = 0;
+    while (i < h->nrecs64 && h->recs64[i].stream != stream) ++i;
+    if (i < h->nrecs64 && h->recs64[i].buf.n >= need) return h->recs64[i].buf.p;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (i == 4 || hipStreamIsCapturing((hipStream_t)stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone ||
+        h->recs64[i].buf.alloc(need) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    h->recs64[i].stream = stream;
+    h->nrecs64 = std::max(h->nrecs64, i + 1);
+    return h->recs64[i].buf.p;
 }
 
 // configurations whose SCVFs are coupled within an element: the FLOW
@@ -1209,7 +1239,7 @@ static int assemble_impl(nsfv1_handle* h, const double* u, const double* u_old, 
                                             "needs one nsfv1_assemble call with the same jprec first (it builds the plan)");
         int rc = make_plan(h, IncView{h->h_node_inc, h->h_inc_info, h->h_inc_elem, h->ninc, h->inc_pos},
                            jprec == NSFV1_F64 ? 8 : 4, P);
-        if (!rc && jprec == NSFV1_F32) rc = ensure_simplex_lists(h);
+        if (!rc) rc = ensure_simplex_lists(h, jprec);
         if (rc) return rc;
     }
     for (auto& gp : h->groups) {
@@ -1277,6 +1307,36 @@ static int assemble_impl(nsfv1_handle* h, const double* u, const double* u_old, 
         k.conv_upwind == k.stab_upwind && (k.conv_upwind == UPW_NO || k.conv_upwind == UPW_FULL || k.conv_upwind == UPW_SKEWED) &&
         ((uintptr_t)jvals & 15) == 0 && ((uintptr_t)defect & 15) == 0)
         mfast = k.conv_upwind;
+    // split path (FP32 SCVF records) and simplex path (element records)
+    const bool split = !h->mixed() && mfast < 0 && !coupled_config(h) &&
+                       (h->path == 0 || h->path == 2 || h->path == 3) && (parts & NSFV1_PART_A) && !h->ip_imports() &&
+                       split_supported(h->et, k);
+    if (split && jprec == NSFV1_F32 && scratch) {
+        const size_t need = sizeof(float) * (size_t)split_record_floats(h->et, h->ne);
+        if (need > NOALLOC_SCRATCH_BYTES)
+            return fail(NSFV1_ERR_ARGUMENT, "the split path needs " + std::to_string(need) +
+                                                " bytes of SCVF records for this mesh; the no-allocation entry holds at most " +
+                                                std::to_string(NOALLOC_SCRATCH_BYTES));
+    }
+    bool simplex = split && h->sx_valid && (jprec == NSFV1_F32 || h->et == ET_TET) &&
+                   !(h->path == 2 && P.rowlane);
+    void* sx_recs = scratch;
+    if (simplex) {
+        const size_t need = (size_t)simplex_record_bytes(h->et, jprec, h->ne);
+        if (jprec == NSFV1_F32 && !scratch) {
+            if (h->recs.n < need && h->recs.alloc(need) != hipSuccess) return fail(NSFV1_ERR_DEVICE, "record buffer");
+            sx_recs = h->recs.p;
+        } else if (jprec == NSFV1_F64) {
+            // the fused kernel needs no records: it takes meshes whose records
+            // exceed the no-allocation entry's scratch (both entries give the
+            // same bits) and calls that cannot allocate them now
+            simplex = need <= NOALLOC_SCRATCH_BYTES;
+            if (simplex && !scratch) {
+                sx_recs = stream_records(h, stream, need);
+                simplex = sx_recs != nullptr;
+            }
+        }
+    }
     if (h->mixed()) {
         // a mixed mesh: every element group on the fused kernel (or the
         // coupled path), in group order on the one stream; the first group
@@ -1386,35 +1446,26 @@ static int assemble_impl(nsfv1_handle* h, const double* u, const double* u_old, 
         e = launch_assemble_coupled(h->et, jprec, m, k, u, u_old, jvals, defect, h->errflag.as<int>(), P.nwg, P.lds,
                                     h->ne, recs, nullptr, (hipStream_t)stream);
         h->last_path = 4;
-    } else if ((h->path == 0 || h->path == 2 || h->path == 3) && jprec == NSFV1_F32 && (parts & NSFV1_PART_A) &&
-               !h->ip_imports() && split_supported(h->et, k)) {
+    } else if (simplex) {
+        // triangles and tetrahedra: element records and block lists, also
+        // without a Jacobian, so that the defect is bitwise the same
+        const SxLists l{h->sx_blk.as<uint32_t>(), h->sx_node.as<int32_t>(), h->sx_items.as<uint16_t>(),
+                        h->sx_wg.as<int32_t>()};
+        e = launch_assemble_simplex(h->et, jprec, l, m, k, u, u_old, jvals, defect, h->errflag.as<int>(), h->ne, h->sx_nwg,
+                                    sx_recs, (hipStream_t)stream);
+        h->last_path = 0;
+    } else if (split && jprec == NSFV1_F32) {
         // also without a Jacobian (defect only): the gather then reads only
         // the records' fluxes, and the defect is bitwise the one assembled
         // together with the Jacobian
-        // triangles and tetrahedra: element records and block lists (16-byte
-        // stores need an aligned J in 3D); the row-lane gather on request
-        const bool simplex = h->sx_valid && !(h->path == 2 && P.rowlane) &&
-                             (h->dim == 2 || ((uintptr_t)jvals & 15) == 0);
         const size_t need = sizeof(float) * (size_t)split_record_floats(h->et, h->ne);
         float* recs = static_cast<float*>(scratch);
-        if (scratch) {
-            if (need > NOALLOC_SCRATCH_BYTES)
-                return fail(NSFV1_ERR_ARGUMENT, "the split path needs " + std::to_string(need) +
-                                                    " bytes of SCVF records for this mesh; the no-allocation entry holds at most " +
-                                                    std::to_string(NOALLOC_SCRATCH_BYTES));
-        } else {
-            const size_t take = simplex ? (size_t)simplex_record_bytes(h->et, h->ne) : need;
-            if (h->recs.n < take && h->recs.alloc(take) != hipSuccess) return fail(NSFV1_ERR_DEVICE, "record buffer");
+        if (!scratch) {
+            if (h->recs.n < need && h->recs.alloc(need) != hipSuccess) return fail(NSFV1_ERR_DEVICE, "record buffer");
             recs = h->recs.as<float>();
         }
-        if (simplex) {
-            const SxLists l{h->sx_blk.as<uint32_t>(), h->sx_node.as<int32_t>(), h->sx_items.as<uint16_t>(),
-                            h->sx_wg.as<int32_t>()};
-            e = launch_assemble_simplex(h->et, l, m, k, u, u_old, static_cast<float*>(jvals), defect, h->errflag.as<int>(),
-                                        h->ne, h->sx_nwg, recs, (hipStream_t)stream);
-        } else
-            e = launch_assemble_split(h->et, m, k, u, u_old, static_cast<float*>(jvals), defect, h->errflag.as<int>(), P.nwg,
-                                      P.lds, h->ne, recs, h->path == 2 && P.rowlane, (hipStream_t)stream);
+        e = launch_assemble_split(h->et, m, k, u, u_old, static_cast<float*>(jvals), defect, h->errflag.as<int>(), P.nwg,
+                                  P.lds, h->ne, recs, h->path == 2 && P.rowlane, (hipStream_t)stream);
         h->last_path = (h->path == 2 && P.rowlane) ? 2 : 0;
     } else {
         e = launch_assemble(h->et, jprec, m, k, u, u_old, jvals, defect, h->errflag.as<int>(), P.nwg, P.lds,

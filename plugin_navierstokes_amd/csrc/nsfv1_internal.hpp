@@ -61,12 +61,12 @@ struct SxLists {
     uint16_t* items;        // [nsh ninc] incidence of the node << 2 | corner of the neighbour, per node sorted by block
     const int32_t* wg_node; // [nwg + 1] first node of each workgroup (at most 255 nodes, 256 incidences)
 };
-bool simplex_supported(int et, int64_t max_inc);
-int64_t simplex_record_bytes(int et, int64_t ne);
+bool simplex_supported(int et, int jprec, int64_t max_inc);
+int64_t simplex_record_bytes(int et, int jprec, int64_t ne);
 hipError_t launch_simplex_lists(int et, const SxLists& l, const KMeshPtrs& m, int64_t nv, hipStream_t stream);
-hipError_t launch_assemble_simplex(int et, const SxLists& l, const KMeshPtrs& m, const KParams& p, const double* u,
-                                   const double* uold, float* J, double* d, int* err, int64_t ne, int nwg, void* recs,
-                                   hipStream_t stream);
+hipError_t launch_assemble_simplex(int et, int jprec, const SxLists& l, const KMeshPtrs& m, const KParams& p,
+                                   const double* u, const double* uold, void* J, double* d, int* err, int64_t ne,
+                                   int nwg, void* recs, hipStream_t stream);
 
 // stabilised SCVF velocities of every element: out[ne][nip][dim]
 hipError_t launch_export_stab_vel(int et, const KMeshPtrs& m, const KParams& p, const double* u, const double* uold,

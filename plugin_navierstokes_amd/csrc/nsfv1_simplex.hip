@@ -1,5 +1,5 @@
-// nsfv1_simplex.hip -- assembly of triangle and tetrahedron meshes with FP32
-// Jacobian in the common configuration (FIELDS, one upwind object of type
+// nsfv1_simplex.hip -- assembly of triangle and tetrahedron meshes in the
+// common configuration (FIELDS, one upwind object of type
 // no/full/skewed/LPS, no Stokes/PAC/Peclet/exact terms): one lane per element
 // evaluates every SCVF once, one lane per (node, element) forms the rows'
 // contributions, and lanes that own blocks add them.
@@ -7,8 +7,8 @@
 //   simplex_records  one lane per element, in the element's own corner order:
 //     the shape gradients are constant, so they, the inverse Jacobian and the
 //     state gradients are formed once for all SCVFs.  Writes the corner
-//     gradients, a 48-byte FP32 record per SCVF and the FP64 defect of every
-//     corner (the SCVF fluxes already added with their signs).
+//     gradients, a record of 12 values per SCVF (in the Jacobian's type) and
+//     the FP64 defect of every corner (the SCVF fluxes already added).
 //   simplex_rows     a workgroup owns consecutive nodes, a lane one incidence:
 //     it forms the element's row block of the node from the record and puts
 //     it into LDS, two rows at a time; then one lane per (block, row) adds the
@@ -31,21 +31,49 @@
 
 namespace nsfv1 {
 
-// Record of an element, in 16-byte chunks.  The chunks of eight consecutive
-// elements are interleaved (chunk c of the eight: 128 contiguous bytes), so a
-// wave writes whole cache lines and neighbouring elements share them when
-// read.
-template <int ET>
+// Record of an element, in 16-byte chunks of VT (the Jacobian's type).  The
+// chunks of eight consecutive elements are interleaved (chunk c of the eight:
+// 128 contiguous bytes), so a wave writes whole cache lines and neighbouring
+// elements share them when read.
+template <int ET, typename VT>
 struct SxRec {
     static constexpr int D = Topo<ET>::dim, N = Topo<ET>::nsh, NC = D + 1, NIP = Topo<ET>::nip;
-    static constexpr int GS = D == 2 ? 2 : 4;              // floats per corner gradient
-    static constexpr int G = 0;                            // corner gradients
-    static constexpr int S = (N * GS + 3) / 4 * 4;         // per SCVF 12 floats:
+    static constexpr int GS = D == 2 ? 2 : 4;              // values per corner gradient
+    static constexpr int S = (N * GS + 3) / 4 * 4;         // after the gradients, per SCVF 12 values:
     //   normal (from -> to) and flux weight | vv, vc, sp factors, -nu rho | upwind shapes
-    static constexpr int FLOATS = S + 12 * NIP;
-    static constexpr int DEF = FLOATS / 4;                 // first chunk of the corner defects
+    static constexpr int VALUES = S + 12 * NIP;
+    static constexpr int VPC = 16 / (int)sizeof(VT);
+    static constexpr int DEF = VALUES / VPC;               // first chunk of the corner defects
     static constexpr int CHUNKS = DEF + (N * NC + 1) / 2;
 };
+
+// four values of a record from value i (a multiple of four)
+template <typename VT>
+struct Sx4 {
+    VT x, y, z, w;
+};
+template <typename VT>
+__device__ __forceinline__ void sx_put(float4* rec, int i, double a, double b, double c, double d)
+{
+    if constexpr (sizeof(VT) == 4) {
+        rec[i / 4 * 8] = make_float4((float)a, (float)b, (float)c, (float)d);
+    } else {
+        *reinterpret_cast<double2*>(rec + i / 2 * 8) = make_double2(a, b);
+        *reinterpret_cast<double2*>(rec + (i / 2 + 1) * 8) = make_double2(c, d);
+    }
+}
+template <typename VT>
+__device__ __forceinline__ Sx4<VT> sx_get(const float4* rec, int i)
+{
+    if constexpr (sizeof(VT) == 4) {
+        const float4 t = rec[i / 4 * 8];
+        return {t.x, t.y, t.z, t.w};
+    } else {
+        const double2 a = *reinterpret_cast<const double2*>(rec + i / 2 * 8);
+        const double2 b = *reinterpret_cast<const double2*>(rec + (i / 2 + 1) * 8);
+        return {a.x, a.y, b.x, b.y};
+    }
+}
 
 // SCVFs at a corner: the SCVF, the other end of its edge, whether the corner is
 // its `from` corner, packed for lookups by a lane's corner
@@ -67,10 +95,10 @@ struct SxCorner {
     static constexpr uint64_t IP = pack(0), OTHER = pack(1), FROM = pack(2);
 };
 
-template <int ET>
-__device__ __forceinline__ int64_t sx_chunk(int64_t e, int c)
+template <int ET, typename VT>
+__device__ __forceinline__ int64_t sx_first(int64_t e)
 {
-    return ((e >> 3) * SxRec<ET>::CHUNKS + c) * 8 + (e & 7);
+    return (e >> 3) * (SxRec<ET, VT>::CHUNKS * 8) + (e & 7);
 }
 
 // upwind of SCVF IP (upwind.cpp:52-80, 133-172, 337-430, 505-575) in the
@@ -172,12 +200,12 @@ struct SxElem {
     double *uo, *d;  // this lane's old velocities and defect sums in LDS, value i at i * SX_REC_BLOCK
 };
 
-template <int ET, int FAST, int IP>
+template <int ET, typename VT, int FAST, int IP>
 __device__ __forceinline__ void sx_scvf(SxElem<ET>& E, const KParams& P, double nu, const double* __restrict__ l2,
                                         uint8_t* dec, float4* __restrict__ rec, bool wantJ, bool& oku)
 {
     using T = Topo<ET>;
-    using R = SxRec<ET>;
+    using R = SxRec<ET, VT>;
     constexpr int D = T::dim, N = T::nsh, NC = D + 1;
     if constexpr (IP < T::nip) {
         double ipg[D], n[D], me[D], sv[D], pr = 0.0;
@@ -240,24 +268,23 @@ __device__ __forceinline__ void sx_scvf(SxElem<ET>& E, const KParams& P, double 
             E.d[(T::edge[IP][1] * NC + a) * SX_REC_BLOCK] -= fl[a];
         }
         if (wantJ) {
-            constexpr int C = (R::S + 12 * IP) / 4;
-            rec[C * 8] = make_float4((float)n[0], (float)n[1], D == 3 ? (float)n[D - 1] : 0.f, (float)prod);
-            rec[(C + 1) * 8] = make_float4((float)(vv * idg), (float)(vc * idg), (float)(-P.inv_rho * idg),
-                                           (float)(-1.0 * nu * P.rho));
-            rec[(C + 2) * 8] = make_float4((float)U[0], (float)U[1], (float)U[2], N == 4 ? (float)U[N - 1] : 0.f);
+            constexpr int C = R::S + 12 * IP;
+            sx_put<VT>(rec, C, n[0], n[1], D == 3 ? n[D - 1] : 0.0, prod);
+            sx_put<VT>(rec, C + 4, vv * idg, vc * idg, -P.inv_rho * idg, -1.0 * nu * P.rho);
+            sx_put<VT>(rec, C + 8, U[0], U[1], U[2], N == 4 ? U[N - 1] : 0.0);
         }
         __builtin_amdgcn_sched_barrier(0);  // one SCVF's values at a time in registers
-        sx_scvf<ET, FAST, IP + 1>(E, P, nu, l2, dec, rec, wantJ, oku);
+        sx_scvf<ET, VT, FAST, IP + 1>(E, P, nu, l2, dec, rec, wantJ, oku);
     }
 }
 
-template <int ET, int FAST>
+template <int ET, typename VT, int FAST>
 __global__ void __launch_bounds__(SX_REC_BLOCK, 2)
 simplex_records(KMeshPtrs M, KParams P, const double* __restrict__ u, const double* __restrict__ uold, int64_t ne,
                 float4* __restrict__ recs, int wantJ, int* __restrict__ err)
 {
     using T = Topo<ET>;
-    using R = SxRec<ET>;
+    using R = SxRec<ET, VT>;
     constexpr int D = T::dim, N = T::nsh, NC = D + 1, NIP = T::nip;
     const int64_t e = (int64_t)blockIdx.x * SX_REC_BLOCK + threadIdx.x;
     __shared__ double lds[N * (NC + D) * SX_REC_BLOCK];
@@ -329,19 +356,18 @@ simplex_records(KMeshPtrs M, KParams P, const double* __restrict__ u, const doub
             for (int k = 0; k < N; ++k) s += E.ul[k][a] * E.g[k][i];
             E.gv[a][i] = s;
         }
-    float4* rec = recs + sx_chunk<ET>(e, 0);
+    float4* rec = recs + sx_first<ET, VT>(e);
     if (wantJ) {
         if constexpr (D == 3) {
 #pragma unroll
-            for (int k = 0; k < N; ++k)
-                rec[k * 8] = make_float4((float)E.g[k][0], (float)E.g[k][1], (float)E.g[k][2], 0.f);
+            for (int k = 0; k < N; ++k) sx_put<VT>(rec, 4 * k, E.g[k][0], E.g[k][1], E.g[k][D - 1], 0.0);
         } else {
-            rec[0] = make_float4((float)E.g[0][0], (float)E.g[0][1], (float)E.g[1][0], (float)E.g[1][1]);
-            rec[8] = make_float4((float)E.g[2][0], (float)E.g[2][1], 0.f, 0.f);
+            sx_put<VT>(rec, 0, E.g[0][0], E.g[0][1], E.g[1][0], E.g[1][1]);
+            sx_put<VT>(rec, 4, E.g[2][0], E.g[2][1], 0.0, 0.0);
         }
     }
     uint8_t* dec = (P.upw_mode != 0 && M.upw_dec) ? M.upw_dec + e * NIP : nullptr;
-    sx_scvf<ET, FAST, 0>(E, P, M.nu_elem ? M.nu_elem[e] : P.nu, M.l2inv + e * NIP, dec, rec, wantJ != 0, oku);
+    sx_scvf<ET, VT, FAST, 0>(E, P, M.nu_elem ? M.nu_elem[e] : P.nu, M.l2inv + e * NIP, dec, rec, wantJ != 0, oku);
     if (!oku) kernel_error(err, KERR_CUT_SIDE);
     if (!okg) kernel_error(err, KERR_DEGENERATE);
     double f[(N * NC + 1) / 2 * 2];
@@ -352,26 +378,64 @@ simplex_records(KMeshPtrs M, KParams P, const double* __restrict__ u, const doub
         *reinterpret_cast<double2*>(rec + (R::DEF + q) * 8) = make_double2(f[2 * q], f[2 * q + 1]);
 }
 
+// NC values of a row segment, in 16-byte pieces where there are four
+template <int NC, typename VT>
+__device__ __forceinline__ void sx_seg_put(VT* p, const VT (&x)[NC])
+{
+    if constexpr (NC == 4 && sizeof(VT) == 4) {
+        *reinterpret_cast<float4*>(p) = make_float4(x[0], x[1], x[2], x[3]);
+    } else if constexpr (NC == 4) {
+        reinterpret_cast<double2*>(p)[0] = make_double2(x[0], x[1]);
+        reinterpret_cast<double2*>(p)[1] = make_double2(x[2], x[3]);
+    } else {
+#pragma unroll
+        for (int c = 0; c < NC; ++c) p[c] = x[c];
+    }
+}
+template <int NC, typename VT>
+__device__ __forceinline__ void sx_seg_get(const VT* p, VT (&x)[NC])
+{
+    if constexpr (NC == 4 && sizeof(VT) == 4) {
+        const float4 t = *reinterpret_cast<const float4*>(p);
+        x[0] = t.x;
+        x[1] = t.y;
+        x[2] = t.z;
+        x[3] = t.w;
+    } else if constexpr (NC == 4) {
+        const double2 a = reinterpret_cast<const double2*>(p)[0], b = reinterpret_cast<const double2*>(p)[1];
+        x[0] = a.x;
+        x[1] = a.y;
+        x[2] = b.x;
+        x[3] = b.y;
+    } else {
+#pragma unroll
+        for (int c = 0; c < NC; ++c) x[c] = p[c];
+    }
+}
+
+// rows per pass: 32 KB of segments for 256 lanes, so four workgroups fit a CU
+template <typename VT>
+constexpr int SX_RP = sizeof(VT) == 4 ? 2 : 1;
+
 // Row gather.  Block b of the pattern (node v, neighbour slot) is described by
 // L.blk[b] = slot | first item << 8 | items << 18, the item positions relative
 // to the node's, and L.items = incidence of the node << 2 | corner of the
 // neighbour in that element, sorted by block, then element.
-template <int ET>
+template <int ET, typename VT>
 __global__ void __launch_bounds__(256)
 simplex_rows(SxLists L, KMeshPtrs M, KParams P, const double* __restrict__ u, const float4* __restrict__ recs,
-             float* __restrict__ J, double* __restrict__ dout)
+             VT* __restrict__ J, double* __restrict__ dout)
 {
     using T = Topo<ET>;
-    using R = SxRec<ET>;
+    using R = SxRec<ET, VT>;
     using C = SxCorner<ET>;
     constexpr int D = T::dim, N = T::nsh, NC = D + 1;
-    constexpr int RP = 2;                       // rows per pass
+    constexpr int RP = SX_RP<VT>;
     constexpr int NB = 256;                     // lanes of the LDS layout
-    constexpr int Q = NC == 4 ? 4 : 3;          // floats per (block, row)
     extern __shared__ __align__(16) unsigned char smem[];
     // [corner][row of the pass][lane] row segments; the node table; the items
-    float* seg = reinterpret_cast<float*>(smem);                           // N * RP * NB * Q
-    int* ntab = reinterpret_cast<int*>(smem + sizeof(float) * N * RP * NB * Q);  // per node: first lane, first block
+    VT* seg = reinterpret_cast<VT*>(smem);                                        // N * RP * NB * NC
+    int* ntab = reinterpret_cast<int*>(smem + sizeof(VT) * N * RP * NB * NC);     // per node: first lane, first block
     uint16_t* sit = reinterpret_cast<uint16_t*>(ntab + 2 * (NB + 1));      // items of the workgroup: N * NB
     double* dseg = reinterpret_cast<double*>(smem);                        // defects [component][lane], after the passes
     // consecutive workgroups (shared element data) go to the same XCD
@@ -383,7 +447,7 @@ simplex_rows(SxLists L, KMeshPtrs M, KParams P, const double* __restrict__ u, co
     const int v0 = L.wg_node[w], v1 = L.wg_node[w + 1], nn = v1 - v0;
     const int t = threadIdx.x, nt = (int)blockDim.x;
     const int i0 = M.node_inc[v0], i1 = M.node_inc[v1];
-    const bool wantJ = J != nullptr;
+    const bool wantJ = J != nullptr, vec = ((uintptr_t)J & 15) == 0;
     if (t <= nn) {
         ntab[2 * t] = M.node_inc[v0 + t] - i0;
         ntab[2 * t + 1] = (int)(M.rowptr[(int64_t)(v0 + t) * NC] / (NC * NC));
@@ -392,7 +456,7 @@ simplex_rows(SxLists L, KMeshPtrs M, KParams P, const double* __restrict__ u, co
         for (int i = t; i < N * (i1 - i0); i += nt) sit[i] = L.items[(int64_t)N * i0 + i];
     const int inc = i0 + t;
     const bool active = inc < i1;
-    float B[N][NC][NC];
+    VT B[N][NC][NC];
     double dl[NC];
 #pragma unroll
     for (int a = 0; a < NC; ++a) dl[a] = 0.0;
@@ -401,11 +465,11 @@ simplex_rows(SxLists L, KMeshPtrs M, KParams P, const double* __restrict__ u, co
 #pragma unroll
         for (int a = 0; a < NC; ++a)
 #pragma unroll
-            for (int c = 0; c < NC; ++c) B[k][a][c] = 0.f;
+            for (int c = 0; c < NC; ++c) B[k][a][c] = VT(0);
     if (active) {
         const int64_t e = M.inc_elem[inc];
         const int kv = M.inc_info[inc] & 0xff;
-        const float4* rec = recs + sx_chunk<ET>(e, 0);
+        const float4* rec = recs + sx_first<ET, VT>(e);
 #pragma unroll
         for (int q = 0; q < (NC + 1) / 2; ++q) {
             // N NC doubles in chunks of two; a corner of a triangle starts mid-chunk
@@ -421,17 +485,17 @@ simplex_rows(SxLists L, KMeshPtrs M, KParams P, const double* __restrict__ u, co
             }
         }
         if (wantJ) {
-            float g[N][D];
+            VT g[N][D];
             if constexpr (D == 3) {
 #pragma unroll
                 for (int k = 0; k < N; ++k) {
-                    const float4 x = rec[k * 8];
+                    const Sx4<VT> x = sx_get<VT>(rec, 4 * k);
                     g[k][0] = x.x;
                     g[k][1] = x.y;
                     g[k][D - 1] = x.z;
                 }
             } else {
-                const float4 x = rec[0], y = rec[8];
+                const Sx4<VT> x = sx_get<VT>(rec, 0), y = sx_get<VT>(rec, 4);
                 g[0][0] = x.x;
                 g[0][1] = x.y;
                 g[1][0] = x.z;
@@ -440,32 +504,32 @@ simplex_rows(SxLists L, KMeshPtrs M, KParams P, const double* __restrict__ u, co
                 g[N - 1][1] = y.y;
             }
             // shape values at an SCVF's ip: one for the ends of its edge, one for the rest
-            constexpr float PE = (float)TabH<ET>::t.phi[0][T::edge[0][0]];
-            constexpr float PO = (float)TabH<ET>::t.phi[0][3 - T::edge[0][0] - T::edge[0][1]];
-            const float s_ = (float)P.s_a, rh = (float)P.rho;
+            constexpr VT PE = (VT)TabH<ET>::t.phi[0][T::edge[0][0]];
+            constexpr VT PO = (VT)TabH<ET>::t.phi[0][3 - T::edge[0][0] - T::edge[0][1]];
+            const VT s_ = (VT)P.s_a, rh = (VT)P.rho;
             // navier_stokes_fv1.cpp:317-593 for the SCVFs at the corner
 #pragma unroll
             for (int q = 0; q < T::cip; ++q) {
                 const int sh = 3 * (3 * kv + q);
                 const int ip = (int)(C::IP >> sh) & 7, oth = (int)(C::OTHER >> sh) & 7;
-                const float sg = ((C::FROM >> sh) & 1) ? 1.f : -1.f;
-                const float4* r = rec + (R::S / 4 + 3 * ip) * 8;
-                const float4 A = r[0], F = r[8], Ux = r[16];
-                const float Us[4] = {Ux.x, Ux.y, Ux.z, Ux.w};
-                float n[D];
+                const VT sg = ((C::FROM >> sh) & 1) ? VT(1) : VT(-1);
+                const float4* r = rec + 12 * ip / R::VPC * 8;
+                const Sx4<VT> A = sx_get<VT>(r, R::S), F = sx_get<VT>(r, R::S + 4), Ux = sx_get<VT>(r, R::S + 8);
+                const VT Us[4] = {Ux.x, Ux.y, Ux.z, Ux.w};
+                VT n[D];
                 n[0] = sg * A.x;
                 n[1] = sg * A.y;
                 if constexpr (D == 3) n[D - 1] = sg * A.z;
-                const float pw = sg * A.w, nr = F.w;
+                const VT pw = sg * A.w, nr = F.w;
 #pragma unroll
                 for (int k = 0; k < N; ++k) {
-                    const float ph = (k == kv || k == oth) ? PE : PO;
-                    const float Sv = F.x * ph + F.y * Us[k];
-                    float gn = 0.f;
+                    const VT ph = (k == kv || k == oth) ? PE : PO;
+                    const VT Sv = F.x * ph + F.y * Us[k];
+                    VT gn = VT(0);
 #pragma unroll
                     for (int i = 0; i < D; ++i) gn += g[k][i] * n[i];
-                    const float dg = nr * gn + Us[k] * pw;
-                    float cpp = 0.f;
+                    const VT dg = nr * gn + Us[k] * pw;
+                    VT cpp = VT(0);
 #pragma unroll
                     for (int a = 0; a < D; ++a) {
                         B[k][a][a] += s_ * dg;
@@ -489,7 +553,7 @@ simplex_rows(SxLists L, KMeshPtrs M, KParams P, const double* __restrict__ u, co
 #pragma unroll
                 for (int a = 0; a < D; ++a) {
 #pragma unroll
-                    for (int k = 0; k < N; ++k) B[k][a][a] += k == kv ? (float)(P.s_m * m) : 0.f;
+                    for (int k = 0; k < N; ++k) B[k][a][a] += k == kv ? (VT)(P.s_m * m) : VT(0);
                     dl[a] += P.s_m * (uv[a] * m);
                 }
             }
@@ -507,16 +571,7 @@ simplex_rows(SxLists L, KMeshPtrs M, KParams P, const double* __restrict__ u, co
             for (int k = 0; k < N; ++k)
 #pragma unroll
                 for (int r = 0; r < RP; ++r)
-                    if (r0 + r < NC) {
-                        float* p = seg + ((k * RP + r) * NB + t) * Q;
-                        const int a = r0 + r < NC ? r0 + r : 0;
-                        if constexpr (NC == 4) {
-                            *reinterpret_cast<float4*>(p) = make_float4(B[k][a][0], B[k][a][1], B[k][a][2], B[k][a][NC - 1]);
-                        } else {
-#pragma unroll
-                            for (int c = 0; c < NC; ++c) p[c] = B[k][a][c];
-                        }
-                    }
+                    if (r0 + r < NC) sx_seg_put<NC>(seg + ((k * RP + r) * NB + t) * NC, B[k][r0 + r < NC ? r0 + r : 0]);
             __syncthreads();
             // one lane per (block, row): rows of a block side by side
             for (int x = t; x < (b1 - b0) * RP; x += nt) {
@@ -527,28 +582,20 @@ simplex_rows(SxLists L, KMeshPtrs M, KParams P, const double* __restrict__ u, co
                 const int slot = info & 0xff, first = (info >> 8) & 0x3ff, cnt = info >> 18;
                 const int lane0 = ntab[2 * v];
                 const uint16_t* it = sit + N * lane0 + first;
-                float s[NC];
+                VT s[NC], y[NC];
 #pragma unroll
-                for (int c = 0; c < NC; ++c) s[c] = 0.f;
+                for (int c = 0; c < NC; ++c) s[c] = VT(0);
 #pragma unroll 4
                 for (int i = 0; i < cnt; ++i) {
                     const int z = it[i];
-                    const float* p = seg + (((z & 3) * RP + r) * NB + lane0 + (z >> 2)) * Q;
-                    if constexpr (NC == 4) {
-                        const float4 y = *reinterpret_cast<const float4*>(p);
-                        s[0] += y.x;
-                        s[1] += y.y;
-                        s[2] += y.z;
-                        s[NC - 1] += y.w;
-                    } else {
+                    sx_seg_get<NC>(seg + (((z & 3) * RP + r) * NB + lane0 + (z >> 2)) * NC, y);
 #pragma unroll
-                        for (int c = 0; c < NC; ++c) s[c] += p[c];
-                    }
+                    for (int c = 0; c < NC; ++c) s[c] += y[c];
                 }
                 const int bv = ntab[2 * v + 1], nb = ntab[2 * v + 3] - bv;
-                float* dst = J + (int64_t)bv * (NC * NC) + (int64_t)(r0 + r) * (nb * NC) + slot * NC;
-                if constexpr (NC == 4) {
-                    *reinterpret_cast<float4*>(dst) = make_float4(s[0], s[1], s[2], s[NC - 1]);
+                VT* dst = J + (int64_t)bv * (NC * NC) + (int64_t)(r0 + r) * (nb * NC) + slot * NC;
+                if (vec) {
+                    sx_seg_put<NC>(dst, s);
                 } else {
 #pragma unroll
                     for (int c = 0; c < NC; ++c) dst[c] = s[c];
@@ -571,11 +618,11 @@ simplex_rows(SxLists L, KMeshPtrs M, KParams P, const double* __restrict__ u, co
     }
 }
 
-template <int ET>
+template <int ET, typename VT>
 constexpr size_t sx_lds()
 {
     constexpr int N = Topo<ET>::nsh, NC = Topo<ET>::dim + 1;
-    return sizeof(float) * N * 2 * 256 * (NC == 4 ? 4 : 3) + sizeof(int) * 2 * 257 + sizeof(uint16_t) * N * 256;
+    return sizeof(VT) * N * SX_RP<VT> * 256 * NC + sizeof(int) * 2 * 257 + sizeof(uint16_t) * N * 256;
 }
 
 // the lists of a mesh (once per plan)
@@ -625,15 +672,19 @@ simplex_lists(SxLists L, KMeshPtrs M, int64_t nv)
 // ---------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------
-bool simplex_supported(int et, int64_t max_inc)
+// Triangles with FP64 Jacobian stay on the fused kernel: 300 x 300 cells 39 (full
+// upwind) and 62 us (LPS) against 54 and 55 us; tetrahedra 200 against 80 us (22^3
+// cells, LPS) and 42 against 33 us (6^3)
+bool simplex_supported(int et, int jprec, int64_t max_inc)
 {
     // list fields: 10 bits for a node's items, so at most 255 incidences a node
-    return (et == ET_TRI || et == ET_TET) && max_inc <= 255;
+    return ((et == ET_TRI && jprec == 32) || et == ET_TET) && max_inc <= 255;
 }
 
-int64_t simplex_record_bytes(int et, int64_t ne)
+int64_t simplex_record_bytes(int et, int jprec, int64_t ne)
 {
-    const int64_t chunks = et == ET_TRI ? SxRec<ET_TRI>::CHUNKS : SxRec<ET_TET>::CHUNKS;
+    const int64_t chunks = et == ET_TRI ? SxRec<ET_TRI, float>::CHUNKS
+                                        : (jprec == 64 ? SxRec<ET_TET, double>::CHUNKS : SxRec<ET_TET, float>::CHUNKS);
     return (ne + 7) / 8 * 8 * chunks * 16;
 }
 
@@ -647,34 +698,37 @@ hipError_t launch_simplex_lists(int et, const SxLists& l, const KMeshPtrs& m, in
     return hipGetLastError();
 }
 
-template <int ET>
+template <int ET, typename VT>
 static hipError_t launch_simplex_et(const SxLists& l, const KMeshPtrs& m, const KParams& p, const double* u,
-                                    const double* uold, float* J, double* d, int* err, int64_t ne, int nwg,
+                                    const double* uold, void* J, double* d, int* err, int64_t ne, int nwg,
                                     float4* recs, hipStream_t s)
 {
     const unsigned ge = (unsigned)((ne + SX_REC_BLOCK - 1) / SX_REC_BLOCK);
     const int wj = J != nullptr;
     if (ne > 0) {
         switch (p.conv_upwind) {
-        case UPW_NO: simplex_records<ET, UPW_NO><<<ge, SX_REC_BLOCK, 0, s>>>(m, p, u, uold, ne, recs, wj, err); break;
-        case UPW_FULL: simplex_records<ET, UPW_FULL><<<ge, SX_REC_BLOCK, 0, s>>>(m, p, u, uold, ne, recs, wj, err); break;
-        case UPW_SKEWED: simplex_records<ET, UPW_SKEWED><<<ge, SX_REC_BLOCK, 0, s>>>(m, p, u, uold, ne, recs, wj, err); break;
-        case UPW_LPS: simplex_records<ET, UPW_LPS><<<ge, SX_REC_BLOCK, 0, s>>>(m, p, u, uold, ne, recs, wj, err); break;
+        case UPW_NO: simplex_records<ET, VT, UPW_NO><<<ge, SX_REC_BLOCK, 0, s>>>(m, p, u, uold, ne, recs, wj, err); break;
+        case UPW_FULL: simplex_records<ET, VT, UPW_FULL><<<ge, SX_REC_BLOCK, 0, s>>>(m, p, u, uold, ne, recs, wj, err); break;
+        case UPW_SKEWED: simplex_records<ET, VT, UPW_SKEWED><<<ge, SX_REC_BLOCK, 0, s>>>(m, p, u, uold, ne, recs, wj, err); break;
+        case UPW_LPS: simplex_records<ET, VT, UPW_LPS><<<ge, SX_REC_BLOCK, 0, s>>>(m, p, u, uold, ne, recs, wj, err); break;
         default: return hipErrorInvalidValue;
         }
     }
-    static_assert(sx_lds<ET>() <= 64 * 1024, "dynamic LDS limit");
-    if (nwg > 0) simplex_rows<ET><<<nwg, 256, sx_lds<ET>(), s>>>(l, m, p, u, recs, J, d);
+    static_assert(sx_lds<ET, VT>() <= 64 * 1024, "dynamic LDS limit");
+    if (nwg > 0)
+        simplex_rows<ET, VT><<<nwg, 256, sx_lds<ET, VT>(), s>>>(l, m, p, u, recs, static_cast<VT*>(J), d);
     return hipGetLastError();
 }
 
-hipError_t launch_assemble_simplex(int et, const SxLists& l, const KMeshPtrs& m, const KParams& p, const double* u,
-                                   const double* uold, float* J, double* d, int* err, int64_t ne, int nwg, void* recs,
-                                   hipStream_t s)
+hipError_t launch_assemble_simplex(int et, int jprec, const SxLists& l, const KMeshPtrs& m, const KParams& p,
+                                   const double* u, const double* uold, void* J, double* d, int* err, int64_t ne,
+                                   int nwg, void* recs, hipStream_t s)
 {
     float4* r = static_cast<float4*>(recs);
-    if (et == ET_TRI) return launch_simplex_et<ET_TRI>(l, m, p, u, uold, J, d, err, ne, nwg, r, s);
-    if (et == ET_TET) return launch_simplex_et<ET_TET>(l, m, p, u, uold, J, d, err, ne, nwg, r, s);
+    if (et == ET_TRI && jprec == 32) return launch_simplex_et<ET_TRI, float>(l, m, p, u, uold, J, d, err, ne, nwg, r, s);
+    if (et == ET_TET)
+        return jprec == 64 ? launch_simplex_et<ET_TET, double>(l, m, p, u, uold, J, d, err, ne, nwg, r, s)
+                           : launch_simplex_et<ET_TET, float>(l, m, p, u, uold, J, d, err, ne, nwg, r, s);
     return hipErrorInvalidValue;
 }
 
