@@ -1318,7 +1318,15 @@ static int assemble_impl(nsfv1_handle* h, const double* u, const double* u_old, 
                                                 " bytes of SCVF records for this mesh; the no-allocation entry holds at most " +
                                                 std::to_string(NOALLOC_SCRATCH_BYTES));
     }
-    bool simplex = split && h->sx_valid && (jprec == NSFV1_F32 || h->et == ET_TET) &&
+    // 2D with FP32 Jacobian by default: the fused kernel without a ray cast (the
+    // second kernel and the records cost more than the doubled SCVF work: 500 x 500
+    // quads 63 against 83 us, 512 x 512 x 2 triangles 88 against 112 us) and below 96 Ki
+    // elements with one (LPS, 65000 triangles 25 against 29 us, 115000: 36 against
+    // 33 us; 26000 quads 17 against 24 us, 90000: 44 against 46 us, 250000: 105
+    // against 91 us)
+    const bool fused2d = h->path == 3 && h->dim == 2 && jprec == NSFV1_F32 &&
+                         (k.conv_upwind == UPW_NO || k.conv_upwind == UPW_FULL || h->ne < 96 * 1024);
+    bool simplex = split && !fused2d && h->sx_valid && (jprec == NSFV1_F32 || h->et == ET_TET) &&
                    !(h->path == 2 && P.rowlane);
     void* sx_recs = scratch;
     if (simplex) {
@@ -1454,7 +1462,7 @@ static int assemble_impl(nsfv1_handle* h, const double* u, const double* u_old, 
         e = launch_assemble_simplex(h->et, jprec, l, m, k, u, u_old, jvals, defect, h->errflag.as<int>(), h->ne, h->sx_nwg,
                                     sx_recs, (hipStream_t)stream);
         h->last_path = 0;
-    } else if (split && jprec == NSFV1_F32) {
+    } else if (split && jprec == NSFV1_F32 && !fused2d) {
         // also without a Jacobian (defect only): the gather then reads only
         // the records' fluxes, and the defect is bitwise the one assembled
         // together with the Jacobian
