@@ -80,6 +80,11 @@ struct Plan {
     // wg_a[2w+1] = {jbase low, jbase high, jlen, rounds}
     DevBuf lane_a, lane_pos, wg_a;
     bool rowlane = false;  // built for the row-lane split gather
+    // lists of the gathers that sum by owners (rnwg = 0: none), and simplices'
+    // own workgroups
+    DevBuf rown, ritems, rlane, rwg;
+    int rnwg = 0;
+    RowLists rows{};
 };
 
 }  // namespace
@@ -188,10 +193,6 @@ struct nsfv1_handle {
     };
     StreamBuf recs64[4];
     int nrecs64 = 0;
-    // block lists of the simplex path (triangle and tetrahedron meshes)
-    DevBuf sx_blk, sx_node, sx_items, sx_wg;
-    int sx_nwg = 0;
-    bool sx_valid = false;
     int64_t nblk() const { return nnz / ((dim + 1) * (dim + 1)); }
     // 0: split where supported, 1: fused kernel only, 2: split with row lanes,
     // 3: plane march on structured grids of parallelepipeds, otherwise 0
@@ -899,7 +900,6 @@ static int set_mesh_groups(nsfv1_handle* h, const double* xyz, int64_t nv, const
     for (auto& r : h->recs64) r.buf.release();
     h->nrecs64 = 0;
     h->cpl_recs.release();
-    h->sx_valid = false;
     return NSFV1_OK;
 }
 
@@ -1006,7 +1006,7 @@ static int make_plan(nsfv1_handle* h, const IncView& g, int jbytes, Plan& P, int
             const int64_t incs = g.node_inc[v + 1] - g.node_inc[v0];
             const int64_t vals = h->h_rowptr[(v + 1) * nc] - h->h_rowptr[v0 * nc];
             const size_t lds = ((size_t)vals * jbytes + (size_t)(v + 1 - v0) * 16 + 15) / 16 * 16 + (size_t)(v + 1 - v0) * nc * 8;
-            if (incs > inc_budget || lds > h->lds_cap) {
+            if (incs > inc_budget || lds > h->lds_cap || v - v0 >= 255) {
                 if (v == v0) return fail(NSFV1_ERR_ARGUMENT, "one node row exceeds the workgroup budget");
                 break;
             }
@@ -1093,37 +1093,51 @@ static int make_plan(nsfv1_handle* h, const IncView& g, int jbytes, Plan& P, int
     return NSFV1_OK;
 }
 
-// workgroups (nodes with at most 256 incidences together, at most 255 nodes)
-// and block lists of the simplex path, the lists built on the device
-static int ensure_simplex_lists(nsfv1_handle* h, int jprec)
+// lists of the row gathers that sum their blocks by owners: simplices in
+// workgroups of their own (up to 256 incidences and 255 nodes, in the order of
+// the incidences), hexahedra in the plan's workgroups and lane order
+static int make_row_lists(nsfv1_handle* h, int jprec, Plan& P)
 {
-    if (h->sx_valid || h->mixed()) return NSFV1_OK;
-    int64_t most = 0;
-    std::vector<int32_t> wn{0};
-    for (int64_t v = 0, v0 = 0; v < h->nv; ++v) {
-        most = std::max(most, h->h_node_inc[v + 1] - h->h_node_inc[v]);
-        if (h->h_node_inc[v + 1] - h->h_node_inc[v0] > 256 || v - v0 >= 255) {
-            wn.push_back((int32_t)v);
-            v0 = v;
-        }
+    P.rnwg = 0;
+    if (h->mixed()) return NSFV1_OK;
+    const bool simplex = simplex_supported(h->et, jprec);
+    if (!simplex && !(jprec == NSFV1_F32 && !P.rowlane && h->et == ET_HEX)) return NSFV1_OK;
+    std::vector<int32_t> wn;
+    if (simplex) {
+        wn.push_back(0);
+        for (int64_t v = 0, v0 = 0; v < h->nv; ++v)
+            if (h->h_node_inc[v + 1] - h->h_node_inc[v0] > 256 || v - v0 >= 255) {
+                wn.push_back((int32_t)v);
+                v0 = v;
+            }
+        wn.push_back((int32_t)h->nv);
+        if (P.rwg.alloc(sizeof(int32_t) * wn.size()) != hipSuccess ||
+            hipMemcpy(P.rwg.p, wn.data(), sizeof(int32_t) * wn.size(), hipMemcpyHostToDevice) != hipSuccess)
+            return fail(NSFV1_ERR_DEVICE, "row lists");
+    } else {
+        wn.resize(P.nwg + 1);
+        if (hipMemcpy(wn.data(), P.wg_node.p, sizeof(int32_t) * wn.size(), hipMemcpyDeviceToHost) != hipSuccess)
+            return fail(NSFV1_ERR_DEVICE, "row lists");
     }
-    wn.push_back((int32_t)h->nv);
-    if (!simplex_supported(h->et, jprec, most)) return NSFV1_OK;
-    if (h->sx_blk.alloc(sizeof(uint32_t) * h->nblk()) != hipSuccess ||
-        h->sx_node.alloc(sizeof(int32_t) * h->nblk()) != hipSuccess ||
-        h->sx_items.alloc(sizeof(uint16_t) * h->ninc * nsh_count(h->et)) != hipSuccess ||
-        h->sx_wg.alloc(sizeof(int32_t) * wn.size()) != hipSuccess ||
-        hipMemcpy(h->sx_wg.p, wn.data(), sizeof(int32_t) * wn.size(), hipMemcpyHostToDevice) != hipSuccess)
-        return fail(NSFV1_ERR_DEVICE, "block lists");
+    const int nwg = (int)wn.size() - 1, nc = h->dim + 1;
+    int64_t cap = 0;
+    for (int w = 0; w < nwg; ++w)
+        cap = std::max(cap, (h->h_rowptr[(int64_t)wn[w + 1] * nc] - h->h_rowptr[(int64_t)wn[w] * nc]) / (nc * nc));
+    if (P.rown.alloc(sizeof(uint2) * h->nblk()) != hipSuccess ||
+        P.ritems.alloc(sizeof(uint16_t) * h->ninc * nsh_count(h->et)) != hipSuccess ||
+        P.rlane.alloc((size_t)h->ninc) != hipSuccess)
+        return fail(NSFV1_ERR_DEVICE, "row lists");
     KMeshPtrs m{};
     m.rowptr = h->rowptr.as<int64_t>();
     m.node_inc = h->node_inc.as<int32_t>();
     m.inc_pos = h->inc_pos.as<uint64_t>();
-    const SxLists l{h->sx_blk.as<uint32_t>(), h->sx_node.as<int32_t>(), h->sx_items.as<uint16_t>(), h->sx_wg.as<int32_t>()};
-    if (launch_simplex_lists(h->et, l, m, h->nv, nullptr) != hipSuccess || hipStreamSynchronize(nullptr) != hipSuccess)
-        return fail(NSFV1_ERR_DEVICE, "block lists");
-    h->sx_nwg = (int)wn.size() - 1;
-    h->sx_valid = true;
+    const int32_t* dwn = simplex ? P.rwg.as<int32_t>() : P.wg_node.as<int32_t>();
+    if (launch_row_lists(h->et, m, dwn, simplex ? nullptr : P.perm.as<int32_t>(), nwg, P.rown.as<uint2>(),
+                         P.ritems.as<uint16_t>(), P.rlane.as<uint8_t>(), nullptr) != hipSuccess ||
+        hipStreamSynchronize(nullptr) != hipSuccess)
+        return fail(NSFV1_ERR_DEVICE, "row lists");
+    P.rnwg = nwg;
+    P.rows = RowLists{P.rown.as<uint2>(), P.ritems.as<uint16_t>(), P.rlane.as<uint8_t>(), dwn, (int)cap};
     return NSFV1_OK;
 }
 
@@ -1239,7 +1253,8 @@ static int assemble_impl(nsfv1_handle* h, const double* u, const double* u_old, 
                                             "needs one nsfv1_assemble call with the same jprec first (it builds the plan)");
         int rc = make_plan(h, IncView{h->h_node_inc, h->h_inc_info, h->h_inc_elem, h->ninc, h->inc_pos},
                            jprec == NSFV1_F64 ? 8 : 4, P);
-        if (!rc) rc = ensure_simplex_lists(h, jprec);
+        if (!rc) rc = make_row_lists(h, jprec, P);
+        if (rc) P.valid = false;
         if (rc) return rc;
     }
     for (auto& gp : h->groups) {
@@ -1326,8 +1341,7 @@ static int assemble_impl(nsfv1_handle* h, const double* u, const double* u_old, 
     // against 91 us)
     const bool fused2d = h->path == 3 && h->dim == 2 && jprec == NSFV1_F32 &&
                          (k.conv_upwind == UPW_NO || k.conv_upwind == UPW_FULL || h->ne < 96 * 1024);
-    bool simplex = split && !fused2d && h->sx_valid && (jprec == NSFV1_F32 || h->et == ET_TET) &&
-                   !(h->path == 2 && P.rowlane);
+    bool simplex = split && !fused2d && P.rnwg > 0 && simplex_supported(h->et, jprec) && !(h->path == 2 && P.rowlane);
     void* sx_recs = scratch;
     if (simplex) {
         const size_t need = (size_t)simplex_record_bytes(h->et, jprec, h->ne);
@@ -1457,9 +1471,7 @@ static int assemble_impl(nsfv1_handle* h, const double* u, const double* u_old, 
     } else if (simplex) {
         // triangles and tetrahedra: element records and block lists, also
         // without a Jacobian, so that the defect is bitwise the same
-        const SxLists l{h->sx_blk.as<uint32_t>(), h->sx_node.as<int32_t>(), h->sx_items.as<uint16_t>(),
-                        h->sx_wg.as<int32_t>()};
-        e = launch_assemble_simplex(h->et, jprec, l, m, k, u, u_old, jvals, defect, h->errflag.as<int>(), h->ne, h->sx_nwg,
+        e = launch_assemble_simplex(h->et, jprec, P.rows, m, k, u, u_old, jvals, defect, h->errflag.as<int>(), h->ne, P.rnwg,
                                     sx_recs, (hipStream_t)stream);
         h->last_path = 0;
     } else if (split && jprec == NSFV1_F32 && !fused2d) {
@@ -1472,7 +1484,7 @@ static int assemble_impl(nsfv1_handle* h, const double* u, const double* u_old, 
             if (h->recs.n < need && h->recs.alloc(need) != hipSuccess) return fail(NSFV1_ERR_DEVICE, "record buffer");
             recs = h->recs.as<float>();
         }
-        e = launch_assemble_split(h->et, m, k, u, u_old, static_cast<float*>(jvals), defect, h->errflag.as<int>(), P.nwg,
+        e = launch_assemble_split(h->et, P.rows, m, k, u, u_old, static_cast<float*>(jvals), defect, h->errflag.as<int>(), P.nwg,
                                   P.lds, h->ne, recs, h->path == 2 && P.rowlane, (hipStream_t)stream);
         h->last_path = (h->path == 2 && P.rowlane) ? 2 : 0;
     } else {

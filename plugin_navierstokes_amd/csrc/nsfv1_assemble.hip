@@ -31,6 +31,7 @@
 #include "nsfv1_geom.hpp"
 #include "nsfv1_internal.hpp"
 #include "nsfv1_ray.hpp"
+#include "nsfv1_rows.hpp"
 #include "nsfv1_topo.hpp"
 
 namespace nsfv1 {
@@ -914,9 +915,10 @@ assemble_rows(KMeshPtrs M, KParams P, const double* __restrict__ u, const double
 //     `from` corner; writes the FP64 flux (added to `from`, subtracted
 //     from `to`) and the FP32 record of its Jacobian block, expressed in
 //     the original corner order and reference frame (128 B per SCVF).
-//   assemble_rows_split: the row-owner gather of assemble_rows, reading the
-//     three records of each (node, element) pair instead of recomputing
-//     them; the `to` row takes the negated block (every term of the block is
+//   assemble_rows_split (quadrilaterals), split_rows (hexahedra; simplices
+//     have element records): a lane per (node, element) pair reads its two or
+//     three records; the blocks are added in rounds as in assemble_rows, or
+//     summed by owners (nsfv1_rows.hpp).  The `to` row takes the negated block (every term of the block is
 //     linear in the normal or in the flux weight).
 // ---------------------------------------------------------------------
 constexpr int REC_FLOATS = 32;
@@ -1066,16 +1068,16 @@ struct IpsOfQ {
 };
 
 template <int ET, int FAST, int Q>
-__global__ void __launch_bounds__(256)
-scvf_records(KMeshPtrs M, KParams P, const double* __restrict__ u, const double* __restrict__ uold, int64_t ne,
-             int64_t ne_pad, float* __restrict__ recs, int* __restrict__ err)
+__device__ __forceinline__ void records_block(const KMeshPtrs& M, const KParams& P, const double* __restrict__ u,
+                                              const double* __restrict__ uold, int64_t ne, int64_t ne_pad,
+                                              float* __restrict__ recs, int* __restrict__ err, int64_t block)
 {
     using T = Topo<ET>;
     constexpr int D = T::dim, N = T::nsh, NC = D + 1, NIP = T::nip;
     // wavefront w takes SCVF w % count of the 64 elements block w / count:
     // consecutive wavefronts share their elements' data in L2
     constexpr int CNT = IpsOfQ<ET, Q>::count;
-    const int64_t L = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t L = block * 256 + threadIdx.x;
     const int64_t wave = L >> 6;
     const int idx = (int)(wave % CNT);
     const int64_t e = (wave / CNT) * 64 + (L & 63);
@@ -1106,6 +1108,32 @@ scvf_records(KMeshPtrs M, KParams P, const double* __restrict__ u, const double*
                             affine);
     if (!oku) kernel_error(err, KERR_CUT_SIDE);
     if (!okg) kernel_error(err, KERR_DEGENERATE);
+}
+
+template <int ET, int Q>
+__host__ __device__ constexpr int64_t records_blocks(int64_t ne_pad)
+{
+    return (IpsOfQ<ET, Q>::count * ne_pad + 255) / 256;
+}
+
+// the workgroups of frame index Q = 0, then 1, then 2 (one launch: they run
+// side by side; LPS, 56^3 cells 283 -> 215 us, a mesh of one workgroup 29 -> 10 us)
+template <int ET, int FAST>
+__global__ void __launch_bounds__(256, 2)
+scvf_records(KMeshPtrs M, KParams P, const double* __restrict__ u, const double* __restrict__ uold, int64_t ne,
+             int64_t ne_pad, float* __restrict__ recs, int* __restrict__ err)
+{
+    int64_t b = blockIdx.x;
+    if constexpr (IpsOfQ<ET, 0>::count > 0) {
+        if (b < records_blocks<ET, 0>(ne_pad)) return records_block<ET, FAST, 0>(M, P, u, uold, ne, ne_pad, recs, err, b);
+        b -= records_blocks<ET, 0>(ne_pad);
+    }
+    if constexpr (IpsOfQ<ET, 1>::count > 0) {
+        if (b < records_blocks<ET, 1>(ne_pad)) return records_block<ET, FAST, 1>(M, P, u, uold, ne, ne_pad, recs, err, b);
+        b -= records_blocks<ET, 1>(ne_pad);
+    }
+    if constexpr (Topo<ET>::cip > 2 && IpsOfQ<ET, 2>::count > 0)
+        records_block<ET, FAST, 2>(M, P, u, uold, ne, ne_pad, recs, err, b);
 }
 
 template <int ET, int FAST, int Q>
@@ -1303,6 +1331,75 @@ assemble_rows_split(KMeshPtrs M, KParams P, const double* __restrict__ u, const 
         for (int i = threadIdx.x; i < dlen; i += blockDim.x) dout[(int64_t)v0 * NC + i] = dbuf[i];
 }
 
+// the row gather of nsfv1_rows.hpp from the SCVF records, in the plan's lane order
+// (by corner slot, then node: the lanes of a wave read records of consecutive
+// elements)
+template <int ET, int FAST>
+__global__ void __launch_bounds__(256)
+split_rows(RowLists LL, KMeshPtrs M, KParams P, const double* __restrict__ u, const float* __restrict__ recs,
+           int64_t ne_pad, float* __restrict__ J, double* __restrict__ dout)
+{
+    using T = Topo<ET>;
+    constexpr int D = T::dim, N = T::nsh, NC = D + 1;
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int w = [] {
+        const int nwg = (int)gridDim.x, i = (int)blockIdx.x;
+        const int per = nwg >> 3, rem = nwg & 7, x = i & 7, k = i >> 3;
+        return x * per + (x < rem ? x : rem) + k;
+    }();
+    const bool wantJ = J != nullptr, vec = ((uintptr_t)J & 15) == 0;
+    OwnedRows<N, NC, float, 1, true> rows(smem, LL, M, w, LL.cap, wantJ);
+    const bool active = (int)threadIdx.x < rows.ni;
+    Lane<ET, float> L;
+#pragma unroll
+    for (int a = 0; a < NC; ++a) {
+        L.dacc[a] = 0.0;
+#pragma unroll
+        for (int k = 0; k < N; ++k)
+#pragma unroll
+            for (int b = 0; b < NC; ++b) L.jacc[a][k][b] = 0.f;
+    }
+    int pk[N];
+#pragma unroll
+    for (int k = 0; k < N; ++k) pk[k] = k;
+    if (active) {
+        const int4 la = M.lane_a[rows.i0 + (int)threadIdx.x];
+        const int e = la.x, v = la.y, kv = la.z & 0xff;
+#pragma unroll
+        for (int k = 0; k < N; ++k) pk[k] = CanonH<ET>::c.perm[kv][k];
+        if (P.parts & 1) {
+            const Cfg<FAST> C{P, M.nu_elem ? M.nu_elem[e] : P.nu};
+            gather_jac<ET, FAST, 0>(C, recs, ne_pad, e, kv, pk, L, wantJ);
+        }
+        if (P.parts & 6) {
+            const double volk = M.vol[(int64_t)e * N + kv];
+            if (P.parts & 2) {
+                const double m = volk * P.rho;
+#pragma unroll
+                for (int d = 0; d < D; ++d) {
+                    if (wantJ) L.jacc[d][0][d] += float(P.s_m * m);
+                    L.dacc[d] += P.s_m * (u[(int64_t)v * NC + d] * m);
+                }
+            }
+            if ((P.parts & 4) && P.has_source)
+#pragma unroll
+                for (int d = 0; d < D; ++d) {
+                    const double fk = M.f_scv ? M.f_scv[((int64_t)e * N + kv) * D + d] : P.f[d];
+                    L.dacc[d] += P.s_f * (fk * volk * P.rho);
+                }
+        }
+    }
+    if (wantJ) {
+#pragma unroll
+        for (int r = 0; r < NC; ++r) {
+#pragma unroll
+            for (int k = 0; k < N; ++k) rows.put(pk[k], 0, L.jacc[r][k]);
+            rows.sum(LL, M, r, 1, J, vec);
+        }
+    }
+    if (dout) rows.defect(L.dacc, active, dout);
+}
+
 // ---------------------------------------------------------------------
 // host launchers
 // ---------------------------------------------------------------------
@@ -1314,7 +1411,7 @@ assemble_rows_split(KMeshPtrs M, KParams P, const double* __restrict__ u, const 
 // fit and each keeps all its loads in flight.  The terms and their order
 // of addition per entry are those of scvf_jac for the split configurations
 // (FIELDS, one upwind, no Stokes/PAC/Peclet/exact), so the result is
-// bitwise that of assemble_rows_split.
+// bitwise that of the one-lane gather.
 // ---------------------------------------------------------------------
 template <int ET, int FAST, int Q>
 __device__ inline void row_terms(const Cfg<FAST>& C, const float4* __restrict__ rec, int64_t cs, int kv, const int* pk,
@@ -1591,38 +1688,41 @@ hipError_t launch_assemble(int et, int jprec, const KMeshPtrs& m, const KParams&
 
 // split path: records then row gather (FP32 Jacobian, common configuration)
 template <int ET, int FAST>
-static hipError_t launch_split_cfg(const KMeshPtrs& m, const KParams& p, const double* u, const double* uold,
-                                   float* J, double* d, int* err, int nwg, size_t lds, int64_t ne, float* recs,
+static hipError_t launch_split_cfg(const RowLists& l, const KMeshPtrs& m, const KParams& p, const double* u,
+                                   const double* uold, float* J, double* d, int* err, int nwg, size_t lds, int64_t ne, float* recs,
                                    bool rowlane, hipStream_t s)
 {
     const int64_t ne_pad = (ne + 63) / 64 * 64;
-    if (p.parts & 1) {
-        // one launch per frame index Q that has SCVFs (triangles use Q = 0 only)
-        if constexpr (IpsOfQ<ET, 0>::count > 0)
-            scvf_records<ET, FAST, 0><<<(unsigned)((IpsOfQ<ET, 0>::count * ne_pad + 255) / 256), 256, 0, s>>>(
-                m, p, u, uold, ne, ne_pad, recs, err);
-        if constexpr (IpsOfQ<ET, 1>::count > 0)
-            scvf_records<ET, FAST, 1><<<(unsigned)((IpsOfQ<ET, 1>::count * ne_pad + 255) / 256), 256, 0, s>>>(
-                m, p, u, uold, ne, ne_pad, recs, err);
-        if constexpr (Topo<ET>::cip > 2 && IpsOfQ<ET, 2>::count > 0)
-            scvf_records<ET, FAST, 2><<<(unsigned)((IpsOfQ<ET, 2>::count * ne_pad + 255) / 256), 256, 0, s>>>(
-                m, p, u, uold, ne, ne_pad, recs, err);
+    if ((p.parts & 1) && ne > 0) {
+        const int64_t nb = records_blocks<ET, 0>(ne_pad) + records_blocks<ET, 1>(ne_pad) +
+                           (Topo<ET>::cip > 2 ? records_blocks<ET, 2>(ne_pad) : 0);
+        scvf_records<ET, FAST><<<(unsigned)nb, 256, 0, s>>>(m, p, u, uold, ne, ne_pad, recs, err);
     }
-    if (rowlane) assemble_rows_rowlane<ET, FAST><<<nwg, 64, lds, s>>>(m, p, u, recs, ne_pad, J, d);
-    else assemble_rows_split<ET, FAST><<<nwg, m.block, lds, s>>>(m, p, u, recs, ne_pad, J, d);
+    if (rowlane) {
+        assemble_rows_rowlane<ET, FAST><<<nwg, 64, lds, s>>>(m, p, u, recs, ne_pad, J, d);
+    } else if constexpr (ET == ET_QUAD) {
+        assemble_rows_split<ET, FAST><<<nwg, m.block, lds, s>>>(m, p, u, recs, ne_pad, J, d);
+    } else if constexpr (ET == ET_HEX) {
+        using Rows = OwnedRows<Topo<ET>::nsh, Topo<ET>::dim + 1, float, 1, true>;
+        RowLists lr = l;
+        lr.cap = Rows::out_cap(l.cap);
+        split_rows<ET, FAST><<<nwg, m.block, Rows::BASE + Rows::out_bytes(lr.cap), s>>>(lr, m, p, u, recs, ne_pad, J, d);
+    } else {
+        return hipErrorInvalidValue;  // simplices have element records
+    }
     return hipGetLastError();
 }
 
 template <int ET>
-static hipError_t launch_split_et(const KMeshPtrs& m, const KParams& p, const double* u, const double* uold, float* J,
-                                  double* d, int* err, int nwg, size_t lds, int64_t ne, float* recs, bool rl,
+static hipError_t launch_split_et(const RowLists& l, const KMeshPtrs& m, const KParams& p, const double* u,
+                                  const double* uold, float* J, double* d, int* err, int nwg, size_t lds, int64_t ne, float* recs, bool rl,
                                   hipStream_t s)
 {
     switch (fast_path(p)) {
-    case UPW_NO: return launch_split_cfg<ET, UPW_NO>(m, p, u, uold, J, d, err, nwg, lds, ne, recs, rl, s);
-    case UPW_FULL: return launch_split_cfg<ET, UPW_FULL>(m, p, u, uold, J, d, err, nwg, lds, ne, recs, rl, s);
-    case UPW_SKEWED: return launch_split_cfg<ET, UPW_SKEWED>(m, p, u, uold, J, d, err, nwg, lds, ne, recs, rl, s);
-    case UPW_LPS: return launch_split_cfg<ET, UPW_LPS>(m, p, u, uold, J, d, err, nwg, lds, ne, recs, rl, s);
+    case UPW_NO: return launch_split_cfg<ET, UPW_NO>(l, m, p, u, uold, J, d, err, nwg, lds, ne, recs, rl, s);
+    case UPW_FULL: return launch_split_cfg<ET, UPW_FULL>(l, m, p, u, uold, J, d, err, nwg, lds, ne, recs, rl, s);
+    case UPW_SKEWED: return launch_split_cfg<ET, UPW_SKEWED>(l, m, p, u, uold, J, d, err, nwg, lds, ne, recs, rl, s);
+    case UPW_LPS: return launch_split_cfg<ET, UPW_LPS>(l, m, p, u, uold, J, d, err, nwg, lds, ne, recs, rl, s);
     }
     return hipErrorInvalidValue;
 }
@@ -1641,17 +1741,17 @@ int64_t split_record_floats(int et, int64_t ne)
     return (int64_t)nip * ((ne + 63) / 64 * 64) * REC_FLOATS;
 }
 
-hipError_t launch_assemble_split(int et, const KMeshPtrs& m, const KParams& p, const double* u, const double* uold,
-                                 float* J, double* d, int* err, int nwg, size_t lds, int64_t ne, float* recs,
-                                 bool rowlane, hipStream_t s)
+hipError_t launch_assemble_split(int et, const RowLists& l, const KMeshPtrs& m, const KParams& p, const double* u,
+                                 const double* uold, float* J, double* d, int* err, int nwg, size_t lds, int64_t ne,
+                                 float* recs, bool rowlane, hipStream_t s)
 {
     if (lds > 65536 || m.block < 64 || m.block > 256 || m.block % 64 || !split_supported(et, p)) return hipErrorInvalidValue;
     if (rowlane && m.block != 64) return hipErrorInvalidValue;
     switch (et) {
-    case ET_TRI:  return launch_split_et<ET_TRI>(m, p, u, uold, J, d, err, nwg, lds, ne, recs, rowlane, s);
-    case ET_QUAD: return launch_split_et<ET_QUAD>(m, p, u, uold, J, d, err, nwg, lds, ne, recs, rowlane, s);
-    case ET_TET:  return launch_split_et<ET_TET>(m, p, u, uold, J, d, err, nwg, lds, ne, recs, rowlane, s);
-    case ET_HEX:  return launch_split_et<ET_HEX>(m, p, u, uold, J, d, err, nwg, lds, ne, recs, rowlane, s);
+    case ET_TRI:  return launch_split_et<ET_TRI>(l, m, p, u, uold, J, d, err, nwg, lds, ne, recs, rowlane, s);
+    case ET_QUAD: return launch_split_et<ET_QUAD>(l, m, p, u, uold, J, d, err, nwg, lds, ne, recs, rowlane, s);
+    case ET_TET:  return launch_split_et<ET_TET>(l, m, p, u, uold, J, d, err, nwg, lds, ne, recs, rowlane, s);
+    case ET_HEX:  return launch_split_et<ET_HEX>(l, m, p, u, uold, J, d, err, nwg, lds, ne, recs, rowlane, s);
     }
     return hipErrorInvalidValue;
 }

@@ -43,28 +43,35 @@ hipError_t launch_assemble(int et, int jprec, const KMeshPtrs& m, const KParams&
                            const double* uold, void* J, double* d, int* err, int nwg, size_t lds_bytes,
                            hipStream_t stream);
 
+// lists of a row gather that sums its blocks by owners (nsfv1_rows.hpp)
+struct RowLists {
+    const uint2* own;        // [nblk] blocks of each workgroup, most items first: first item | items << 12 | blocks
+                             // of the node << 23, (first block of the node NC + slot) | block << 16, both from the
+                             // workgroup's first
+    const uint16_t* items;   // [nsh ninc] lane << 3 | corner, sorted by block, then element
+    const uint8_t* lane_of;  // [ninc] lane of the incidence
+    const int32_t* wg_node;  // [nwg + 1] first node of each workgroup (at most 255 nodes, 256 incidences)
+    int cap;                 // most blocks of a workgroup
+};
+// perm: lane order of the incidences of a workgroup (null: their own)
+hipError_t launch_row_lists(int et, const KMeshPtrs& m, const int32_t* wg_node, const int32_t* perm, int nwg, uint2* own,
+                            uint16_t* items, uint8_t* lane_of, hipStream_t stream);
+
 // split path (FP32 Jacobian, common configuration): per-SCVF records, then
 // the row gather; recs holds split_record_floats(et, ne) floats
 bool split_supported(int et, const KParams& p);
 int64_t split_record_floats(int et, int64_t ne);
 // rowlane: one lane per (node, element, row) in the gather (plan with
 // 64 / (dim+1) incidences per 64-lane workgroup)
-hipError_t launch_assemble_split(int et, const KMeshPtrs& m, const KParams& p, const double* u, const double* uold,
-                                 float* J, double* d, int* err, int nwg, size_t lds, int64_t ne, float* recs,
-                                 bool rowlane, hipStream_t stream);
+hipError_t launch_assemble_split(int et, const RowLists& l, const KMeshPtrs& m, const KParams& p, const double* u,
+                                 const double* uold, float* J, double* d, int* err, int nwg, size_t lds, int64_t ne,
+                                 float* recs, bool rowlane, hipStream_t stream);
 
 // simplex path (nsfv1_simplex.hip; same configurations as the split path):
-// block lists of a mesh, and the assembly from element records
-struct SxLists {
-    uint32_t* blk;          // [nblk] slot | first item << 8 | items << 18 of each (node, neighbour) block
-    int32_t* blk_node;      // [nblk] node of the block
-    uint16_t* items;        // [nsh ninc] incidence of the node << 2 | corner of the neighbour, per node sorted by block
-    const int32_t* wg_node; // [nwg + 1] first node of each workgroup (at most 255 nodes, 256 incidences)
-};
-bool simplex_supported(int et, int jprec, int64_t max_inc);
+// element records, then the row gather
+bool simplex_supported(int et, int jprec);
 int64_t simplex_record_bytes(int et, int jprec, int64_t ne);
-hipError_t launch_simplex_lists(int et, const SxLists& l, const KMeshPtrs& m, int64_t nv, hipStream_t stream);
-hipError_t launch_assemble_simplex(int et, int jprec, const SxLists& l, const KMeshPtrs& m, const KParams& p,
+hipError_t launch_assemble_simplex(int et, int jprec, const RowLists& l, const KMeshPtrs& m, const KParams& p,
                                    const double* u, const double* uold, void* J, double* d, int* err, int64_t ne,
                                    int nwg, void* recs, hipStream_t stream);
 

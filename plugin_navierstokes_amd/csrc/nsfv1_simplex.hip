@@ -27,6 +27,7 @@
 #include "nsfv1_geom.hpp"
 #include "nsfv1_internal.hpp"
 #include "nsfv1_ray.hpp"
+#include "nsfv1_rows.hpp"
 #include "nsfv1_topo.hpp"
 
 namespace nsfv1 {
@@ -378,52 +379,15 @@ simplex_records(KMeshPtrs M, KParams P, const double* __restrict__ u, const doub
         *reinterpret_cast<double2*>(rec + (R::DEF + q) * 8) = make_double2(f[2 * q], f[2 * q + 1]);
 }
 
-// NC values of a row segment, in 16-byte pieces where there are four
-template <int NC, typename VT>
-__device__ __forceinline__ void sx_seg_put(VT* p, const VT (&x)[NC])
-{
-    if constexpr (NC == 4 && sizeof(VT) == 4) {
-        *reinterpret_cast<float4*>(p) = make_float4(x[0], x[1], x[2], x[3]);
-    } else if constexpr (NC == 4) {
-        reinterpret_cast<double2*>(p)[0] = make_double2(x[0], x[1]);
-        reinterpret_cast<double2*>(p)[1] = make_double2(x[2], x[3]);
-    } else {
-#pragma unroll
-        for (int c = 0; c < NC; ++c) p[c] = x[c];
-    }
-}
-template <int NC, typename VT>
-__device__ __forceinline__ void sx_seg_get(const VT* p, VT (&x)[NC])
-{
-    if constexpr (NC == 4 && sizeof(VT) == 4) {
-        const float4 t = *reinterpret_cast<const float4*>(p);
-        x[0] = t.x;
-        x[1] = t.y;
-        x[2] = t.z;
-        x[3] = t.w;
-    } else if constexpr (NC == 4) {
-        const double2 a = reinterpret_cast<const double2*>(p)[0], b = reinterpret_cast<const double2*>(p)[1];
-        x[0] = a.x;
-        x[1] = a.y;
-        x[2] = b.x;
-        x[3] = b.y;
-    } else {
-#pragma unroll
-        for (int c = 0; c < NC; ++c) x[c] = p[c];
-    }
-}
-
 // rows per pass: 32 KB of segments for 256 lanes, so four workgroups fit a CU
 template <typename VT>
 constexpr int SX_RP = sizeof(VT) == 4 ? 2 : 1;
 
-// Row gather.  Block b of the pattern (node v, neighbour slot) is described by
-// L.blk[b] = slot | first item << 8 | items << 18, the item positions relative
-// to the node's, and L.items = incidence of the node << 2 | corner of the
-// neighbour in that element, sorted by block, then element.
+// the row gather of nsfv1_rows.hpp from the element records, lanes in the order of
+// the nodes' incidences
 template <int ET, typename VT>
 __global__ void __launch_bounds__(256)
-simplex_rows(SxLists L, KMeshPtrs M, KParams P, const double* __restrict__ u, const float4* __restrict__ recs,
+simplex_rows(RowLists L, KMeshPtrs M, KParams P, const double* __restrict__ u, const float4* __restrict__ recs,
              VT* __restrict__ J, double* __restrict__ dout)
 {
     using T = Topo<ET>;
@@ -431,31 +395,17 @@ simplex_rows(SxLists L, KMeshPtrs M, KParams P, const double* __restrict__ u, co
     using C = SxCorner<ET>;
     constexpr int D = T::dim, N = T::nsh, NC = D + 1;
     constexpr int RP = SX_RP<VT>;
-    constexpr int NB = 256;                     // lanes of the LDS layout
     extern __shared__ __align__(16) unsigned char smem[];
-    // [corner][row of the pass][lane] row segments; the node table; the items
-    VT* seg = reinterpret_cast<VT*>(smem);                                        // N * RP * NB * NC
-    int* ntab = reinterpret_cast<int*>(smem + sizeof(VT) * N * RP * NB * NC);     // per node: first lane, first block
-    uint16_t* sit = reinterpret_cast<uint16_t*>(ntab + 2 * (NB + 1));      // items of the workgroup: N * NB
-    double* dseg = reinterpret_cast<double*>(smem);                        // defects [component][lane], after the passes
     // consecutive workgroups (shared element data) go to the same XCD
     const int w = [] {
         const int nwg = (int)gridDim.x, i = (int)blockIdx.x;
         const int per = nwg >> 3, rem = nwg & 7, x = i & 7, k = i >> 3;
         return x * per + (x < rem ? x : rem) + k;
     }();
-    const int v0 = L.wg_node[w], v1 = L.wg_node[w + 1], nn = v1 - v0;
-    const int t = threadIdx.x, nt = (int)blockDim.x;
-    const int i0 = M.node_inc[v0], i1 = M.node_inc[v1];
     const bool wantJ = J != nullptr, vec = ((uintptr_t)J & 15) == 0;
-    if (t <= nn) {
-        ntab[2 * t] = M.node_inc[v0 + t] - i0;
-        ntab[2 * t + 1] = (int)(M.rowptr[(int64_t)(v0 + t) * NC] / (NC * NC));
-    }
-    if (wantJ)
-        for (int i = t; i < N * (i1 - i0); i += nt) sit[i] = L.items[(int64_t)N * i0 + i];
-    const int inc = i0 + t;
-    const bool active = inc < i1;
+    OwnedRows<N, NC, VT, RP, false> rows(smem, L, M, w, 0, wantJ);
+    const int inc = rows.i0 + (int)threadIdx.x;
+    const bool active = (int)threadIdx.x < rows.ni;
     VT B[N][NC][NC];
     double dl[NC];
 #pragma unroll
@@ -562,111 +512,18 @@ simplex_rows(SxLists L, KMeshPtrs M, KParams P, const double* __restrict__ u, co
                 for (int a = 0; a < D; ++a) dl[a] += P.s_f * (P.f[a] * vol * P.rho);
         }
     }
-    const int b0 = (int)(M.rowptr[(int64_t)v0 * NC] / (NC * NC)), b1 = (int)(M.rowptr[(int64_t)v1 * NC] / (NC * NC));
     if (wantJ) {
 #pragma unroll
         for (int r0 = 0; r0 < NC; r0 += RP) {
-            const int nr = NC - r0 < RP ? NC - r0 : RP;
 #pragma unroll
             for (int k = 0; k < N; ++k)
 #pragma unroll
                 for (int r = 0; r < RP; ++r)
-                    if (r0 + r < NC) sx_seg_put<NC>(seg + ((k * RP + r) * NB + t) * NC, B[k][r0 + r < NC ? r0 + r : 0]);
-            __syncthreads();
-            // one lane per (block, row): rows of a block side by side
-            for (int x = t; x < (b1 - b0) * RP; x += nt) {
-                const int b = b0 + x / RP, r = x % RP;
-                if (r >= nr) continue;
-                const int v = L.blk_node[b] - v0;
-                const uint32_t info = L.blk[b];
-                const int slot = info & 0xff, first = (info >> 8) & 0x3ff, cnt = info >> 18;
-                const int lane0 = ntab[2 * v];
-                const uint16_t* it = sit + N * lane0 + first;
-                VT s[NC], y[NC];
-#pragma unroll
-                for (int c = 0; c < NC; ++c) s[c] = VT(0);
-#pragma unroll 4
-                for (int i = 0; i < cnt; ++i) {
-                    const int z = it[i];
-                    sx_seg_get<NC>(seg + (((z & 3) * RP + r) * NB + lane0 + (z >> 2)) * NC, y);
-#pragma unroll
-                    for (int c = 0; c < NC; ++c) s[c] += y[c];
-                }
-                const int bv = ntab[2 * v + 1], nb = ntab[2 * v + 3] - bv;
-                VT* dst = J + (int64_t)bv * (NC * NC) + (int64_t)(r0 + r) * (nb * NC) + slot * NC;
-                if (vec) {
-                    sx_seg_put<NC>(dst, s);
-                } else {
-#pragma unroll
-                    for (int c = 0; c < NC; ++c) dst[c] = s[c];
-                }
-            }
-            __syncthreads();
+                    if (r0 + r < NC) rows.put(k, r, B[k][r0 + r < NC ? r0 + r : 0]);
+            rows.sum(L, M, r0, NC - r0 < RP ? NC - r0 : RP, J, vec);
         }
     }
-    if (!dout) return;
-    if (active)
-#pragma unroll
-        for (int a = 0; a < NC; ++a) dseg[a * NB + t] = dl[a];
-    __syncthreads();
-    for (int x = t; x < nn * NC; x += nt) {
-        const int v = x / NC, a = x % NC;
-        double s = 0.0;
-#pragma unroll 4
-        for (int i = ntab[2 * v]; i < ntab[2 * v + 2]; ++i) s += dseg[a * NB + i];
-        dout[(int64_t)v0 * NC + x] = s;
-    }
-}
-
-template <int ET, typename VT>
-constexpr size_t sx_lds()
-{
-    constexpr int N = Topo<ET>::nsh, NC = Topo<ET>::dim + 1;
-    return sizeof(VT) * N * SX_RP<VT> * 256 * NC + sizeof(int) * 2 * 257 + sizeof(uint16_t) * N * 256;
-}
-
-// the lists of a mesh (once per plan)
-template <int ET>
-__global__ void __launch_bounds__(256)
-simplex_lists(SxLists L, KMeshPtrs M, int64_t nv)
-{
-    constexpr int N = Topo<ET>::nsh, NC = Topo<ET>::dim + 1;
-    const int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= nv) return;
-    const int64_t r0 = M.rowptr[v * NC];
-    const int nb = (int)((M.rowptr[v * NC + 1] - r0) / NC);
-    const int64_t b0 = r0 / (NC * NC);
-    const int i0 = M.node_inc[v], i1 = M.node_inc[v + 1];
-    // items per block, then the blocks' first items, then the items
-    for (int s = 0; s < nb; ++s) {
-        L.blk[b0 + s] = 0;
-        L.blk_node[b0 + s] = (int)v;
-    }
-    for (int i = i0; i < i1; ++i) {
-        const uint64_t pos = M.inc_pos[i];
-#pragma unroll
-        for (int k = 0; k < N; ++k) L.blk[b0 + ((pos >> (8 * k)) & 0xff)] += 1u << 18;
-    }
-    uint32_t at = 0;
-    for (int s = 0; s < nb; ++s) {
-        const uint32_t c = L.blk[b0 + s];
-        L.blk[b0 + s] = c | at << 8;
-        at += c >> 18;
-    }
-    for (int i = i0; i < i1; ++i) {
-        const uint64_t pos = M.inc_pos[i];
-#pragma unroll
-        for (int k = 0; k < N; ++k) {
-            uint32_t* b = &L.blk[b0 + ((pos >> (8 * k)) & 0xff)];
-            L.items[(int64_t)N * i0 + ((*b >> 8) & 0x3ff)] = (uint16_t)((i - i0) << 2 | k);
-            *b += 1u << 8;
-        }
-    }
-    // the first items were advanced past the block: back by the count
-    for (int s = 0; s < nb; ++s) {
-        const uint32_t b = L.blk[b0 + s];
-        L.blk[b0 + s] = (b - ((b >> 18) << 8)) | (uint32_t)s;
-    }
+    if (dout) rows.defect(dl, active, dout);
 }
 
 // ---------------------------------------------------------------------
@@ -675,11 +532,7 @@ simplex_lists(SxLists L, KMeshPtrs M, int64_t nv)
 // Triangles with FP64 Jacobian stay on the fused kernel: 300 x 300 cells 39 (full
 // upwind) and 62 us (LPS) against 54 and 55 us; tetrahedra 200 against 80 us (22^3
 // cells, LPS) and 42 against 33 us (6^3)
-bool simplex_supported(int et, int jprec, int64_t max_inc)
-{
-    // list fields: 10 bits for a node's items, so at most 255 incidences a node
-    return ((et == ET_TRI && jprec == 32) || et == ET_TET) && max_inc <= 255;
-}
+bool simplex_supported(int et, int jprec) { return (et == ET_TRI && jprec == 32) || et == ET_TET; }
 
 int64_t simplex_record_bytes(int et, int jprec, int64_t ne)
 {
@@ -688,18 +541,8 @@ int64_t simplex_record_bytes(int et, int jprec, int64_t ne)
     return (ne + 7) / 8 * 8 * chunks * 16;
 }
 
-hipError_t launch_simplex_lists(int et, const SxLists& l, const KMeshPtrs& m, int64_t nv, hipStream_t s)
-{
-    const unsigned g = (unsigned)((nv + 255) / 256);
-    if (nv <= 0) return hipSuccess;
-    if (et == ET_TRI) simplex_lists<ET_TRI><<<g, 256, 0, s>>>(l, m, nv);
-    else if (et == ET_TET) simplex_lists<ET_TET><<<g, 256, 0, s>>>(l, m, nv);
-    else return hipErrorInvalidValue;
-    return hipGetLastError();
-}
-
 template <int ET, typename VT>
-static hipError_t launch_simplex_et(const SxLists& l, const KMeshPtrs& m, const KParams& p, const double* u,
+static hipError_t launch_simplex_et(const RowLists& l, const KMeshPtrs& m, const KParams& p, const double* u,
                                     const double* uold, void* J, double* d, int* err, int64_t ne, int nwg,
                                     float4* recs, hipStream_t s)
 {
@@ -714,13 +557,13 @@ static hipError_t launch_simplex_et(const SxLists& l, const KMeshPtrs& m, const 
         default: return hipErrorInvalidValue;
         }
     }
-    static_assert(sx_lds<ET, VT>() <= 64 * 1024, "dynamic LDS limit");
-    if (nwg > 0)
-        simplex_rows<ET, VT><<<nwg, 256, sx_lds<ET, VT>(), s>>>(l, m, p, u, recs, static_cast<VT*>(J), d);
+    using Rows = OwnedRows<Topo<ET>::nsh, Topo<ET>::dim + 1, VT, SX_RP<VT>, false>;
+    static_assert(Rows::BASE <= 64 * 1024, "dynamic LDS limit");
+    if (nwg > 0) simplex_rows<ET, VT><<<nwg, 256, Rows::BASE, s>>>(l, m, p, u, recs, static_cast<VT*>(J), d);
     return hipGetLastError();
 }
 
-hipError_t launch_assemble_simplex(int et, int jprec, const SxLists& l, const KMeshPtrs& m, const KParams& p,
+hipError_t launch_assemble_simplex(int et, int jprec, const RowLists& l, const KMeshPtrs& m, const KParams& p,
                                    const double* u, const double* uold, void* J, double* d, int* err, int64_t ne,
                                    int nwg, void* recs, hipStream_t s)
 {
