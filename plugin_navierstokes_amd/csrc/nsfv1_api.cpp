@@ -79,6 +79,7 @@ struct Plan {
     // column blocks of the corners; wg_a[2w] = {v0, v1, i0, i1},
     // wg_a[2w+1] = {jbase low, jbase high, jlen, rounds}
     DevBuf lane_a, lane_pos, wg_a;
+    DevBuf lane_conn;  // 2D: the nodes of each lane's element
     bool rowlane = false;  // built for the row-lane split gather
     // lists of the gathers that sum by owners (rnwg = 0: none), and simplices'
     // own workgroups
@@ -1141,6 +1142,16 @@ static int make_row_lists(nsfv1_handle* h, int jprec, Plan& P)
     return NSFV1_OK;
 }
 
+static int make_lane_nodes(nsfv1_handle* h, int et, const DevBuf& conn, int64_t ninc, Plan& P)
+{
+    if (h->dim != 2) return NSFV1_OK;
+    if (P.lane_conn.alloc(sizeof(int4) * std::max<int64_t>(ninc, 1)) != hipSuccess ||
+        launch_lane_nodes(et, P.lane_a.as<int4>(), conn.as<int32_t>(), ninc, P.lane_conn.as<int4>(), nullptr) != hipSuccess ||
+        hipStreamSynchronize(nullptr) != hipSuccess)
+        return fail(NSFV1_ERR_DEVICE, "plan nodes");
+    return NSFV1_OK;
+}
+
 // FP64 element records of the stream (null: none to be had)
 static void* stream_records(nsfv1_handle* h, void* stream, size_t need)
 {
@@ -1253,6 +1264,7 @@ static int assemble_impl(nsfv1_handle* h, const double* u, const double* u_old, 
                                             "needs one nsfv1_assemble call with the same jprec first (it builds the plan)");
         int rc = make_plan(h, IncView{h->h_node_inc, h->h_inc_info, h->h_inc_elem, h->ninc, h->inc_pos},
                            jprec == NSFV1_F64 ? 8 : 4, P);
+        if (!rc) rc = make_lane_nodes(h, h->et, h->conn, h->ninc, P);
         if (!rc) rc = make_row_lists(h, jprec, P);
         if (rc) P.valid = false;
         if (rc) return rc;
@@ -1266,6 +1278,8 @@ static int assemble_impl(nsfv1_handle* h, const double* u, const double* u_old, 
                                             "needs one nsfv1_assemble call with the same jprec first (it builds the plan)");
         int rc = make_plan(h, IncView{G.h_node_inc, G.h_inc_info, G.h_inc_elem, G.ninc, G.inc_pos},
                            jprec == NSFV1_F64 ? 8 : 4, PG);
+        if (!rc) rc = make_lane_nodes(h, G.et, G.conn, G.ninc, PG);
+        if (rc) PG.valid = false;
         if (rc) return rc;
     }
     KParams k{};
@@ -1388,7 +1402,7 @@ static int assemble_impl(nsfv1_handle* h, const double* u, const double* u_old, 
         auto launch = [&](int et, const KMeshPtrs& mm, const KParams& kk, const Plan& PP, int64_t ne) {
             return cpl ? launch_assemble_coupled(et, jprec, mm, kk, u, u_old, jvals, defect, h->errflag.as<int>(), PP.nwg,
                                                  PP.lds, ne, crecs, nullptr, (hipStream_t)stream)
-                       : launch_assemble(et, jprec, mm, kk, u, u_old, jvals, defect, h->errflag.as<int>(), PP.nwg, PP.lds,
+                       : launch_assemble(et, jprec, mm, PP.lane_conn.as<int4>(), kk, u, u_old, jvals, defect, h->errflag.as<int>(), PP.nwg, PP.lds,
                                          (hipStream_t)stream);
         };
         // J and d start from zero; the first group writes the rows of its
@@ -1488,7 +1502,7 @@ static int assemble_impl(nsfv1_handle* h, const double* u, const double* u_old, 
                                   P.lds, h->ne, recs, h->path == 2 && P.rowlane, (hipStream_t)stream);
         h->last_path = (h->path == 2 && P.rowlane) ? 2 : 0;
     } else {
-        e = launch_assemble(h->et, jprec, m, k, u, u_old, jvals, defect, h->errflag.as<int>(), P.nwg, P.lds,
+        e = launch_assemble(h->et, jprec, m, P.lane_conn.as<int4>(), k, u, u_old, jvals, defect, h->errflag.as<int>(), P.nwg, P.lds,
                             (hipStream_t)stream);
         h->last_path = 1;
     }

@@ -908,6 +908,145 @@ assemble_rows(KMeshPtrs M, KParams P, const double* __restrict__ u, const double
 }
 
 
+// 2D meshes: the same kernel with the plan's data packed, one load for the
+// workgroup and one round of loads for the lane, its nodes included, before
+// those of the nodes.  A mesh of a few workgroups waits for that chain of loads,
+// which was seven long, a large one re-reads less: FP64, 64^2 quads full upwind
+// 11.3 -> 10.4 us, 512^2 x 2 triangles LPS 189 -> 164 us.
+template <int ET, typename JT, int FAST>
+__global__ void __launch_bounds__(256)
+assemble_rows_2d(KMeshPtrs M, const int4* __restrict__ lane_conn, KParams P, const double* __restrict__ u,
+                 const double* __restrict__ uold, JT* __restrict__ J, double* __restrict__ dout,
+                 int* __restrict__ err)
+{
+    using T = Topo<ET>;
+    constexpr int D = T::dim, N = T::nsh, NC = D + 1, NIP = T::nip;
+    extern __shared__ __align__(16) unsigned char smem[];
+
+    const int w = [] {
+        const int nwg = (int)gridDim.x, i = (int)blockIdx.x;
+        const int per = nwg >> 3, rem = nwg & 7, x = i & 7, k = i >> 3;
+        return x * per + (x < rem ? x : rem) + k;
+    }();
+    const int4 wa = M.wg_a[2 * w], wb = M.wg_a[2 * w + 1];
+    const int v0 = wa.x, v1 = wa.y, i0 = wa.z, i1 = wa.w, jlen = wb.z, rounds = wb.w;
+    const int64_t jbase = (int64_t)(uint32_t)wb.x | ((int64_t)wb.y << 32);
+    const int dlen = (v1 - v0) * NC;
+    JT* jbuf = reinterpret_cast<JT*>(smem);
+    double* dbuf = reinterpret_cast<double*>(smem + ((jlen * (int)sizeof(JT) + 15) & ~15));
+    const bool wantJ = J != nullptr;
+    if (P.accum && i0 == i1) return;
+    if (P.accum == 1) {
+        if (wantJ)
+            for (int i = threadIdx.x; i < jlen; i += blockDim.x) jbuf[i] = J[jbase + i];
+        for (int i = threadIdx.x; i < dlen; i += blockDim.x) dbuf[i] = dout ? dout[(int64_t)v0 * NC + i] : 0.0;
+    } else {
+        if (wantJ)
+            for (int i = threadIdx.x; i < jlen; i += blockDim.x) jbuf[i] = JT(0);
+        for (int i = threadIdx.x; i < dlen; i += blockDim.x) dbuf[i] = 0.0;
+    }
+
+    const int lane_inc = i0 + (int)threadIdx.x;
+    const bool active = lane_inc < i1;
+
+    Lane<ET, JT> L;
+#pragma unroll
+    for (int a = 0; a < NC; ++a) {
+        L.dacc[a] = 0.0;
+#pragma unroll
+        for (int k = 0; k < N; ++k)
+#pragma unroll
+            for (int b = 0; b < NC; ++b) L.jacc[a][k][b] = JT(0);
+    }
+    int v = v0, slot = -1, rbase = 0, rlen = 0;
+    int pos[N];
+#pragma unroll
+    for (int k = 0; k < N; ++k) pos[k] = 0;
+    if (active) {
+        const int4 la = M.lane_a[lane_inc], lc = lane_conn[lane_inc];
+        const uint64_t pw = M.lane_pos[lane_inc];
+        const int e = la.x, kv = la.z & 0xff;
+        const int32_t cn[4] = {lc.x, lc.y, lc.z, lc.w};
+        v = la.y;
+        slot = (la.z >> 8) & 0xff;
+        rlen = la.z >> 16;
+        rbase = la.w;
+        int pk[N];
+        int32_t ccn[N];
+        double co[N][D], ul[N][NC];
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+            pk[k] = CanonH<ET>::c.perm[kv][k];
+            ccn[k] = cn[k];
+#pragma unroll
+            for (int i = 0; i < D; ++i) co[k][i] = M.xyz[(int64_t)ccn[k] * D + i];
+#pragma unroll
+            for (int a = 0; a < NC; ++a) ul[k][a] = u[(int64_t)ccn[k] * NC + a];
+        }
+        bool okg = true, oku = true;
+        if (P.parts & 1) {
+            double c[D];
+            elem_centre<ET>(co, c);
+            Rec<ET, JT> R[T::cip];
+            const Cfg<FAST> C{P, M.nu_elem ? M.nu_elem[e] : P.nu, M.nu_ip ? M.nu_ip + (int64_t)e * NIP : nullptr,
+                              M.f_scvf ? M.f_scvf + (int64_t)e * NIP * D : nullptr,
+                              M.rho_ip ? M.rho_ip + (int64_t)e * NIP : nullptr};
+            scvf_all<ET, FAST, 0, JT>(C, co, M.xyz, M.conn + (int64_t)e * N, ul, pk, ccn, c, uold, M.l2inv + (int64_t)e * NIP,
+                                      (P.upw_mode != 0 && M.upw_dec) ? M.upw_dec + (int64_t)e * NIP : nullptr, kv, wantJ, L, R,
+                                      okg, oku, (ET == 0 || ET == 2) || (M.affine != nullptr && M.affine[e] != 0));
+            if (wantJ) jac_all<ET, FAST, 0, JT>(C, R, L, kv);
+        }
+        // mass part and source: navier_stokes_fv1.cpp:781-869
+        if (P.parts & 6) {
+            const double volk = M.vol[(int64_t)e * N + kv];
+            const double rk = M.rho_scv ? M.rho_scv[(int64_t)e * N + kv] : P.rho;  // density at the SCV ip
+            if (P.parts & 2) {
+                const double m = volk * rk;
+#pragma unroll
+                for (int d = 0; d < D; ++d) {
+                    if (wantJ) L.jacc[d][0][d] += JT(P.s_m * m);
+                    L.dacc[d] += P.s_m * (ul[0][d] * m);
+                }
+            }
+            if ((P.parts & 4) && P.has_source)
+#pragma unroll
+                for (int d = 0; d < D; ++d) {
+                    const double fk = M.f_scv ? M.f_scv[((int64_t)e * N + kv) * D + d] : P.f[d];
+                    L.dacc[d] += P.s_f * (fk * volk * rk);
+                }
+        }
+        if (!oku) kernel_error(err, KERR_CUT_SIDE);
+        if (!okg) kernel_error(err, KERR_DEGENERATE);
+        // column slots of the (canonically ordered) corners in v's block row
+#pragma unroll
+        for (int k = 0; k < N; ++k) pos[k] = (int)((pw >> (8 * pk[k])) & 0xffu) * NC;
+    }
+    __syncthreads();
+
+    // ordered accumulation: round r adds the incidences of slot r
+    for (int r = 0; r < rounds; ++r) {
+        if (active && slot == r) {
+            if (wantJ) {
+#pragma unroll
+                for (int a = 0; a < NC; ++a) {
+                    const int ra = rbase + a * rlen;
+#pragma unroll
+                    for (int k = 0; k < N; ++k) lds_add_block<NC>(jbuf + ra + pos[k], L.jacc[a][k]);
+                }
+            }
+#pragma unroll
+            for (int a = 0; a < NC; ++a) dbuf[(v - v0) * NC + a] += L.dacc[a];
+        }
+        __syncthreads();
+    }
+
+    if (wantJ)
+        for (int i = threadIdx.x; i < jlen; i += blockDim.x) J[jbase + i] = jbuf[i];
+    if (dout)
+        for (int i = threadIdx.x; i < dlen; i += blockDim.x) dout[(int64_t)v0 * NC + i] = dbuf[i];
+}
+
+
 // ---------------------------------------------------------------------
 // Split path (FP32 Jacobian, common configuration): every SCVF is
 // evaluated once.
@@ -1640,16 +1779,26 @@ assemble_rows_rowlane(KMeshPtrs M, KParams P, const double* __restrict__ u, cons
         for (int i = threadIdx.x; i < dlen; i += blockDim.x) dout[(int64_t)v0 * NC + i] = dbuf[i];
 }
 
+template <int ET, typename JT, int FAST>
+static void launch_rows(const KMeshPtrs& m, const int4* lane_conn, const KParams& p, const double* u, const double* uold,
+                        JT* J, double* d, int* err, int nwg, size_t lds, hipStream_t s)
+{
+    if constexpr (Topo<ET>::dim == 2)
+        assemble_rows_2d<ET, JT, FAST><<<nwg, m.block, lds, s>>>(m, lane_conn, p, u, uold, J, d, err);
+    else
+        assemble_rows<ET, JT, FAST><<<nwg, m.block, lds, s>>>(m, p, u, uold, J, d, err);
+}
+
 template <int ET, typename JT>
-static hipError_t launch_cfg(int fast, const KMeshPtrs& m, const KParams& p, const double* u, const double* uold,
-                             JT* J, double* d, int* err, int nwg, size_t lds, hipStream_t s)
+static hipError_t launch_cfg(int fast, const KMeshPtrs& m, const int4* lc, const KParams& p, const double* u,
+                             const double* uold, JT* J, double* d, int* err, int nwg, size_t lds, hipStream_t s)
 {
     switch (fast) {
-    case UPW_NO: assemble_rows<ET, JT, UPW_NO><<<nwg, m.block, lds, s>>>(m, p, u, uold, J, d, err); break;
-    case UPW_FULL: assemble_rows<ET, JT, UPW_FULL><<<nwg, m.block, lds, s>>>(m, p, u, uold, J, d, err); break;
-    case UPW_SKEWED: assemble_rows<ET, JT, UPW_SKEWED><<<nwg, m.block, lds, s>>>(m, p, u, uold, J, d, err); break;
-    case UPW_LPS: assemble_rows<ET, JT, UPW_LPS><<<nwg, m.block, lds, s>>>(m, p, u, uold, J, d, err); break;
-    default: assemble_rows<ET, JT, -1><<<nwg, m.block, lds, s>>>(m, p, u, uold, J, d, err); break;
+    case UPW_NO: launch_rows<ET, JT, UPW_NO>(m, lc, p, u, uold, J, d, err, nwg, lds, s); break;
+    case UPW_FULL: launch_rows<ET, JT, UPW_FULL>(m, lc, p, u, uold, J, d, err, nwg, lds, s); break;
+    case UPW_SKEWED: launch_rows<ET, JT, UPW_SKEWED>(m, lc, p, u, uold, J, d, err, nwg, lds, s); break;
+    case UPW_LPS: launch_rows<ET, JT, UPW_LPS>(m, lc, p, u, uold, J, d, err, nwg, lds, s); break;
+    default: launch_rows<ET, JT, -1>(m, lc, p, u, uold, J, d, err, nwg, lds, s); break;
     }
     return hipGetLastError();
 }
@@ -1663,24 +1812,24 @@ static int fast_path(const KParams& p)
 }
 
 template <int ET>
-static hipError_t launch_et(int jprec, const KMeshPtrs& m, const KParams& p, const double* u, const double* uold,
+static hipError_t launch_et(int jprec, const KMeshPtrs& m, const int4* lc, const KParams& p, const double* u, const double* uold,
                             void* J, double* d, int* err, int nwg, size_t lds, hipStream_t s)
 {
     const int fast = fast_path(p);
-    if (jprec == 64) return launch_cfg<ET, double>(fast, m, p, u, uold, static_cast<double*>(J), d, err, nwg, lds, s);
-    return launch_cfg<ET, float>(fast, m, p, u, uold, static_cast<float*>(J), d, err, nwg, lds, s);
+    if (jprec == 64) return launch_cfg<ET, double>(fast, m, lc, p, u, uold, static_cast<double*>(J), d, err, nwg, lds, s);
+    return launch_cfg<ET, float>(fast, m, lc, p, u, uold, static_cast<float*>(J), d, err, nwg, lds, s);
 }
 
-hipError_t launch_assemble(int et, int jprec, const KMeshPtrs& m, const KParams& p, const double* u,
-                           const double* uold, void* J, double* d, int* err, int nwg, size_t lds, hipStream_t s)
+hipError_t launch_assemble(int et, int jprec, const KMeshPtrs& m, const int4* lane_conn, const KParams& p,
+                           const double* u, const double* uold, void* J, double* d, int* err, int nwg, size_t lds, hipStream_t s)
 {
     if (lds > 65536 || m.block < 64 || m.block > 256 || m.block % 64) return hipErrorInvalidValue;
     switch (et) {
-    case ET_TRI:  return launch_et<ET_TRI>(jprec, m, p, u, uold, J, d, err, nwg, lds, s);
-    case ET_QUAD: return launch_et<ET_QUAD>(jprec, m, p, u, uold, J, d, err, nwg, lds, s);
-    case ET_TET:  return launch_et<ET_TET>(jprec, m, p, u, uold, J, d, err, nwg, lds, s);
-    case ET_HEX:  return launch_et<ET_HEX>(jprec, m, p, u, uold, J, d, err, nwg, lds, s);
-    case ET_PRISM: return launch_et<ET_PRISM>(jprec, m, p, u, uold, J, d, err, nwg, lds, s);
+    case ET_TRI:  return launch_et<ET_TRI>(jprec, m, lane_conn, p, u, uold, J, d, err, nwg, lds, s);
+    case ET_QUAD: return launch_et<ET_QUAD>(jprec, m, lane_conn, p, u, uold, J, d, err, nwg, lds, s);
+    case ET_TET:  return launch_et<ET_TET>(jprec, m, lane_conn, p, u, uold, J, d, err, nwg, lds, s);
+    case ET_HEX:  return launch_et<ET_HEX>(jprec, m, lane_conn, p, u, uold, J, d, err, nwg, lds, s);
+    case ET_PRISM: return launch_et<ET_PRISM>(jprec, m, lane_conn, p, u, uold, J, d, err, nwg, lds, s);
     }
     return hipErrorInvalidValue;
 }
@@ -1754,6 +1903,30 @@ hipError_t launch_assemble_split(int et, const RowLists& l, const KMeshPtrs& m, 
     case ET_HEX:  return launch_split_et<ET_HEX>(l, m, p, u, uold, J, d, err, nwg, lds, ne, recs, rowlane, s);
     }
     return hipErrorInvalidValue;
+}
+
+// the nodes of every lane's element in its corner's order
+template <int ET>
+__global__ void lane_nodes(const int4* __restrict__ lane_a, const int32_t* __restrict__ conn, int64_t ninc, int4* __restrict__ out)
+{
+    constexpr int N = Topo<ET>::nsh;
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= ninc) return;
+    const int4 la = lane_a[t];
+    int32_t c[4] = {0, 0, 0, 0};
+#pragma unroll
+    for (int k = 0; k < N; ++k) c[k] = conn[(int64_t)la.x * N + CanonH<ET>::c.perm[la.z & 0xff][k]];
+    out[t] = make_int4(c[0], c[1], c[2], c[3]);
+}
+
+hipError_t launch_lane_nodes(int et, const int4* lane_a, const int32_t* conn, int64_t ninc, int4* out, hipStream_t s)
+{
+    if (ninc <= 0) return hipSuccess;
+    const unsigned g = (unsigned)((ninc + 255) / 256);
+    if (et == ET_TRI) lane_nodes<ET_TRI><<<g, 256, 0, s>>>(lane_a, conn, ninc, out);
+    else if (et == ET_QUAD) lane_nodes<ET_QUAD><<<g, 256, 0, s>>>(lane_a, conn, ninc, out);
+    else return hipErrorInvalidValue;
+    return hipGetLastError();
 }
 
 hipError_t launch_geometry_cache(int et, const double* xyz, const int32_t* conn, int64_t ne, int difflen,

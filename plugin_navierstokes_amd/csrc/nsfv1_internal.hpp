@@ -39,8 +39,13 @@ struct KMeshPtrs {
     const int4* wg_a;         // [2 nwg]: {v0, v1, i0, i1}, {jbase low, jbase high, jlen, rounds}
 };
 
-hipError_t launch_assemble(int et, int jprec, const KMeshPtrs& m, const KParams& p, const double* u,
-                           const double* uold, void* J, double* d, int* err, int nwg, size_t lds_bytes,
+// 2D plans: the nodes of every lane's element in the order of its corner
+hipError_t launch_lane_nodes(int et, const int4* lane_a, const int32_t* conn, int64_t ninc, int4* out,
+                             hipStream_t stream);
+
+// lane_conn: of the plan (2D, else null)
+hipError_t launch_assemble(int et, int jprec, const KMeshPtrs& m, const int4* lane_conn, const KParams& p,
+                           const double* u, const double* uold, void* J, double* d, int* err, int nwg, size_t lds_bytes,
                            hipStream_t stream);
 
 // lists of a row gather that sums its blocks by owners (nsfv1_rows.hpp)
