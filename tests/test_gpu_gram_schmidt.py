@@ -1,6 +1,7 @@
 """Orthogonalisation against the Krylov basis and norms (device reductions of the
 GMRES loops) at the edges of their blocks (1024 entries below 2^20 unknowns,
-4096 from there on) and vector groups (8), and a workspace across meshes."""
+4096 from there on, 1024 or 512 with a held basis of up to 24 vectors) and
+vector groups (4, 8), and a workspace across meshes."""
 import ctypes as C
 
 import numpy as np
@@ -17,7 +18,9 @@ HS = 61
 
 
 @pytest.mark.parametrize("n,k", [(1, 1), (255, 2), (1023, 7), (1024, 8), (1025, 9), (5000, 60), ((1 << 20) - 1, 3),
-                                 (1 << 20, 8), ((1 << 20) + 1, 16), ((1 << 20) + 4099, 17)])
+                                 (1 << 20, 8), ((1 << 20) + 1, 16), ((1 << 20) + 4099, 17),
+                                 ((1 << 20) + 511, 1), ((1 << 20) + 513, 5), ((1 << 20) + 1025, 12), (1 << 20, 24),
+                                 ((1 << 20) + 1023, 25)])
 def test_orthogonalise(cuda, n, k):
     import torch
 
