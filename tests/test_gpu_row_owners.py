@@ -64,3 +64,29 @@ def test_routes_agree(cuda, mesh):
     # every sum runs in element order, whatever the workgroup holds
     for J, d in out[1:]:
         assert torch.equal(J, out[0][0]) and torch.equal(d, out[0][1])
+
+
+def test_lists_after_the_plane_march(cuda):
+    """The march needs no lists: the first call on records builds them; one that may
+    not allocate before that takes the fused kernel."""
+    import torch
+
+    mesh = M.cavity_3d(6, M.HEX)
+    u = torch.from_numpy(M.random_state(mesh, 4)).to(cuda)
+    disc = NavierStokesFV1("u,v,w,p", "Inner")
+    configure_disc(disc, {"upwind": "full", "nu": 0.02})
+    disc.set_mesh(mesh)
+    J, d = disc.assemble(u, jprec=F32)
+    assert disc.assembly_path_used() == 3
+    configure_disc(disc, {"upwind": "full", "nu": 0.02, "difflen": "fivepoint"})  # not a march configuration
+    J1, d1 = disc.assemble(u, J=torch.empty_like(J), d=torch.empty_like(d), jprec=F32, noalloc=True)
+    assert disc.assembly_path_used() == 1
+    J2, d2 = disc.assemble(u, jprec=F32)
+    assert disc.assembly_path_used() == 0
+    J3, d3 = disc.assemble(u, J=torch.empty_like(J), d=torch.empty_like(d), jprec=F32, noalloc=True)
+    assert torch.equal(J2, J3) and torch.equal(d2, d3)
+    # the routes round the same terms differently: entries of one row block are sums of
+    # at most eight of them
+    s = J2.abs().max()
+    assert float((J1 - J2).abs().max()) <= 64 * 2.0 ** -24 * float(s)
+    assert float((d1 - d2).abs().max()) <= 1e-12 * float(d2.abs().max())
