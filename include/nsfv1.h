@@ -252,9 +252,7 @@ int nsfv1_assemble(nsfv1_handle* h, const double* u, const double* u_old, double
    mode, no decision buffer yet (one nsfv1_assemble call with the same
    settings builds them).  The structured-hexahedra plane march and the
    fused path (FP64 Jacobians, the generic configuration) keep no records
-   and have no size limit; FP64 tetrahedra in the common configuration use
-   the array up to about 161 000 elements and the fused path beyond, in
-   both entries.
+   and have no size limit.
    Nothing in the array has to start at zero.  All calls on one device share
    its array: calls that overlap on one device (other streams, other host
    threads) race. */

@@ -185,15 +185,6 @@ struct nsfv1_handle {
     int geo_difflen = -1;
     // split assembly path (per-SCVF or, for simplices, per-element records)
     DevBuf recs;
-    // FP64 element records, one buffer per stream that assembles (at most 4, the
-    // others take the fused kernel): FP64 assemblies of one handle on several
-    // streams share nothing but the error flag
-    struct StreamBuf {
-        void* stream = nullptr;
-        DevBuf buf;
-    };
-    StreamBuf recs64[4];
-    int nrecs64 = 0;
     int64_t nblk() const { return nnz / ((dim + 1) * (dim + 1)); }
     // 0: split where supported, 1: fused kernel only, 2: split with row lanes,
     // 3: plane march on structured grids of parallelepipeds, otherwise 0
@@ -898,8 +889,6 @@ static int set_mesh_groups(nsfv1_handle* h, const double* xyz, int64_t nv, const
     }
     h->ninst = 0;
     h->recs.release();
-    for (auto& r : h->recs64) r.buf.release();
-    h->nrecs64 = 0;
     h->cpl_recs.release();
     return NSFV1_OK;
 }
@@ -1152,23 +1141,6 @@ static int make_lane_nodes(nsfv1_handle* h, int et, const DevBuf& conn, int64_t 
     return NSFV1_OK;
 }
 
-// FP64 element records of the stream (null: none to be had)
-static void* stream_records(nsfv1_handle* h, void* stream, size_t need)
-{
-    int i = 0;
-    while (i < h->nrecs64 && h->recs64[i].stream != stream) ++i;
-    if (i < h->nrecs64 && h->recs64[i].buf.n >= need) return h->recs64[i].buf.p;
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (i == 4 || hipStreamIsCapturing((hipStream_t)stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone ||
-        h->recs64[i].buf.alloc(need) != hipSuccess) {
-        (void)hipGetLastError();
-        return nullptr;
-    }
-    h->recs64[i].stream = stream;
-    h->nrecs64 = std::max(h->nrecs64, i + 1);
-    return h->recs64[i].buf.p;
-}
-
 // configurations whose SCVFs are coupled within an element: the FLOW
 // stabilisation (connected velocity components) and upwinds with ip shapes
 static bool coupled_config(const nsfv1_handle* h)
@@ -1367,22 +1339,13 @@ static int assemble_impl(nsfv1_handle* h, const double* u, const double* u_old, 
         int rc = fused3d ? NSFV1_OK : make_row_lists(h, jprec, P);
         if (rc) return rc;
     }
-    bool simplex = split && !fused2d && P.rnwg > 0 && simplex_supported(h->et, jprec) && !(h->path == 2 && P.rowlane);
+    const bool simplex = split && !fused2d && P.rnwg > 0 && simplex_supported(h->et, jprec) && !(h->path == 2 && P.rowlane);
     void* sx_recs = scratch;
     if (simplex) {
-        const size_t need = (size_t)simplex_record_bytes(h->et, jprec, h->ne);
-        if (jprec == NSFV1_F32 && !scratch) {
+        const size_t need = (size_t)simplex_record_bytes(h->et, h->ne);
+        if (!scratch) {
             if (h->recs.n < need && h->recs.alloc(need) != hipSuccess) return fail(NSFV1_ERR_DEVICE, "record buffer");
             sx_recs = h->recs.p;
-        } else if (jprec == NSFV1_F64) {
-            // the fused kernel needs no records: it takes meshes whose records
-            // exceed the no-allocation entry's scratch (both entries give the
-            // same bits) and calls that cannot allocate them now
-            simplex = need <= NOALLOC_SCRATCH_BYTES;
-            if (simplex && !scratch) {
-                sx_recs = stream_records(h, stream, need);
-                simplex = sx_recs != nullptr;
-            }
         }
     }
     if (h->mixed()) {
@@ -1497,8 +1460,8 @@ static int assemble_impl(nsfv1_handle* h, const double* u, const double* u_old, 
     } else if (simplex) {
         // triangles and tetrahedra: element records and block lists, also
         // without a Jacobian, so that the defect is bitwise the same
-        e = launch_assemble_simplex(h->et, jprec, P.rows, m, k, u, u_old, jvals, defect, h->errflag.as<int>(), h->ne, P.rnwg,
-                                    sx_recs, (hipStream_t)stream);
+        e = launch_assemble_simplex(h->et, P.rows, m, k, u, u_old, static_cast<float*>(jvals), defect, h->errflag.as<int>(),
+                                    h->ne, P.rnwg, sx_recs, (hipStream_t)stream);
         h->last_path = 0;
     } else if (split && jprec == NSFV1_F32 && !fused2d && !fused3d) {
         // also without a Jacobian (defect only): the gather then reads only

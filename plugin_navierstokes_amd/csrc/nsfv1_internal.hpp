@@ -75,10 +75,10 @@ hipError_t launch_assemble_split(int et, const RowLists& l, const KMeshPtrs& m, 
 // simplex path (nsfv1_simplex.hip; same configurations as the split path):
 // element records, then the row gather
 bool simplex_supported(int et, int jprec);
-int64_t simplex_record_bytes(int et, int jprec, int64_t ne);
-hipError_t launch_assemble_simplex(int et, int jprec, const RowLists& l, const KMeshPtrs& m, const KParams& p,
-                                   const double* u, const double* uold, void* J, double* d, int* err, int64_t ne,
-                                   int nwg, void* recs, hipStream_t stream);
+int64_t simplex_record_bytes(int et, int64_t ne);
+hipError_t launch_assemble_simplex(int et, const RowLists& l, const KMeshPtrs& m, const KParams& p, const double* u,
+                                   const double* uold, float* J, double* d, int* err, int64_t ne, int nwg, void* recs,
+                                   hipStream_t stream);
 
 // stabilised SCVF velocities of every element: out[ne][nip][dim]
 hipError_t launch_export_stab_vel(int et, const KMeshPtrs& m, const KParams& p, const double* u, const double* uold,

@@ -1,4 +1,4 @@
-// nsfv1_simplex.hip -- assembly of triangle and tetrahedron meshes in the
+// nsfv1_simplex.hip -- FP32 assembly of triangle and tetrahedron meshes in the
 // common configuration (FIELDS, one upwind object of type
 // no/full/skewed/LPS, no Stokes/PAC/Peclet/exact terms): one lane per element
 // evaluates every SCVF once, one lane per (node, element) forms the rows'
@@ -7,8 +7,8 @@
 //   simplex_records  one lane per element, in the element's own corner order:
 //     the shape gradients are constant, so they, the inverse Jacobian and the
 //     state gradients are formed once for all SCVFs.  Writes the corner
-//     gradients, a record of 12 values per SCVF (in the Jacobian's type) and
-//     the FP64 defect of every corner (the SCVF fluxes already added).
+//     gradients, a record of 12 floats per SCVF and the FP64 defect of every
+//     corner (the SCVF fluxes already added).
 //   simplex_rows     a workgroup owns consecutive nodes, a lane one incidence:
 //     it forms the element's row block of the node from the record and puts
 //     it into LDS, two rows at a time; then one lane per (block, row) adds the
@@ -32,49 +32,27 @@
 
 namespace nsfv1 {
 
-// Record of an element, in 16-byte chunks of VT (the Jacobian's type).  The
+// Record of an element, in 16-byte chunks.  The
 // chunks of eight consecutive elements are interleaved (chunk c of the eight:
 // 128 contiguous bytes), so a wave writes whole cache lines and neighbouring
 // elements share them when read.
-template <int ET, typename VT>
+template <int ET>
 struct SxRec {
     static constexpr int D = Topo<ET>::dim, N = Topo<ET>::nsh, NC = D + 1, NIP = Topo<ET>::nip;
     static constexpr int GS = D == 2 ? 2 : 4;              // values per corner gradient
     static constexpr int S = (N * GS + 3) / 4 * 4;         // after the gradients, per SCVF 12 values:
     //   normal (from -> to) and flux weight | vv, vc, sp factors, -nu rho | upwind shapes
     static constexpr int VALUES = S + 12 * NIP;
-    static constexpr int VPC = 16 / (int)sizeof(VT);
-    static constexpr int DEF = VALUES / VPC;               // first chunk of the corner defects
+    static constexpr int DEF = VALUES / 4;                 // first chunk of the corner defects
     static constexpr int CHUNKS = DEF + (N * NC + 1) / 2;
 };
 
 // four values of a record from value i (a multiple of four)
-template <typename VT>
-struct Sx4 {
-    VT x, y, z, w;
-};
-template <typename VT>
 __device__ __forceinline__ void sx_put(float4* rec, int i, double a, double b, double c, double d)
 {
-    if constexpr (sizeof(VT) == 4) {
-        rec[i / 4 * 8] = make_float4((float)a, (float)b, (float)c, (float)d);
-    } else {
-        *reinterpret_cast<double2*>(rec + i / 2 * 8) = make_double2(a, b);
-        *reinterpret_cast<double2*>(rec + (i / 2 + 1) * 8) = make_double2(c, d);
-    }
+    rec[i / 4 * 8] = make_float4((float)a, (float)b, (float)c, (float)d);
 }
-template <typename VT>
-__device__ __forceinline__ Sx4<VT> sx_get(const float4* rec, int i)
-{
-    if constexpr (sizeof(VT) == 4) {
-        const float4 t = rec[i / 4 * 8];
-        return {t.x, t.y, t.z, t.w};
-    } else {
-        const double2 a = *reinterpret_cast<const double2*>(rec + i / 2 * 8);
-        const double2 b = *reinterpret_cast<const double2*>(rec + (i / 2 + 1) * 8);
-        return {a.x, a.y, b.x, b.y};
-    }
-}
+__device__ __forceinline__ float4 sx_get(const float4* rec, int i) { return rec[i / 4 * 8]; }
 
 // SCVFs at a corner: the SCVF, the other end of its edge, whether the corner is
 // its `from` corner, packed for lookups by a lane's corner
@@ -96,10 +74,10 @@ struct SxCorner {
     static constexpr uint64_t IP = pack(0), OTHER = pack(1), FROM = pack(2);
 };
 
-template <int ET, typename VT>
+template <int ET>
 __device__ __forceinline__ int64_t sx_first(int64_t e)
 {
-    return (e >> 3) * (SxRec<ET, VT>::CHUNKS * 8) + (e & 7);
+    return (e >> 3) * (SxRec<ET>::CHUNKS * 8) + (e & 7);
 }
 
 // upwind of SCVF IP (upwind.cpp:52-80, 133-172, 337-430, 505-575) in the
@@ -201,12 +179,12 @@ struct SxElem {
     double *uo, *d;  // this lane's old velocities and defect sums in LDS, value i at i * SX_REC_BLOCK
 };
 
-template <int ET, typename VT, int FAST, int IP>
+template <int ET, int FAST, int IP>
 __device__ __forceinline__ void sx_scvf(SxElem<ET>& E, const KParams& P, double nu, const double* __restrict__ l2,
                                         uint8_t* dec, float4* __restrict__ rec, bool wantJ, bool& oku)
 {
     using T = Topo<ET>;
-    using R = SxRec<ET, VT>;
+    using R = SxRec<ET>;
     constexpr int D = T::dim, N = T::nsh, NC = D + 1;
     if constexpr (IP < T::nip) {
         double ipg[D], n[D], me[D], sv[D], pr = 0.0;
@@ -270,22 +248,22 @@ __device__ __forceinline__ void sx_scvf(SxElem<ET>& E, const KParams& P, double 
         }
         if (wantJ) {
             constexpr int C = R::S + 12 * IP;
-            sx_put<VT>(rec, C, n[0], n[1], D == 3 ? n[D - 1] : 0.0, prod);
-            sx_put<VT>(rec, C + 4, vv * idg, vc * idg, -P.inv_rho * idg, -1.0 * nu * P.rho);
-            sx_put<VT>(rec, C + 8, U[0], U[1], U[2], N == 4 ? U[N - 1] : 0.0);
+            sx_put(rec, C, n[0], n[1], D == 3 ? n[D - 1] : 0.0, prod);
+            sx_put(rec, C + 4, vv * idg, vc * idg, -P.inv_rho * idg, -1.0 * nu * P.rho);
+            sx_put(rec, C + 8, U[0], U[1], U[2], N == 4 ? U[N - 1] : 0.0);
         }
         __builtin_amdgcn_sched_barrier(0);  // one SCVF's values at a time in registers
-        sx_scvf<ET, VT, FAST, IP + 1>(E, P, nu, l2, dec, rec, wantJ, oku);
+        sx_scvf<ET, FAST, IP + 1>(E, P, nu, l2, dec, rec, wantJ, oku);
     }
 }
 
-template <int ET, typename VT, int FAST>
+template <int ET, int FAST>
 __global__ void __launch_bounds__(SX_REC_BLOCK, 2)
 simplex_records(KMeshPtrs M, KParams P, const double* __restrict__ u, const double* __restrict__ uold, int64_t ne,
                 float4* __restrict__ recs, int wantJ, int* __restrict__ err)
 {
     using T = Topo<ET>;
-    using R = SxRec<ET, VT>;
+    using R = SxRec<ET>;
     constexpr int D = T::dim, N = T::nsh, NC = D + 1, NIP = T::nip;
     const int64_t e = (int64_t)blockIdx.x * SX_REC_BLOCK + threadIdx.x;
     __shared__ double lds[N * (NC + D) * SX_REC_BLOCK];
@@ -357,18 +335,18 @@ simplex_records(KMeshPtrs M, KParams P, const double* __restrict__ u, const doub
             for (int k = 0; k < N; ++k) s += E.ul[k][a] * E.g[k][i];
             E.gv[a][i] = s;
         }
-    float4* rec = recs + sx_first<ET, VT>(e);
+    float4* rec = recs + sx_first<ET>(e);
     if (wantJ) {
         if constexpr (D == 3) {
 #pragma unroll
-            for (int k = 0; k < N; ++k) sx_put<VT>(rec, 4 * k, E.g[k][0], E.g[k][1], E.g[k][D - 1], 0.0);
+            for (int k = 0; k < N; ++k) sx_put(rec, 4 * k, E.g[k][0], E.g[k][1], E.g[k][D - 1], 0.0);
         } else {
-            sx_put<VT>(rec, 0, E.g[0][0], E.g[0][1], E.g[1][0], E.g[1][1]);
-            sx_put<VT>(rec, 4, E.g[2][0], E.g[2][1], 0.0, 0.0);
+            sx_put(rec, 0, E.g[0][0], E.g[0][1], E.g[1][0], E.g[1][1]);
+            sx_put(rec, 4, E.g[2][0], E.g[2][1], 0.0, 0.0);
         }
     }
     uint8_t* dec = (P.upw_mode != 0 && M.upw_dec) ? M.upw_dec + e * NIP : nullptr;
-    sx_scvf<ET, VT, FAST, 0>(E, P, M.nu_elem ? M.nu_elem[e] : P.nu, M.l2inv + e * NIP, dec, rec, wantJ != 0, oku);
+    sx_scvf<ET, FAST, 0>(E, P, M.nu_elem ? M.nu_elem[e] : P.nu, M.l2inv + e * NIP, dec, rec, wantJ != 0, oku);
     if (!oku) kernel_error(err, KERR_CUT_SIDE);
     if (!okg) kernel_error(err, KERR_DEGENERATE);
     double f[(N * NC + 1) / 2 * 2];
@@ -380,21 +358,20 @@ simplex_records(KMeshPtrs M, KParams P, const double* __restrict__ u, const doub
 }
 
 // rows per pass: 32 KB of segments for 256 lanes, so four workgroups fit a CU
-template <typename VT>
-constexpr int SX_RP = sizeof(VT) == 4 ? 2 : 1;
+constexpr int SX_RP = 2;
 
 // the row gather of nsfv1_rows.hpp from the element records, lanes in the order of
 // the nodes' incidences
-template <int ET, typename VT>
+template <int ET>
 __global__ void __launch_bounds__(256)
 simplex_rows(RowLists L, KMeshPtrs M, KParams P, const double* __restrict__ u, const float4* __restrict__ recs,
-             VT* __restrict__ J, double* __restrict__ dout)
+             float* __restrict__ J, double* __restrict__ dout)
 {
     using T = Topo<ET>;
-    using R = SxRec<ET, VT>;
+    using R = SxRec<ET>;
     using C = SxCorner<ET>;
     constexpr int D = T::dim, N = T::nsh, NC = D + 1;
-    constexpr int RP = SX_RP<VT>;
+    constexpr int RP = SX_RP;
     extern __shared__ __align__(16) unsigned char smem[];
     // consecutive workgroups (shared element data) go to the same XCD
     const int w = [] {
@@ -403,10 +380,10 @@ simplex_rows(RowLists L, KMeshPtrs M, KParams P, const double* __restrict__ u, c
         return x * per + (x < rem ? x : rem) + k;
     }();
     const bool wantJ = J != nullptr, vec = ((uintptr_t)J & 15) == 0;
-    OwnedRows<N, NC, VT, RP, false> rows(smem, L, M, w, 0, wantJ);
+    OwnedRows<N, NC, float, RP, false> rows(smem, L, M, w, 0, wantJ);
     const int inc = rows.i0 + (int)threadIdx.x;
     const bool active = (int)threadIdx.x < rows.ni;
-    VT B[N][NC][NC];
+    float B[N][NC][NC];
     double dl[NC];
 #pragma unroll
     for (int a = 0; a < NC; ++a) dl[a] = 0.0;
@@ -415,11 +392,11 @@ simplex_rows(RowLists L, KMeshPtrs M, KParams P, const double* __restrict__ u, c
 #pragma unroll
         for (int a = 0; a < NC; ++a)
 #pragma unroll
-            for (int c = 0; c < NC; ++c) B[k][a][c] = VT(0);
+            for (int c = 0; c < NC; ++c) B[k][a][c] = 0.f;
     if (active) {
         const int64_t e = M.inc_elem[inc];
         const int kv = M.inc_info[inc] & 0xff;
-        const float4* rec = recs + sx_first<ET, VT>(e);
+        const float4* rec = recs + sx_first<ET>(e);
 #pragma unroll
         for (int q = 0; q < (NC + 1) / 2; ++q) {
             // N NC doubles in chunks of two; a corner of a triangle starts mid-chunk
@@ -435,17 +412,17 @@ simplex_rows(RowLists L, KMeshPtrs M, KParams P, const double* __restrict__ u, c
             }
         }
         if (wantJ) {
-            VT g[N][D];
+            float g[N][D];
             if constexpr (D == 3) {
 #pragma unroll
                 for (int k = 0; k < N; ++k) {
-                    const Sx4<VT> x = sx_get<VT>(rec, 4 * k);
+                    const float4 x = sx_get(rec, 4 * k);
                     g[k][0] = x.x;
                     g[k][1] = x.y;
                     g[k][D - 1] = x.z;
                 }
             } else {
-                const Sx4<VT> x = sx_get<VT>(rec, 0), y = sx_get<VT>(rec, 4);
+                const float4 x = sx_get(rec, 0), y = sx_get(rec, 4);
                 g[0][0] = x.x;
                 g[0][1] = x.y;
                 g[1][0] = x.z;
@@ -454,32 +431,32 @@ simplex_rows(RowLists L, KMeshPtrs M, KParams P, const double* __restrict__ u, c
                 g[N - 1][1] = y.y;
             }
             // shape values at an SCVF's ip: one for the ends of its edge, one for the rest
-            constexpr VT PE = (VT)TabH<ET>::t.phi[0][T::edge[0][0]];
-            constexpr VT PO = (VT)TabH<ET>::t.phi[0][3 - T::edge[0][0] - T::edge[0][1]];
-            const VT s_ = (VT)P.s_a, rh = (VT)P.rho;
+            constexpr float PE = (float)TabH<ET>::t.phi[0][T::edge[0][0]];
+            constexpr float PO = (float)TabH<ET>::t.phi[0][3 - T::edge[0][0] - T::edge[0][1]];
+            const float s_ = (float)P.s_a, rh = (float)P.rho;
             // navier_stokes_fv1.cpp:317-593 for the SCVFs at the corner
 #pragma unroll
             for (int q = 0; q < T::cip; ++q) {
                 const int sh = 3 * (3 * kv + q);
                 const int ip = (int)(C::IP >> sh) & 7, oth = (int)(C::OTHER >> sh) & 7;
-                const VT sg = ((C::FROM >> sh) & 1) ? VT(1) : VT(-1);
-                const float4* r = rec + 12 * ip / R::VPC * 8;
-                const Sx4<VT> A = sx_get<VT>(r, R::S), F = sx_get<VT>(r, R::S + 4), Ux = sx_get<VT>(r, R::S + 8);
-                const VT Us[4] = {Ux.x, Ux.y, Ux.z, Ux.w};
-                VT n[D];
+                const float sg = ((C::FROM >> sh) & 1) ? 1.f : -1.f;
+                const float4* r = rec + 3 * ip * 8;
+                const float4 A = sx_get(r, R::S), F = sx_get(r, R::S + 4), Ux = sx_get(r, R::S + 8);
+                const float Us[4] = {Ux.x, Ux.y, Ux.z, Ux.w};
+                float n[D];
                 n[0] = sg * A.x;
                 n[1] = sg * A.y;
                 if constexpr (D == 3) n[D - 1] = sg * A.z;
-                const VT pw = sg * A.w, nr = F.w;
+                const float pw = sg * A.w, nr = F.w;
 #pragma unroll
                 for (int k = 0; k < N; ++k) {
-                    const VT ph = (k == kv || k == oth) ? PE : PO;
-                    const VT Sv = F.x * ph + F.y * Us[k];
-                    VT gn = VT(0);
+                    const float ph = (k == kv || k == oth) ? PE : PO;
+                    const float Sv = F.x * ph + F.y * Us[k];
+                    float gn = 0.f;
 #pragma unroll
                     for (int i = 0; i < D; ++i) gn += g[k][i] * n[i];
-                    const VT dg = nr * gn + Us[k] * pw;
-                    VT cpp = VT(0);
+                    const float dg = nr * gn + Us[k] * pw;
+                    float cpp = 0.f;
 #pragma unroll
                     for (int a = 0; a < D; ++a) {
                         B[k][a][a] += s_ * dg;
@@ -503,7 +480,7 @@ simplex_rows(RowLists L, KMeshPtrs M, KParams P, const double* __restrict__ u, c
 #pragma unroll
                 for (int a = 0; a < D; ++a) {
 #pragma unroll
-                    for (int k = 0; k < N; ++k) B[k][a][a] += k == kv ? (VT)(P.s_m * m) : VT(0);
+                    for (int k = 0; k < N; ++k) B[k][a][a] += k == kv ? (float)(P.s_m * m) : 0.f;
                     dl[a] += P.s_m * (uv[a] * m);
                 }
             }
@@ -529,49 +506,46 @@ simplex_rows(RowLists L, KMeshPtrs M, KParams P, const double* __restrict__ u, c
 // ---------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------
-// Triangles with FP64 Jacobian stay on the fused kernel: 300 x 300 cells 39 (full
-// upwind) and 62 us (LPS) against 54 and 55 us; tetrahedra 200 against 80 us (22^3
-// cells, LPS) and 42 against 33 us (6^3)
-bool simplex_supported(int et, int jprec) { return (et == ET_TRI && jprec == 32) || et == ET_TET; }
+// FP64 Jacobians take the fused kernel, which keeps nothing between the lanes of
+// two kernels: FP64 assemblies of one handle may overlap on several streams, in
+// captured graphs and through the no-allocation entry, with the same bits
+bool simplex_supported(int et, int jprec) { return (et == ET_TRI || et == ET_TET) && jprec == 32; }
 
-int64_t simplex_record_bytes(int et, int jprec, int64_t ne)
+int64_t simplex_record_bytes(int et, int64_t ne)
 {
-    const int64_t chunks = et == ET_TRI ? SxRec<ET_TRI, float>::CHUNKS
-                                        : (jprec == 64 ? SxRec<ET_TET, double>::CHUNKS : SxRec<ET_TET, float>::CHUNKS);
+    const int64_t chunks = et == ET_TRI ? SxRec<ET_TRI>::CHUNKS : SxRec<ET_TET>::CHUNKS;
     return (ne + 7) / 8 * 8 * chunks * 16;
 }
 
-template <int ET, typename VT>
+template <int ET>
 static hipError_t launch_simplex_et(const RowLists& l, const KMeshPtrs& m, const KParams& p, const double* u,
-                                    const double* uold, void* J, double* d, int* err, int64_t ne, int nwg,
+                                    const double* uold, float* J, double* d, int* err, int64_t ne, int nwg,
                                     float4* recs, hipStream_t s)
 {
     const unsigned ge = (unsigned)((ne + SX_REC_BLOCK - 1) / SX_REC_BLOCK);
     const int wj = J != nullptr;
     if (ne > 0) {
         switch (p.conv_upwind) {
-        case UPW_NO: simplex_records<ET, VT, UPW_NO><<<ge, SX_REC_BLOCK, 0, s>>>(m, p, u, uold, ne, recs, wj, err); break;
-        case UPW_FULL: simplex_records<ET, VT, UPW_FULL><<<ge, SX_REC_BLOCK, 0, s>>>(m, p, u, uold, ne, recs, wj, err); break;
-        case UPW_SKEWED: simplex_records<ET, VT, UPW_SKEWED><<<ge, SX_REC_BLOCK, 0, s>>>(m, p, u, uold, ne, recs, wj, err); break;
-        case UPW_LPS: simplex_records<ET, VT, UPW_LPS><<<ge, SX_REC_BLOCK, 0, s>>>(m, p, u, uold, ne, recs, wj, err); break;
+        case UPW_NO: simplex_records<ET, UPW_NO><<<ge, SX_REC_BLOCK, 0, s>>>(m, p, u, uold, ne, recs, wj, err); break;
+        case UPW_FULL: simplex_records<ET, UPW_FULL><<<ge, SX_REC_BLOCK, 0, s>>>(m, p, u, uold, ne, recs, wj, err); break;
+        case UPW_SKEWED: simplex_records<ET, UPW_SKEWED><<<ge, SX_REC_BLOCK, 0, s>>>(m, p, u, uold, ne, recs, wj, err); break;
+        case UPW_LPS: simplex_records<ET, UPW_LPS><<<ge, SX_REC_BLOCK, 0, s>>>(m, p, u, uold, ne, recs, wj, err); break;
         default: return hipErrorInvalidValue;
         }
     }
-    using Rows = OwnedRows<Topo<ET>::nsh, Topo<ET>::dim + 1, VT, SX_RP<VT>, false>;
+    using Rows = OwnedRows<Topo<ET>::nsh, Topo<ET>::dim + 1, float, SX_RP, false>;
     static_assert(Rows::BASE <= 64 * 1024, "dynamic LDS limit");
-    if (nwg > 0) simplex_rows<ET, VT><<<nwg, 256, Rows::BASE, s>>>(l, m, p, u, recs, static_cast<VT*>(J), d);
+    if (nwg > 0) simplex_rows<ET><<<nwg, 256, Rows::BASE, s>>>(l, m, p, u, recs, J, d);
     return hipGetLastError();
 }
 
-hipError_t launch_assemble_simplex(int et, int jprec, const RowLists& l, const KMeshPtrs& m, const KParams& p,
-                                   const double* u, const double* uold, void* J, double* d, int* err, int64_t ne,
-                                   int nwg, void* recs, hipStream_t s)
+hipError_t launch_assemble_simplex(int et, const RowLists& l, const KMeshPtrs& m, const KParams& p, const double* u,
+                                   const double* uold, float* J, double* d, int* err, int64_t ne, int nwg, void* recs,
+                                   hipStream_t s)
 {
     float4* r = static_cast<float4*>(recs);
-    if (et == ET_TRI && jprec == 32) return launch_simplex_et<ET_TRI, float>(l, m, p, u, uold, J, d, err, ne, nwg, r, s);
-    if (et == ET_TET)
-        return jprec == 64 ? launch_simplex_et<ET_TET, double>(l, m, p, u, uold, J, d, err, ne, nwg, r, s)
-                           : launch_simplex_et<ET_TET, float>(l, m, p, u, uold, J, d, err, ne, nwg, r, s);
+    if (et == ET_TRI) return launch_simplex_et<ET_TRI>(l, m, p, u, uold, J, d, err, ne, nwg, r, s);
+    if (et == ET_TET) return launch_simplex_et<ET_TET>(l, m, p, u, uold, J, d, err, ne, nwg, r, s);
     return hipErrorInvalidValue;
 }
 
