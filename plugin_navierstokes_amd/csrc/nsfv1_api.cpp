@@ -1237,10 +1237,10 @@ static int assemble_impl(nsfv1_handle* h, const double* u, const double* u_old, 
         int rc = make_plan(h, IncView{h->h_node_inc, h->h_inc_info, h->h_inc_elem, h->ninc, h->inc_pos},
                            jprec == NSFV1_F64 ? 8 : 4, P);
         if (!rc) rc = make_lane_nodes(h, h->et, h->conn, h->ninc, P);
-        // hexahedra get theirs with the first assembly that needs them: the
-        // plane march does not (96^3 cells: 6 ms of a first assembly's 122 ms)
+        // also where the first assembly needs no lists (the plane march): a later
+        // call that may not allocate finds them and gives the bits of any other
         P.rnwg = 0;
-        if (!rc && h->et != ET_HEX) rc = make_row_lists(h, jprec, P);
+        if (!rc) rc = make_row_lists(h, jprec, P);
         if (rc) P.valid = false;
         if (rc) return rc;
     }
@@ -1330,15 +1330,6 @@ static int assemble_impl(nsfv1_handle* h, const double* u, const double* u_old, 
     // against 91 us)
     const bool fused2d = h->path == 3 && h->dim == 2 && jprec == NSFV1_F32 &&
                          (k.conv_upwind == UPW_NO || k.conv_upwind == UPW_FULL || h->ne < 96 * 1024);
-    // hexahedra whose lists were not needed yet: built here, except in calls that
-    // may not allocate, which take the fused kernel
-    bool fused3d = false;
-    if (split && jprec == NSFV1_F32 && h->et == ET_HEX && !P.rowlane && P.rnwg == 0 && P.nwg > 0) {
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        fused3d = scratch || hipStreamIsCapturing((hipStream_t)stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone;
-        int rc = fused3d ? NSFV1_OK : make_row_lists(h, jprec, P);
-        if (rc) return rc;
-    }
     const bool simplex = split && !fused2d && P.rnwg > 0 && simplex_supported(h->et, jprec) && !(h->path == 2 && P.rowlane);
     void* sx_recs = scratch;
     if (simplex) {
@@ -1463,7 +1454,7 @@ static int assemble_impl(nsfv1_handle* h, const double* u, const double* u_old, 
         e = launch_assemble_simplex(h->et, P.rows, m, k, u, u_old, static_cast<float*>(jvals), defect, h->errflag.as<int>(),
                                     h->ne, P.rnwg, sx_recs, (hipStream_t)stream);
         h->last_path = 0;
-    } else if (split && jprec == NSFV1_F32 && !fused2d && !fused3d) {
+    } else if (split && jprec == NSFV1_F32 && !fused2d) {
         // also without a Jacobian (defect only): the gather then reads only
         // the records' fluxes, and the defect is bitwise the one assembled
         // together with the Jacobian
