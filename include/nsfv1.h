@@ -241,18 +241,19 @@ int nsfv1_assemble(nsfv1_handle* h, const double* u, const double* u_old, double
    reference: it is for callers that cannot call hipMalloc while they
    assemble (code under HIP graph capture, tight serving loops, harnesses
    that forbid allocation).  Same arguments, dispatch and results (bitwise)
-   as nsfv1_assemble; the SCVF records that the split and coupled paths
-   keep between their two kernels live in a fixed device array of
+   as nsfv1_assemble; the records that the split and coupled paths keep
+   between their two kernels live in a fixed device array of
    NSFV1_NOALLOC_SCRATCH_BYTES (one per device, held until the process
    ends) instead of a buffer the handle allocates.  Returns
    NSFV1_ERR_ARGUMENT, before any launch, when the mesh's records exceed
-   that array (split path: 128 bytes per SCVF, so about 87 000 hexahedra,
-   174 000 tetrahedra, 262 000 quadrilaterals or 349 000 triangles), or
-   when the handle has no launch plan for jprec or, in NSFV1_UPWIND_RECORD
-   mode, no decision buffer yet (one nsfv1_assemble call with the same
-   settings builds them).  The structured-hexahedra plane march and the
-   fused path (FP64 Jacobians, the generic configuration) keep no records
-   and have no size limit.
+   that array (split path: about 87 000 hexahedra, 262 000 quadrilaterals,
+   279 000 tetrahedra or 524 000 triangles; with row lanes 174 000
+   tetrahedra or 349 000 triangles), or when the handle has no launch plan
+   for jprec or, in NSFV1_UPWIND_RECORD mode, no decision buffer yet (one
+   nsfv1_assemble call with the same settings builds them).  The
+   structured-hexahedra plane march and the fused path (FP64 Jacobians, the
+   generic configuration, by default 2D meshes with no or full upwind or
+   below 98 304 elements) keep no records and have no size limit.
    Nothing in the array has to start at zero.  All calls on one device share
    its array: calls that overlap on one device (other streams, other host
    threads) race. */

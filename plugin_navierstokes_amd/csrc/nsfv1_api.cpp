@@ -1311,17 +1311,10 @@ static int assemble_impl(nsfv1_handle* h, const double* u, const double* u_old, 
         k.conv_upwind == k.stab_upwind && (k.conv_upwind == UPW_NO || k.conv_upwind == UPW_FULL || k.conv_upwind == UPW_SKEWED) &&
         ((uintptr_t)jvals & 15) == 0 && ((uintptr_t)defect & 15) == 0)
         mfast = k.conv_upwind;
-    // split path (FP32 SCVF records) and simplex path (element records)
+    // split path (FP32 records of the SCVFs, or of the elements of simplices)
     const bool split = !h->mixed() && mfast < 0 && !coupled_config(h) &&
                        (h->path == 0 || h->path == 2 || h->path == 3) && (parts & NSFV1_PART_A) && !h->ip_imports() &&
                        split_supported(h->et, k);
-    if (split && jprec == NSFV1_F32 && scratch) {
-        const size_t need = sizeof(float) * (size_t)split_record_floats(h->et, h->ne);
-        if (need > NOALLOC_SCRATCH_BYTES)
-            return fail(NSFV1_ERR_ARGUMENT, "the split path needs " + std::to_string(need) +
-                                                " bytes of SCVF records for this mesh; the no-allocation entry holds at most " +
-                                                std::to_string(NOALLOC_SCRATCH_BYTES));
-    }
     // 2D with FP32 Jacobian by default: the fused kernel without a ray cast (the
     // second kernel and the records cost more than the doubled SCVF work: 500 x 500
     // quads 63 against 83 us, 512 x 512 x 2 triangles 88 against 112 us) and below 96 Ki
@@ -1331,12 +1324,19 @@ static int assemble_impl(nsfv1_handle* h, const double* u, const double* u_old, 
     const bool fused2d = h->path == 3 && h->dim == 2 && jprec == NSFV1_F32 &&
                          (k.conv_upwind == UPW_NO || k.conv_upwind == UPW_FULL || h->ne < 96 * 1024);
     const bool simplex = split && !fused2d && P.rnwg > 0 && simplex_supported(h->et, jprec) && !(h->path == 2 && P.rowlane);
-    void* sx_recs = scratch;
-    if (simplex) {
-        const size_t need = (size_t)simplex_record_bytes(h->et, h->ne);
-        if (!scratch) {
+    const bool scvf = split && !fused2d && !simplex && jprec == NSFV1_F32;
+    void* recs = scratch;
+    if (simplex || scvf) {
+        const size_t need = simplex ? (size_t)simplex_record_bytes(h->et, h->ne)
+                                    : sizeof(float) * (size_t)split_record_floats(h->et, h->ne);
+        if (scratch) {
+            if (need > NOALLOC_SCRATCH_BYTES)
+                return fail(NSFV1_ERR_ARGUMENT, "the split path needs " + std::to_string(need) +
+                                                    " bytes of records for this mesh; the no-allocation entry holds at most " +
+                                                    std::to_string(NOALLOC_SCRATCH_BYTES));
+        } else {
             if (h->recs.n < need && h->recs.alloc(need) != hipSuccess) return fail(NSFV1_ERR_DEVICE, "record buffer");
-            sx_recs = h->recs.p;
+            recs = h->recs.p;
         }
     }
     if (h->mixed()) {
@@ -1434,7 +1434,7 @@ static int assemble_impl(nsfv1_handle* h, const double* u, const double* u_old, 
             return fail(NSFV1_ERR_NOT_IMPLEMENTED, "recorded upwind decisions are not available with the FLOW "
                                                    "stabilization or the positive upwind");
         const size_t need = (size_t)coupled_record_bytes(h->et, jprec, h->ne);
-        void* recs = scratch;
+        void* crecs = scratch;
         if (scratch) {
             if (need > NOALLOC_SCRATCH_BYTES)
                 return fail(NSFV1_ERR_ARGUMENT, "the coupled path needs " + std::to_string(need) +
@@ -1443,29 +1443,23 @@ static int assemble_impl(nsfv1_handle* h, const double* u, const double* u_old, 
         } else {
             if (h->cpl_recs.n < need && h->cpl_recs.alloc(need) != hipSuccess)
                 return fail(NSFV1_ERR_DEVICE, "coupled record buffer");
-            recs = h->cpl_recs.p;
+            crecs = h->cpl_recs.p;
         }
         e = launch_assemble_coupled(h->et, jprec, m, k, u, u_old, jvals, defect, h->errflag.as<int>(), P.nwg, P.lds,
-                                    h->ne, recs, nullptr, (hipStream_t)stream);
+                                    h->ne, crecs, nullptr, (hipStream_t)stream);
         h->last_path = 4;
     } else if (simplex) {
         // triangles and tetrahedra: element records and block lists, also
         // without a Jacobian, so that the defect is bitwise the same
         e = launch_assemble_simplex(h->et, P.rows, m, k, u, u_old, static_cast<float*>(jvals), defect, h->errflag.as<int>(),
-                                    h->ne, P.rnwg, sx_recs, (hipStream_t)stream);
+                                    h->ne, P.rnwg, recs, (hipStream_t)stream);
         h->last_path = 0;
-    } else if (split && jprec == NSFV1_F32 && !fused2d) {
+    } else if (scvf) {
         // also without a Jacobian (defect only): the gather then reads only
         // the records' fluxes, and the defect is bitwise the one assembled
         // together with the Jacobian
-        const size_t need = sizeof(float) * (size_t)split_record_floats(h->et, h->ne);
-        float* recs = static_cast<float*>(scratch);
-        if (!scratch) {
-            if (h->recs.n < need && h->recs.alloc(need) != hipSuccess) return fail(NSFV1_ERR_DEVICE, "record buffer");
-            recs = h->recs.as<float>();
-        }
         e = launch_assemble_split(h->et, P.rows, m, k, u, u_old, static_cast<float*>(jvals), defect, h->errflag.as<int>(), P.nwg,
-                                  P.lds, h->ne, recs, h->path == 2 && P.rowlane, (hipStream_t)stream);
+                                  P.lds, h->ne, static_cast<float*>(recs), h->path == 2 && P.rowlane, (hipStream_t)stream);
         h->last_path = (h->path == 2 && P.rowlane) ? 2 : 0;
     } else {
         e = launch_assemble(h->et, jprec, m, P.lane_conn.as<int4>(), k, u, u_old, jvals, defect, h->errflag.as<int>(), P.nwg, P.lds,

@@ -133,3 +133,37 @@ def test_noalloc_refusals(cuda):
     torch.cuda.synchronize()
     assert bool((Jb == 7.0).all()) and bool((db_ == 7.0).all())
     assert np.isclose(float(P.NOALLOC_SCRATCH_BYTES), 128 * 2 ** 20)
+
+
+# element counts between the limits of SCVF records (128 bytes each) and of the route
+# that runs: element records (480 bytes a tetrahedron), or none (fused kernel)
+@pytest.mark.parametrize("et,n,up,path", [(M.QUAD, 600, "full", 1), (M.TRI, 430, "no", 1), (M.TET, 33, "full", 0)])
+def test_noalloc_limit_is_the_routes_own(cuda, et, n, up, path):
+    import torch
+
+    mesh = M.cavity_3d(n, et, 0.1, 3) if et == M.TET else M.cavity_2d(n, et, 0.1, 3)
+    scvfs = {M.QUAD: 4, M.TRI: 3, M.TET: 6}[et]
+    assert mesh.ne * scvfs * 128 > P.NOALLOC_SCRATCH_BYTES
+    disc = _disc(mesh, {"upwind": up, "nu": 0.01})
+    J0, d0, J1, d1, used = _both(cuda, disc, mesh, 3)
+    assert used == path
+    assert torch.equal(J0, J1) and torch.equal(d0, d1)
+
+
+def test_noalloc_refuses_element_records_beyond_the_array(cuda):
+    import torch
+
+    mesh = M.cavity_3d(37, M.TET, 0.1, 3)
+    assert mesh.ne * 480 > P.NOALLOC_SCRATCH_BYTES
+    disc = _disc(mesh, {"upwind": "full", "nu": 0.01})
+    u, uo = _state(cuda, mesh, 2)
+    J = torch.empty(disc.nnz(), dtype=torch.float32, device=cuda)
+    d = torch.empty(disc.num_dofs(), dtype=torch.float64, device=cuda)
+    assert _call("nsfv1_assemble", disc, u, uo, F32, J, d) == 0
+    assert disc.assembly_path_used() == 0
+    J.fill_(7.0)
+    d.fill_(7.0)
+    assert _call("nsfv1_assemble_noalloc", disc, u, uo, F32, J, d) == ARGUMENT
+    assert b"holds at most" in P.load_library().nsfv1_last_error()
+    torch.cuda.synchronize()
+    assert bool((J == 7.0).all()) and bool((d == 7.0).all())
