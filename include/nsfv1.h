@@ -248,9 +248,11 @@ int nsfv1_assemble(nsfv1_handle* h, const double* u, const double* u_old, double
    NSFV1_ERR_ARGUMENT, before any launch, when the mesh's records exceed
    that array (split path: about 87 000 hexahedra, 262 000 quadrilaterals,
    279 000 tetrahedra or 524 000 triangles; with row lanes 174 000
-   tetrahedra or 349 000 triangles), or when the handle has no launch plan
-   for jprec or, in NSFV1_UPWIND_RECORD mode, no decision buffer yet (one
-   nsfv1_assemble call with the same settings builds them).  The
+   tetrahedra or 349 000 triangles; coupled path, FP32 Jacobian: about
+   30 000 hexahedra, 116 000 tetrahedra, 199 000 quadrilaterals or 338 000
+   triangles), or when the handle has no launch plan for jprec or, in
+   NSFV1_UPWIND_RECORD mode, no decision buffer yet (one nsfv1_assemble call
+   with the same settings builds them).  The
    structured-hexahedra plane march and the fused path (FP64 Jacobians, the
    generic configuration, by default 2D meshes with no or full upwind or
    below 98 304 elements) keep no records and have no size limit.

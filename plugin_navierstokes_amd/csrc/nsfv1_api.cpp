@@ -168,7 +168,7 @@ struct nsfv1_handle {
     size_t lds_cap = 64 * 1024;
     Plan plan32, plan64;
     // Newton-loop linear algebra
-    DevBuf cpl_recs;  // coupled path: per-SCVF row blocks
+    DevBuf cpl_recs;  // coupled path: element matrices and corner defects
     DevBuf dir_rows, dir_mask;  // Dirichlet rows, and 1 per Dirichlet DoF
     DevBuf gm_V, gm_Binv, gm_part, gm_small, gm_w;
     int64_t ndir = 0;
@@ -1356,7 +1356,7 @@ static int assemble_impl(nsfv1_handle* h, const double* u, const double* u_old, 
             if (scratch) {
                 if (need > NOALLOC_SCRATCH_BYTES)
                     return fail(NSFV1_ERR_ARGUMENT, "the coupled path needs " + std::to_string(need) +
-                                                        " bytes of SCVF records for this mesh; the no-allocation entry holds at most " +
+                                                        " bytes of records for this mesh; the no-allocation entry holds at most " +
                                                         std::to_string(NOALLOC_SCRATCH_BYTES));
                 crecs = scratch;
             } else {
@@ -1438,7 +1438,7 @@ static int assemble_impl(nsfv1_handle* h, const double* u, const double* u_old, 
         if (scratch) {
             if (need > NOALLOC_SCRATCH_BYTES)
                 return fail(NSFV1_ERR_ARGUMENT, "the coupled path needs " + std::to_string(need) +
-                                                    " bytes of SCVF records for this mesh; the no-allocation entry holds at most " +
+                                                    " bytes of records for this mesh; the no-allocation entry holds at most " +
                                                     std::to_string(NOALLOC_SCRATCH_BYTES));
         } else {
             if (h->cpl_recs.n < need && h->cpl_recs.alloc(need) != hipSuccess)

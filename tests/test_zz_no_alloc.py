@@ -167,3 +167,28 @@ def test_noalloc_refuses_element_records_beyond_the_array(cuda):
     assert b"holds at most" in P.load_library().nsfv1_last_error()
     torch.cuda.synchronize()
     assert bool((J == 7.0).all()) and bool((d == 7.0).all())
+
+
+@pytest.mark.parametrize("n,fits", [(28, True), (32, False)])
+def test_noalloc_coupled_limit(cuda, n, fits):
+    """Element matrices and corner defects: 8 x 8 blocks of 4 x 4 FP32 values and 8 x 4
+    doubles a hexahedron."""
+    import torch
+
+    mesh = M.box_3d((n, n, n), (1.0, 1.0, 1.0), M.HEX, 0.1, 2)
+    assert (mesh.ne * (8 * 8 * 16 * 4 + 8 * 4 * 8) <= P.NOALLOC_SCRATCH_BYTES) == fits
+    disc = _disc(mesh, {"upwind": "positive", "nu": 0.01})
+    if fits:
+        J0, d0, J1, d1, path = _both(cuda, disc, mesh, 3)
+        assert path == 4
+        assert torch.equal(J0, J1) and torch.equal(d0, d1)
+        return
+    u, uo = _state(cuda, mesh, 2)
+    J = torch.empty(disc.nnz(), dtype=torch.float32, device=cuda)
+    d = torch.empty(disc.num_dofs(), dtype=torch.float64, device=cuda)
+    assert _call("nsfv1_assemble", disc, u, uo, F32, J, d) == 0
+    J.fill_(7.0)
+    assert _call("nsfv1_assemble_noalloc", disc, u, uo, F32, J, d) == ARGUMENT
+    assert b"holds at most" in P.load_library().nsfv1_last_error()
+    torch.cuda.synchronize()
+    assert bool((J == 7.0).all())
