@@ -596,6 +596,14 @@ coupled_scvf(KMeshPtrs M, KParams P, const double* __restrict__ u, const double*
             if (own) mycol = c;
             wave_sync();
         }
+        // a row of NaN never is the largest and does not pivot: the rows of the
+        // inverse that nothing writes then are NaN too
+        if (__any(act && mycol < 0)) {
+            if (act)
+#pragma unroll
+                for (int j = 0; j < NIP; ++j) S.inv[ip][j] = __builtin_nan("");
+            wave_sync();
+        }
         // inverse: entry (k, p_j) is entry j of the row that column k pivoted on
         if (act && mycol >= 0)
 #pragma unroll
