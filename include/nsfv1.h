@@ -433,7 +433,8 @@ int nsfv1_newton_graph_replay(nsfv1_handle* h, void* stream);
 /* Launch-shape autotuner: times `reps` assemblies (HIP events on stream)
    of every assembly path and launch shape the handle accepts (paths 0 and
    1 x 64/128/256 threads x 16/32/64 KiB, path 2 x 64 threads, path 3 on
-   structured grids), keeps the fastest on the handle and returns it in
+   structured grids; triangles and tetrahedra on records, whose shape is
+   fixed, once), keeps the fastest on the handle and returns it in
    best[3] = {path, threads, lds_bytes}; table (host, 4 doubles per
    candidate: path, threads, lds, ms), with capacity and count in *ntable,
    may be NULL.  Shapes the mesh cannot use are skipped.  No counterpart in
@@ -535,11 +536,16 @@ int nsfv1_set_assembly_path(nsfv1_handle* h, int path);
    counterpart in the plugin. */
 int nsfv1_assembly_path_used(nsfv1_handle* h, int* path);
 
-/* Launch shape of the assembly: incidences (threads) per workgroup (64..256,
-   a multiple of 64) and the LDS budget per workgroup in bytes (4..64 KiB);
-   0 keeps the current value.  Set while path 3 is selected, the budget in
-   KiB is instead the number of node planes per work unit of the plane
-   march.  Used by the autotuner. */
+/* Launch shape of the assembly: at most this many incidences (threads) per
+   workgroup (64..256, a multiple of 64) and the LDS budget per workgroup in
+   bytes (4..64 KiB); 0 keeps the current value.  256 and 64 KiB are the
+   defaults; with 256, meshes whose rows fill the budget first (FP64
+   hexahedra) run in workgroups of 128.  Results do not depend on either.
+   Triangles and tetrahedra on records (path 0, FP32 Jacobian) run in
+   workgroups of their own, whatever is set; the row gather of hexahedra on
+   records takes the threads, and the budget as a limit on its nodes.  Set
+   while path 3 is selected, the budget in KiB is instead the number of node
+   planes per work unit of the plane march.  Used by the autotuner. */
 int nsfv1_set_launch(nsfv1_handle* h, int threads, int lds_bytes);
 
 #ifdef __cplusplus

@@ -163,8 +163,7 @@ struct nsfv1_handle {
     std::vector<int32_t> bnd_elem_in[BND_KINDS], bnd_side_in[BND_KINDS];  // the input (element, side) lists
     double slide_k = 0.0, slide_lim = 0.0;
     std::vector<int64_t> h_rowptr, h_node_inc;
-    int max_threads = 256;
-    bool threads_set = false;  // by nsfv1_set_launch
+    int max_threads = 256;  // 256: at most, a plan may take 128 (make_plan)
     size_t lds_cap = 64 * 1024;
     Plan plan32, plan64;
     // Newton-loop linear algebra
@@ -194,6 +193,7 @@ struct nsfv1_handle {
     int march_n[3] = {0, 0, 0};
     int march_zc = 0;  // node planes per work unit (0: chosen from the grid)
     int last_path = -1;  // kernel family of the last element assembly (nsfv1_assembly_path_used)
+    bool last_simplex = false;  // path 0 on element records, whose workgroups no launch shape changes
     // batched instances: per-element viscosity
     DevBuf nu_elem;
     int64_t ninst = 0;
@@ -949,7 +949,6 @@ int nsfv1_set_launch(nsfv1_handle* h, int threads, int lds_bytes)
     if (threads) {
         if (threads < 64 || threads > 256 || threads % 64) return fail(NSFV1_ERR_ARGUMENT, "threads must be 64..256, a multiple of 64");
         h->max_threads = threads;
-        h->threads_set = true;
     }
     if (lds_bytes && h->path == 3) {
         // the plane march reads the budget in KiB as node planes per work unit
@@ -972,7 +971,6 @@ static int make_plan(nsfv1_handle* h, const IncView& g, int jbytes, Plan& P, int
     wn.push_back(0);
     int64_t v = 0;
     size_t maxlds = 0;
-    const bool chosen = threads != 0 || h->threads_set;
     if (!threads) threads = h->max_threads;
     // the row-lane split gather puts dim+1 lanes on each incidence of a
     // 64-lane workgroup
@@ -1012,7 +1010,7 @@ static int make_plan(nsfv1_handle* h, const IncView& g, int jbytes, Plan& P, int
     // CUs hold (one each, by registers), half the lanes, all of them active,
     // are faster (FP64 hexahedra, LPS: 20^3 98 -> 60 us, 36^3 517 -> 322 us,
     // 50^3 1342 -> 874 us; 16^3, one workgroup a CU, 51 against 56 us)
-    if (!chosen && !skip_empty && threads == 256 && wr.size() > 256 && (size_t)g.ninc < wr.size() * 192 &&
+    if (!skip_empty && threads == 256 && wr.size() > 256 && (size_t)g.ninc < wr.size() * 192 &&
         *std::max_element(wr.begin(), wr.end()) <= 128)
         return make_plan(h, g, jbytes, P, 128);
     P.nwg = (int)wr.size();
@@ -1303,6 +1301,7 @@ static int assemble_impl(nsfv1_handle* h, const double* u, const double* u_old, 
                 P.perm.as<int32_t>(), h->nu_elem.as<double>(), h->nu_ip.as<double>(), h->f_scv.as<double>(),
                 h->f_scvf.as<double>(), h->rho_ip.as<double>(), h->rho_scv.as<double>(), P.block, P.lane_a.as<int4>(),
                 P.lane_pos.as<uint64_t>(), P.wg_a.as<int4>()};
+    h->last_simplex = false;
     hipError_t e;
     int mfast = -1;
     if (h->path == 3 && h->march_ok && jprec == NSFV1_F32 && (parts & NSFV1_PART_A) && h->difflen == DL_RAW &&
@@ -1454,6 +1453,7 @@ static int assemble_impl(nsfv1_handle* h, const double* u, const double* u_old, 
         e = launch_assemble_simplex(h->et, P.rows, m, k, u, u_old, static_cast<float*>(jvals), defect, h->errflag.as<int>(),
                                     h->ne, P.rnwg, recs, (hipStream_t)stream);
         h->last_path = 0;
+        h->last_simplex = true;
     } else if (scvf) {
         // also without a Jacobian (defect only): the gather then reads only
         // the records' fluxes, and the defect is bitwise the one assembled
@@ -2644,7 +2644,6 @@ int nsfv1_autotune(nsfv1_handle* h, const double* u, const double* u_old, double
     if (h->march_ok)
         for (int l : {8192, 16384, 32768}) cand.push_back({3, 256, l});
     const int keep_path = h->path, keep_threads = h->max_threads;
-    const bool keep_set = h->threads_set;
     const size_t keep_lds = h->lds_cap;
     const int keep_zc = h->march_zc;
     hipEvent_t e0, e1;
@@ -2654,10 +2653,16 @@ int nsfv1_autotune(nsfv1_handle* h, const double* u, const double* u_old, double
     Cand bc{-1, 0, 0};
     int nt = 0;
     const int cap = ntable ? *ntable : 0;
+    bool one_shape = false;  // path 0 runs in workgroups of its own: timed once, in the default shape
     for (const Cand& c : cand) {
+        if (one_shape && c.path == 0 && (c.threads != 256 || c.lds != 65536)) continue;
         if (nsfv1_set_assembly_path(h, c.path) || nsfv1_set_launch(h, c.threads, c.lds)) continue;
         // a shape the mesh cannot use is refused by the library: skipped
         if (nsfv1_assemble(h, u, u_old, dt, 1.0, s_m, 0.0, parts, jvals, jprec, defect, stream)) continue;
+        if (h->last_simplex && (c.threads != 256 || c.lds != 65536)) {
+            one_shape = true;
+            continue;
+        }
         if (hipEventRecord(e0, s) != hipSuccess) break;
         int rc = 0;
         for (int r = 0; r < reps && !rc; ++r)
@@ -2682,7 +2687,6 @@ int nsfv1_autotune(nsfv1_handle* h, const double* u, const double* u_old, double
     if (bc.path < 0) {
         h->path = keep_path;
         h->max_threads = keep_threads;
-        h->threads_set = keep_set;
         h->lds_cap = keep_lds;
         h->march_zc = keep_zc;
         invalidate_plans(h);

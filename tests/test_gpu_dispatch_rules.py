@@ -59,3 +59,16 @@ def test_fp64_hexahedra_any_workgroup(cuda, n):
     # the order of every sum is the incidence's, whatever the workgroup holds
     for J, d in out[1:]:
         assert torch.equal(J, out[0][0]) and torch.equal(d, out[0][1])
+
+
+def test_autotuner_times_a_fixed_shape_once(cuda):
+    """Tetrahedra on element records run in workgroups of their own: one path-0 entry, the
+    default shape, so that no other shape is left set by chance."""
+    import torch
+
+    mesh = M.cavity_3d(5, M.TET, 0.1, 3)
+    disc = _disc(mesh, "lps")
+    u = torch.from_numpy(M.random_state(mesh, 4)).to(cuda)
+    best, table = disc.autotune_native(u, reps=2, jprec=F32)
+    assert [tuple(t[1:3]) for t in table if t[0] == 0] == [(256, 65536)]
+    assert best in [t[:3] for t in table] and any(t[0] == 1 for t in table)
