@@ -975,17 +975,20 @@ hipError_t launch_dirichlet(int jprec, const int64_t* rowptr, const int32_t* col
     return hipGetLastError();
 }
 
-// node-block launch: G lanes per node, in 3D the power of two (8, 16 or 32) that
-// covers the mean number of neighbour blocks per node; up to 12 blocks of a 2D
-// mesh go by 4 lanes (two or three blocks each: fewer lanes idle, two exchange
-// steps less; FP32, 0.77 M nodes of 9 blocks 94 us against 102 us with 16 lanes)
+// node-block launch: G lanes per node, the power of two (8, 16 or 32) that covers
+// the mean number of neighbour blocks per node; 4 lanes for the 7 to 12 blocks of
+// quadrilaterals (two or three blocks each: fewer lanes idle, two exchange steps
+// less).  0.77 M nodes of 9 blocks, FP32 77 -> 65 us, FP64 150 us with either; 16 k
+// nodes 3.8 -> 3.2 and 4.6 -> 3.7 us.  Triangles (7 blocks less the boundary's share,
+// always below 7) keep 8: with 4 lanes 0.77 M nodes 47 us in FP32 as well, but
+// 124 against 88 us in FP64, and 1 k nodes 3.0 against 2.7 us.
 template <typename JT, int NC, int RES>
 static void launch_nodeblock(const int64_t* rowptr, const int32_t* adj, const JT* A, const double* x, const double* b,
                              double* y, int64_t nv, int64_t nnz, const double* Binv, double omega,
                              const uint8_t* mask, hipStream_t s)
 {
     const int64_t slots = nv > 0 ? nnz / ((int64_t)NC * NC * nv) : 0;
-    if (NC == 3 && slots <= 12)
+    if (NC == 3 && slots >= 7 && slots <= 12)
         nodeblock_mv<JT, NC, 4, RES><<<blocks_for(nv * 4, 256), 256, 0, s>>>(rowptr, adj, A, x, b, y, nv, Binv, omega, mask);
     else if (slots > 16)
         nodeblock_mv<JT, NC, 32, RES><<<blocks_for(nv * 32, 256), 256, 0, s>>>(rowptr, adj, A, x, b, y, nv, Binv, omega, mask);
