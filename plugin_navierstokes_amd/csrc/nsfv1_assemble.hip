@@ -1256,9 +1256,12 @@ __host__ __device__ constexpr int64_t records_blocks(int64_t ne_pad)
 }
 
 // the workgroups of frame index Q = 0, then 1, then 2 (one launch: they run
-// side by side; LPS, 56^3 cells 283 -> 215 us, a mesh of one workgroup 29 -> 10 us)
+// side by side; LPS, 56^3 cells 283 -> 215 us, a mesh of one workgroup 29 -> 10 us).
+// Two waves per SIMD, but for the skewed upwind on hexahedra: held to 256
+// registers its casts spill 340 of them to memory (48^3 cells, the whole assembly
+// 480 us, 397 us with one wave; 20^3: 71 and 46 us; 96^3: 3703 and 3110 us)
 template <int ET, int FAST>
-__global__ void __launch_bounds__(256, 2)
+__global__ void __launch_bounds__(256, ET == ET_HEX && FAST == UPW_SKEWED ? 1 : 2)
 scvf_records(KMeshPtrs M, KParams P, const double* __restrict__ u, const double* __restrict__ uold, int64_t ne,
              int64_t ne_pad, float* __restrict__ recs, int* __restrict__ err)
 {
