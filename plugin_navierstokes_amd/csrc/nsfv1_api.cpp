@@ -1961,12 +1961,13 @@ int nsfv1_set_dirichlet(nsfv1_handle* h, const int64_t* dofs, int64_t n)
         if (x < 0 || x >= h->ndof) return fail(NSFV1_ERR_ARGUMENT, "Dirichlet DoF out of range");
     std::vector<uint8_t> mask((size_t)h->ndof, 0);
     for (int64_t x : d) mask[(size_t)x] = 1;
+    h->ndir = 0;  // until both arrays are there
     if (h->dir_rows.alloc(sizeof(int64_t) * std::max<int64_t>(n, 1)) != hipSuccess ||
         h->dir_mask.alloc(mask.size()) != hipSuccess ||
         (n > 0 && hipMemcpy(h->dir_rows.p, d.data(), sizeof(int64_t) * n, hipMemcpyHostToDevice) != hipSuccess) ||
         (n > 0 && hipMemcpy(h->dir_mask.p, mask.data(), mask.size(), hipMemcpyHostToDevice) != hipSuccess))
         return fail(NSFV1_ERR_DEVICE, "Dirichlet upload");
-    h->ndir = n;
+    h->ndir = std::max<int64_t>(n, 0);
     return NSFV1_OK;
 }
 

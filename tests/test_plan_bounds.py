@@ -1,7 +1,7 @@
 """Launch plans checked on the CPU: every index the fused row kernels take from a plan
 stays inside its array, the workgroup's LDS and the CSR pattern, packed or not, for
 workgroups of 64 to 256 lanes (the 128 of large FP64 hexahedral meshes among them) and
-odd meshes."""
+odd meshes; and set-up calls that run out of memory leave no stale sizes behind."""
 from __future__ import annotations
 
 import ctypes as C
@@ -106,4 +106,25 @@ def test_every_index_of_a_plan(lib, name):
         assert block[0, 0, 64] == block[256, 65536, 64] == 128 and block[0, 0, 32] == 256
     if name == "hex16":
         assert block[0, 0, 64] == 256
+    lib.nsfv1_destroy(h)
+
+
+@pytest.mark.parametrize("first", [0, 1])  # the rows' array, the mask's
+def test_dirichlet_rows_after_a_failed_allocation(lib, first):
+    mesh = M.cavity_3d(3, M.HEX)
+    h = _handle(lib, mesh)
+    lib.nsfv1_set_dirichlet.argtypes = [C.c_void_p, C.c_void_p, C.c_int64]
+    lib.nsfv1_apply_dirichlet.argtypes = [C.c_void_p, C.c_void_p, C.c_int] + [C.c_void_p] * 4
+    rows = np.arange(40, dtype=np.int64)
+    assert lib.nsfv1_set_dirichlet(h, rows.ctypes.data, 40) == 0
+    lib.plan_fail_allocation(first)
+    assert lib.nsfv1_set_dirichlet(h, rows.ctypes.data, 7) != 0
+    lib.plan_fail_allocation(-1)
+    # the call that failed left no rows, in particular not forty in an array of seven
+    assert lib.nsfv1_apply_dirichlet(h, 16, 32, None, None, None, None) == 0
+    assert lib.plan_error() == b"" and lib.plan_dirichlet_rows() == 0
+    # a count below zero is none
+    assert lib.nsfv1_set_dirichlet(h, rows.ctypes.data, -1) == 0
+    assert lib.nsfv1_apply_dirichlet(h, 16, 32, None, None, None, None) == 0
+    assert lib.plan_dirichlet_rows() == 0
     lib.nsfv1_destroy(h)
