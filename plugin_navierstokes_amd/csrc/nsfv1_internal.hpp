@@ -50,9 +50,9 @@ hipError_t launch_assemble(int et, int jprec, const KMeshPtrs& m, const int4* la
 
 // lists of a row gather that sums its blocks by owners (nsfv1_rows.hpp)
 struct RowLists {
-    const uint2* own;        // [nblk] blocks of each workgroup, most items first: first item | items << 12 | blocks
-                             // of the node << 23, (first block of the node NC + slot) | block << 16, both from the
-                             // workgroup's first
+    const uint2* own;        // [nblk] blocks of each workgroup (hexahedra: most items first): first item |
+                             // items << 12 | blocks of the node << 23, (first block of the node NC + slot) |
+                             // block << 16, both from the workgroup's first
     const uint16_t* items;   // [nsh ninc] lane << 3 | corner, sorted by block, then element
     const uint8_t* lane_of;  // [ninc] lane of the incidence
     const int32_t* wg_node;  // [nwg + 1] first node of each workgroup (at most 255 nodes, 256 incidences)

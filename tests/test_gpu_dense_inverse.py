@@ -1,6 +1,6 @@
 """Dense inverse of the coarsest multigrid level (blocked Gauss-Jordan) against
-numpy, at the edges of its panels (16 pivots), update tiles (32 columns, 256
-rows) and rows per thread (1024)."""
+numpy, at the edges of its panels (16 pivots), update tiles (16 x 16, one a wave)
+and rows per thread (512 threads: two rows from 513 on, three from 1025)."""
 import ctypes as C
 
 import numpy as np
@@ -35,7 +35,7 @@ def invert(A, dtype=np.float64):
     return rc, inv.cpu().numpy(), int(err.item())
 
 
-@pytest.mark.parametrize("n", [1, 2, 15, 16, 17, 31, 33, 63, 64, 65, 255, 257, 448, 867, 1023, 1024, 1025, 1200])
+@pytest.mark.parametrize("n", [1, 2, 15, 16, 17, 31, 33, 63, 64, 65, 127, 128, 129, 255, 257, 448, 511, 512, 513, 867, 1023, 1024, 1025, 1200])
 def test_inverse(n):
     rng = np.random.default_rng(n)
     A = rng.standard_normal((n, n))
@@ -53,7 +53,7 @@ def test_inverse(n):
     assert np.array_equal(inv, invert(A)[1])
 
 
-@pytest.mark.parametrize("n,k", [(40, 0), (40, 17), (300, 299), (1100, 1030)])
+@pytest.mark.parametrize("n,k", [(40, 0), (40, 17), (300, 299), (512, 511), (513, 512), (1100, 1030)])
 def test_null_mode_is_pinned(n, k):
     """A zero row and column k: the other unknowns are solved, x_k = 0."""
     rng = np.random.default_rng(k)

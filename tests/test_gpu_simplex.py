@@ -21,9 +21,9 @@ def _cut(mesh, ne):
     return M.Mesh(mesh.et, mesh.xyz, mesh.conn[:ne], {}, ())
 
 
-# element counts around groups of eight and workgroups of 256 elements
-MESHES = [(M.TRI, lambda ne: _cut(M.cavity_2d(14, M.TRI, 0.1, 3), ne), ne) for ne in (1, 7, 8, 9, 255, 257, 392)]
-MESHES += [(M.TET, lambda ne: _cut(M.cavity_3d(4, M.TET, 0.1, 3), ne), ne) for ne in (1, 7, 8, 9, 257, 384)]
+# element counts around groups of eight and the workgroups' 128 elements
+MESHES = [(M.TRI, lambda ne: _cut(M.cavity_2d(14, M.TRI, 0.1, 3), ne), ne) for ne in (1, 7, 8, 9, 127, 128, 129, 255, 257, 392)]
+MESHES += [(M.TET, lambda ne: _cut(M.cavity_3d(4, M.TET, 0.1, 3), ne), ne) for ne in (1, 7, 8, 9, 127, 128, 129, 257, 384)]
 
 
 def _jviol(J, Jr, Ja, jprec):
