@@ -374,15 +374,15 @@ def batched_leg(steps: int = 20, count: int = 256):
 # the kernels of one 128^3 hex assembly per assembly path that ran
 ASSEMBLY_KERNELS = {
     3: "nsfv1::march::march_hex<2, false> (plane march: one launch per assembly)",
-    0: "one assembly = nsfv1::scvf_records<3,2,Q> (Q=0,1,2) + nsfv1::assemble_rows_split<3,2>",
-    2: "one assembly = nsfv1::scvf_records<3,2,Q> (Q=0,1,2) + nsfv1::assemble_rows_rowlane<3,2>",
+    0: "one assembly = nsfv1::scvf_records<3,2> + nsfv1::split_rows<3,2>",
+    2: "one assembly = nsfv1::scvf_records<3,2> + nsfv1::assemble_rows_rowlane<3,2>",
     1: "nsfv1::assemble_rows<3,float,2> (fused, one launch per assembly)",
 }
 
 # the tetrahedral channel (LPS upwind: template argument 3)
 CHANNEL_KERNELS = {
-    0: "one assembly = nsfv1::scvf_records<2,3,Q> + nsfv1::assemble_rows_split<2,3> (split path)",
-    2: "one assembly = nsfv1::scvf_records<2,3,Q> + nsfv1::assemble_rows_rowlane<2,3>",
+    0: "one assembly = nsfv1::simplex_records<2,3> + nsfv1::simplex_rows<2> (element records)",
+    2: "one assembly = nsfv1::scvf_records<2,3> + nsfv1::assemble_rows_rowlane<2,3>",
     1: "nsfv1::assemble_rows<2,float,3> (fused, one launch per assembly)",
 }
 

@@ -473,7 +473,7 @@ predict_scale_final(const double* __restrict__ part, int nparts, int64_t nv, dou
 // Four lanes per node, one per component: a neighbour's state is 32
 // contiguous bytes, and neighbours come from the node-block list (one index
 // each) in ascending order, four in flight.  Latency and L2 bound:
-// 233000 nodes of a quad mesh 78 -> 38 us against one lane per node that walked
+// 233000 nodes of the tetrahedral channel 78 -> 38 us against one lane per node that walked
 // the columns of its first CSR row.
 __global__ void __launch_bounds__(256)
 predict_features(const int64_t* __restrict__ rowptr, const int32_t* __restrict__ adj, const double* __restrict__ u,

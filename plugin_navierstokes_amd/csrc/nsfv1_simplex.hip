@@ -20,10 +20,11 @@
 // tetrahedral mesh) the gather alone took 1.0 ms of the channel's 1.55 ms.  One
 // lane per block reading the records itself was slower still (1.5 ms: every
 // load of a wave touches 64 different lines).
-// 96 x 48 x 48 cells of six tetrahedra (1.33 M elements, 233000 nodes), LPS, mass
-// part: records 279 us (637 MB written; FP64 ray casts at two waves per SIMD),
-// rows 510 us (637 MB read in 16-byte pieces of 128-byte lines, 224 MB written);
-// the call 1553 -> 712 us.
+// 96 x 48 x 48 cells of six tetrahedra less four obstacles (1.28 M elements, 233000
+// nodes), LPS, mass part, by a kernel trace: records 253 us (616 MB written; FP64
+// ray casts at two waves per SIMD), rows 463 us (1.4 GB fetched for 616 MB of
+// records, in 16-byte pieces of 128-byte lines; 229 MB written); the call 735 us
+// in that run.
 #include "nsfv1_geom.hpp"
 #include "nsfv1_internal.hpp"
 #include "nsfv1_ray.hpp"

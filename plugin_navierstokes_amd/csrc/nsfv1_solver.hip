@@ -166,12 +166,12 @@ __device__ inline double block_sums(double (&v)[K], double (&sh)[4][K])
 //   AXPY: w -= sum_i h_i V_i (w written), in ascending i;
 //   DOT:  partial[i][block] = sum over the block of V_i . w (the updated w);
 //   NORM: partial[0][block] = sum over the block of w^2.
-// The update of one pass and the projections of the next share one launch,
-// so the basis streams from HBM three times per Arnoldi step instead of four
-// (the projections' second read of a block's share of V hits the L2).  HBM
-// bound: 2.3 M unknowns, mean k = 10.5: projections 48 us (4.4 TB/s), update and
-// projections 84 us, update and norm 48 us; 3 launches of 180 us where dot and
-// update in launches of their own took 261 us.
+// The update of one pass and the projections of the next share one launch, which
+// reads its block's share of V twice; long vectors hold it in registers instead
+// (gs_hold), since the share outlives the L2 only in part.  HBM bound: 2.3 M
+// unknowns, mean k = 10.5: projections 48 us (4.4 TB/s), update and projections
+// 84 us, update and norm 48 us; 3 launches of 180 us where dot and update in
+// launches of their own took 261 us.
 constexpr int GS_VECS = 8;
 
 template <int E, bool AXPY, bool DOT, bool NORM, bool FULL>
@@ -250,8 +250,11 @@ gs_pass(const double* __restrict__ V, int64_t ld, int k, const double* __restric
 // The update and the next projections of up to GS_HOLD vectors, KH of them (k
 // rounded up to four, the surplus loads repeat the last vector) held in
 // registers between the two: the basis streams once where gs_pass reads it
-// twice (a block's share, 344 KB at k = 10, outlives neither the L2 nor LDS).
+// twice (a block's share is 344 KB at k = 10).
 // 2.3 M unknowns, k = 1 .. 20: 84 -> 52 us on average; 93 us at k = 17 .. 20 (4.3 TB/s).
+// All three launches, 2.3 M unknowns: 276 us at k = 24 (4.8 TB/s), 381 us at k = 25,
+// 451 at 30, 859 at 60 (3.6 to 3.9 TB/s): from 25 on, and below 2^20 unknowns
+// (k = 8: 62 us just below, 49 us from there on), the basis is read twice.
 constexpr int GS_HOLD = 24;
 
 template <int E, int KH, bool FULL>
