@@ -1475,9 +1475,11 @@ assemble_rows_split(KMeshPtrs M, KParams P, const double* __restrict__ u, const 
 
 // the row gather of nsfv1_rows.hpp from the SCVF records, in the plan's lane order
 // (by corner slot, then node: the lanes of a wave read records of consecutive
-// elements)
-template <int ET, int FAST>
-__global__ void __launch_bounds__(256)
+// elements).  LDS is that of the workgroup's lanes: with the 256 lanes' 43 KB a
+// workgroup of 64 leaves a CU three waves (40^3 cells, full upwind, 64 threads, the
+// whole assembly 241 us, 217 us in rounds, 132 us)
+template <int ET, int FAST, int LANES>
+__global__ void __launch_bounds__(LANES)
 split_rows(RowLists LL, KMeshPtrs M, KParams P, const double* __restrict__ u, const float* __restrict__ recs,
            int64_t ne_pad, float* __restrict__ J, double* __restrict__ dout)
 {
@@ -1490,7 +1492,7 @@ split_rows(RowLists LL, KMeshPtrs M, KParams P, const double* __restrict__ u, co
         return x * per + (x < rem ? x : rem) + k;
     }();
     const bool wantJ = J != nullptr, vec = ((uintptr_t)J & 15) == 0;
-    OwnedRows<N, NC, float, 1, true> rows(smem, LL, M, w, LL.cap, wantJ);
+    OwnedRows<N, NC, float, 1, true, LANES> rows(smem, LL, M, w, LL.cap, wantJ);
     const bool active = (int)threadIdx.x < rows.ni;
     Lane<ET, float> L;
 #pragma unroll
@@ -1838,6 +1840,15 @@ hipError_t launch_assemble(int et, int jprec, const KMeshPtrs& m, const int4* la
 }
 
 
+template <int ET, int FAST, int LANES>
+static void launch_split_rows(RowLists l, const KMeshPtrs& m, const KParams& p, const double* u, const float* recs,
+                              int64_t ne_pad, float* J, double* d, int nwg, hipStream_t s)
+{
+    using Rows = OwnedRows<Topo<ET>::nsh, Topo<ET>::dim + 1, float, 1, true, LANES>;
+    l.cap = Rows::out_cap(l.cap);
+    split_rows<ET, FAST, LANES><<<nwg, m.block, Rows::BASE + Rows::out_bytes(l.cap), s>>>(l, m, p, u, recs, ne_pad, J, d);
+}
+
 // split path: records then row gather (FP32 Jacobian, common configuration)
 template <int ET, int FAST>
 static hipError_t launch_split_cfg(const RowLists& l, const KMeshPtrs& m, const KParams& p, const double* u,
@@ -1855,10 +1866,9 @@ static hipError_t launch_split_cfg(const RowLists& l, const KMeshPtrs& m, const 
     } else if constexpr (ET == ET_QUAD) {
         assemble_rows_split<ET, FAST><<<nwg, m.block, lds, s>>>(m, p, u, recs, ne_pad, J, d);
     } else if constexpr (ET == ET_HEX) {
-        using Rows = OwnedRows<Topo<ET>::nsh, Topo<ET>::dim + 1, float, 1, true>;
-        RowLists lr = l;
-        lr.cap = Rows::out_cap(l.cap);
-        split_rows<ET, FAST><<<nwg, m.block, Rows::BASE + Rows::out_bytes(lr.cap), s>>>(lr, m, p, u, recs, ne_pad, J, d);
+        if (m.block <= 64) launch_split_rows<ET, FAST, 64>(l, m, p, u, recs, ne_pad, J, d, nwg, s);
+        else if (m.block <= 128) launch_split_rows<ET, FAST, 128>(l, m, p, u, recs, ne_pad, J, d, nwg, s);
+        else launch_split_rows<ET, FAST, 256>(l, m, p, u, recs, ne_pad, J, d, nwg, s);
     } else {
         return hipErrorInvalidValue;  // simplices have element records
     }

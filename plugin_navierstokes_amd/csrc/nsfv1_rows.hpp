@@ -62,13 +62,12 @@ __device__ __forceinline__ void rows_get(const VT* p, VT (&x)[NC])
     }
 }
 
-// N corners, NC unknowns a node, RP rows a pass
-template <int N, int NC, typename VT, int RP, bool OUT>
+// N corners, NC unknowns a node, RP rows a pass, workgroups of at most NB lanes
+template <int N, int NC, typename VT, int RP, bool OUT, int NB = ROWS_LANES>
 struct OwnedRows {
-    static constexpr int NB = ROWS_LANES;
     static constexpr size_t SEG = sizeof(VT) * N * RP * NB * NC;  // segments, then defects
     static_assert(SEG >= sizeof(double) * NC * NB, "the defects take the segments' place");
-    static constexpr size_t BASE = (SEG + sizeof(int) * (NB + 1) + sizeof(uint16_t) * N * NB + NB + 15) / 16 * 16;
+    static constexpr size_t BASE = (SEG + sizeof(int) * (ROWS_NODES + 1) + sizeof(uint16_t) * N * NB + NB + 15) / 16 * 16;
     // room for the finished segments of cap blocks (the most of a workgroup)
     static constexpr size_t out_bytes(int cap)
     {
@@ -98,7 +97,7 @@ struct OwnedRows {
         opos = reinterpret_cast<uint16_t*>(out + cap * RP * NC);
         seg = reinterpret_cast<VT*>(smem);
         nfirst = reinterpret_cast<int*>(smem + SEG);
-        sit = reinterpret_cast<uint16_t*>(nfirst + NB + 1);
+        sit = reinterpret_cast<uint16_t*>(nfirst + ROWS_NODES + 1);
         slane = reinterpret_cast<uint8_t*>(sit + N * NB);
         v0 = L.wg_node[w];
         nn = L.wg_node[w + 1] - v0;

@@ -38,7 +38,7 @@ def test_parity(cuda, mesh, up):
     assert fp32_violation(J, Jr, Ja) <= 1.0
 
 
-@pytest.mark.parametrize("mesh", ["all", "disjoint"])
+@pytest.mark.parametrize("mesh", ["all", "disjoint", "seven"])
 def test_routes_agree(cuda, mesh):
     import torch
 
