@@ -519,17 +519,17 @@ int nsfv1_predict_target(nsfv1_handle* h, const double* u_next, const double* u,
 /* Assembly path: 0 evaluates every SCVF once into a record (of the SCVF, or
    of the element for triangles and tetrahedra; FP32 Jacobian, common
    configuration: FIELDS, one upwind object, no Stokes/PAC/Peclet/exact
-   terms) and gathers rows from the records; 1
-   always runs the fused kernel (each SCVF evaluated by both of its rows);
-   2 is path 0 with dim+1 gather lanes per (node, element), one per row,
-   when the launch has 64 threads (nsfv1_set_launch); 3 (default) marches
-   through the element layers of a structured grid of parallelepipeds
-   (a lexicographic hexahedral grid, detected by nsfv1_set_mesh) with the
-   SCVF records held on chip -- FP32 Jacobian, no/full/skewed upwind, RAW
-   diffusion length, one viscosity -- and otherwise behaves as 0, except
-   that 2D meshes take the fused kernel with no or full upwind and below
-   98 304 elements.  All are deterministic.  The FLOW stabilisation and the positive upwind always
-   use the coupled path.  No counterpart in the plugin. */
+   terms) and gathers rows from the records; 1 always runs the fused kernel
+   (each SCVF evaluated by both of its rows); 2 is path 0 with dim+1 gather
+   lanes per (node, element), one per row, when the launch has 64 threads
+   (nsfv1_set_launch); 3 (default) marches through the element layers of a
+   structured grid of parallelepipeds (a lexicographic hexahedral grid,
+   detected by nsfv1_set_mesh) with the SCVF records held on chip -- FP32
+   Jacobian, no/full/skewed upwind, RAW diffusion length, one viscosity --
+   and otherwise behaves as 0, except that 2D meshes take the fused kernel
+   with no or full upwind and below 98 304 elements.  All are deterministic.
+   The FLOW stabilisation and the positive upwind always use the coupled
+   path.  No counterpart in the plugin. */
 int nsfv1_set_assembly_path(nsfv1_handle* h, int path);
 
 /* Kernel family that ran the last element assembly of the handle: 3 plane
